@@ -82,7 +82,9 @@ int madam_get_baselines(void *ctx, double *aa, double *yba, double *nna);
  * n_scatter, n_gather, precond_kind, nband, nseg, nof, rr_final, npix_hit,
  * nactive, t_total, t_step, ncg, band_chunks, band_chunks_unique, band_blocks,
  * band_blocks_unique, rec_bytes, band_rows_factored, prec_reused,
- * pointing_reused, nwide (the order of STAT_NAMES in libmadam_amd/__init__.py) */
+ * pointing_reused, nwide, run_records (the order of STAT_NAMES in
+ * libmadam_amd/__init__.py; run_records: runs of samples that the baseline
+ * side of the one-right-hand-side projections reads, 0 where it reads samples) */
 int madam_get_stats(void *ctx, double *out, int n);
 int madam_get_rr_history(void *ctx, double *out, int n);
 int madam_set_profiling(void *ctx, int on);
@@ -133,7 +135,8 @@ int madam_get_filter(void *ctx, int ipsd, double *fcov);
  * sides; + 16 = band factorization computes every row (no periodic
  * continuation of repeating 64-row blocks); + 32 / + 64 = band carry chains
  * always / never several per wave (default: several when there are enough
- * of them); no variant changes a result bit */
+ * of them), + 128 (before the first solve on a pointing) = run records of the
+ * projections whatever the number of samples */
 int madam_set_kernel_variant(void *ctx, int variant);
 /* pointing expansion of the synthetic ring scan: scan5 = {fsample, spin_period,
  * prec_period, opening_turns, lon0_turns}, dets3[ndet][3] = {psi_turns,

@@ -315,9 +315,7 @@ static void batch_operator(Context &c, BatchState &B, const T *x, T *y, T *pw, T
     // the FP32 operator at R >= 8 reads the run-length records
     bool rle = std::is_same<T, float>::value && B.rle_ok && R >= 8;
     if (one)
-        launch_scatter_seg<T>(s, c.nmap, c.nactive, ent_records(c), c.rec_layout, pw, c.sr_s.heads.p, c.sr_s.k0.p,
-                              c.sr_s.fix_end.p, c.sr_s.fix_ord.p, c.d_nzq.p, c.nzpix, Ops<T>::cc(c, B),
-                              Ops<T>::m4(c, B), c.d_sr_part.p);
+        project_to_map<T>(c, pw, Ops<T>::cc(c, B), Ops<T>::m4(c, B));
     else if (rle)
         batch_scatter<T>(s, R, REC16, c.nmap, B.bt_c, B.rs_rec.p, pw, Ops<T>::cc(c, B), c.d_nzq.p, m, part);
     else
@@ -340,8 +338,7 @@ static void batch_operator(Context &c, BatchState &B, const T *x, T *y, T *pw, T
         tm->ga.start(s);
     }
     if (one)
-        launch_gather_flat<T>(s, c.nmap, c.ndet, c.nsamp, c.nbase, c.d_bstart.p, sample_records(c), c.rec_layout,
-                              Ops<T>::m4(c, B), c.ndeg, Ops<T>::dwb(c, B), Ops<T>::nna(c, B), x, y);
+        project_to_baselines<T>(c, Ops<T>::m4(c, B), Ops<T>::dwb(c, B), Ops<T>::nna(c, B), x, y);
     else if (rle)
         batch_gather<T>(s, R, REC16, c.nmap, c.ndet, c.nsamp, c.nbase, B.rg_st.p, B.rg_rec.p, m, 1,
                         Ops<T>::dwb(c, B), Ops<T>::nna(c, B), x, y, active, c.nbase + 1, B.rg_base.p);
@@ -712,6 +709,7 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
             B.fprec_rows32.release();
         }
         if (B.fcov_rows32.p != old_f || B.fprec_rows32.p != old_p) B.drop_graphs();   // bound into the captured step
+        if (R == 1) runs_prepare_fp32(c);
         Vec<float> v = alloc_vectors<float>(c, B);
         B.m4f.alloc((size_t)std::max<int64_t>(c.npix_cross, 1) * 4);
         if (R > 1 && (!B.tables_ok || B.tables_ent != ent_records(c))) {

@@ -111,7 +111,7 @@ enum { ST_NITER, ST_RRINIT, ST_RZINIT, ST_T_POINTING, ST_T_BIN, ST_T_INIT, ST_T_
        ST_T_SCATTER, ST_T_GATHER, ST_T_PRIOR, ST_T_APPLY_PREC, ST_N_SCATTER, ST_N_GATHER, ST_PRECOND_KIND,
        ST_NBAND, ST_NSEG, ST_NOF, ST_RR_FINAL, ST_NPIX_HIT, ST_NACTIVE, ST_T_TOTAL, ST_T_STEP, ST_NCG,
        ST_BAND_CHUNKS, ST_BAND_CHUNKS_UNIQUE, ST_BAND_BLOCKS, ST_BAND_BLOCKS_UNIQUE, ST_REC_BYTES,
-       ST_BAND_ROWS_FACTORED, ST_PREC_REUSED, ST_POINTING_REUSED, ST_NWIDE, ST_COUNT };
+       ST_BAND_ROWS_FACTORED, ST_PREC_REUSED, ST_POINTING_REUSED, ST_NWIDE, ST_RUN_RECORDS, ST_COUNT };
 
 struct Context;
 struct BatchState;
@@ -188,6 +188,19 @@ struct Context {
         int64_t nent = 0;
         bool ok = false;
     } sr_s, sr_g;
+    // run records of the one-right-hand-side projections (madam_runs.hip):
+    // mean_run is the estimated samples per run, runs_ok whether the records
+    // of this pointing exist (word and FP64 sums; the FP32 sums on demand)
+    double mean_run = 0;
+    bool runs_ok = false;
+    int run_sh = 0;
+    int64_t n_rung = 0, n_runs = 0;
+    DBuf<uint32_t> d_rung, d_runs;
+    DBuf<double2> d_rungw, d_runsw;
+    DBuf<float2> d_rungw32, d_runsw32;
+    bool runs32_ok = false;
+    DBuf<int64_t> d_rungst;
+    SegTiles sr_r;   // pixel-side segment tables over the runs
     DBuf<int32_t> d_nzq;
     DBuf<int64_t> d_segstart_s;   // CSR start of each non-empty cross pixel (pixel-side ordinal order)
     DBuf<double> d_ccinv_c;   // inverse cross-pixel matrices in the pixel side's ordinal order
@@ -300,6 +313,16 @@ int group_for(const Context &c);
 template <typename TT>
 void solve_setup(Context &c, const TT *tod);
 void cg_apply(Context &c, const double *r, double *z);
+// the two projections of one right-hand side, from the run records where the
+// pointing has them: m4 = ccinv P^T W F p (pw = p dwb in slot order), and
+// ap += nna p - F^T W P m4
+// the FP32 weight sums of the run records, before FP32 projections (allocates:
+// call outside graph capture)
+void runs_prepare_fp32(Context &c);
+template <typename T>
+void project_to_map(Context &c, const T *pw, const T *cc_c, T *m4);
+template <typename T>
+void project_to_baselines(Context &c, const T *m4, const T *dwb, const T *nna, const T *p, T *ap);
 
 // batched and mixed-precision solves (madam_batch_host.cpp)
 void solve_batch(Context &c, int nrhs, const void *signals, int tod_f32, int on_device, int precision);

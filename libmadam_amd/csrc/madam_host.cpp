@@ -721,15 +721,21 @@ static void set_pointing(Context &c, int32_t *pix, float *w, int on_device, bool
     csr_alloc(cs, n, c.npix_map);
     {
         DBuf<unsigned long long> cnt;
-        cnt.alloc(1);
-        MADAM_CHECK(hipMemsetAsync(cnt.p, 0, sizeof(unsigned long long), s));
+        cnt.alloc(3);
+        MADAM_CHECK(hipMemsetAsync(cnt.p, 0, sizeof(unsigned long long) * 3, s));
+        int dsh = 0;
+        while ((1ll << dsh) < c.ndeg) ++dsh;
         launch_pack(s, c.d_pix, c.d_w, c.nnz, c.nmap, c.ndet, c.nsamp, c.d_ivs.p, c.nival, c.d_dw_ival.p,
-                    c.p.nsubchunk, c.pass, c.d_pixw.p, cs.k[0].p, (uint32_t)c.npix_map, c.d_pixc.p, cnt.p);
+                    c.p.nsubchunk, c.pass, c.d_pixw.p, cs.k[0].p, (uint32_t)c.npix_map, c.d_pixc.p, dsh, cnt.p);
         MADAM_CHECK(hipGetLastError());
-        unsigned long long h = 0;
-        d2h(&h, cnt.p, 1, s);
+        unsigned long long h[3] = {0, 0, 0};
+        d2h(h, cnt.p, 3, s);
         MADAM_CHECK(hipStreamSynchronize(s));
-        if (c.nmap == 3 && h != 0) rl = REC16;
+        if (c.nmap == 3 && h[0] != 0) rl = REC16;
+        // samples per run of one baseline on one cross pixel: runs start at a
+        // new pixel and at every baseline
+        double seen = (double)h[1], per_base = c.nbase > 0 ? (double)c.nsamp / c.nbase : 1.0;
+        c.mean_run = seen > 0 ? seen / (seen - (double)h[2] + seen / per_base) : 0.0;
     }
     c.rec_layout = rl;
     c.stats[ST_REC_BYTES] = rec_bytes(rl);
@@ -771,6 +777,8 @@ static void set_pointing(Context &c, int32_t *pix, float *w, int on_device, bool
     c.stats[ST_NACTIVE] = (double)total;
     c.pointed = true;
     c.tiles_built = false;
+    c.runs_ok = c.runs32_ok = false;
+    c.stats[ST_RUN_RECORDS] = 0;
     c.prec_cached = false;
     c.stats[ST_POINTING_REUSED] = 0;
     batch_invalidate(c);
@@ -787,6 +795,144 @@ static void segtiles_alloc(Context::SegTiles &t, int64_t nent)
     t.fix_end.alloc(nt > 0 ? nt : 1);
     t.fix_ord.alloc(nt > 0 ? nt : 1);
 }
+
+// Whether the one-right-hand-side projections in type T read run records:
+// where a run's record (20 bytes in FP64, 12 in FP32, 4 for temperature) is
+// smaller than its samples' (12 or 4 bytes each) by enough to pay for the
+// separate weight stream (both sides measured in madam_runs.hip).  Building
+// them takes some 0.5 ms of launches and allocations, which a solve of fewer
+// than RUN_SAMPLES samples does not earn back (a 4,000-sample destripe: 5.8 ms
+// without, 6.4 ms with); kernel variant + 128 builds them for any number.
+static constexpr int64_t RUN_SAMPLES = 1 << 18;
+template <typename T>
+static bool runs_wanted(const Context &c)
+{
+    if (c.rec_layout == REC16 || c.nactive <= 0) return false;
+    if (c.nactive < RUN_SAMPLES && !(c.kernel_variant & 128)) return false;
+    return c.mean_run >= (sizeof(T) == 8 ? 2.0 : 1.3);
+}
+
+// run records of both projections, and the pixel side's segment tables over them
+static void build_runs(Context &c)
+{
+    hipStream_t s = c.stream;
+    int dsh = 0;
+    while ((1ll << dsh) < c.ndeg) ++dsh;
+    int sh = 1;
+    while ((1ll << sh) < std::max(c.npix_cross, c.nbtot)) ++sh;
+    if (sh > 28) return;
+    uint32_t maxrun = (1u << (32 - sh)) - 1u;
+    int64_t n = (int64_t)c.ndet * c.nsamp, nent = c.nactive, nmax = std::max(n, nent);
+    DBuf<uint32_t> mask;
+    DBuf<unsigned long long> words;
+    DBuf<int32_t> counts;
+    DBuf<int64_t> offs, tmp, seg;
+    int64_t nsp = runs_spans(nmax);
+    mask.alloc(std::max<int64_t>(c.nsamp, nent) / 32 + 1);
+    words.alloc(nmax / 64 + 9);
+    counts.alloc(nsp);
+    offs.alloc(nsp + 1);
+    tmp.alloc((nsp + 1 + 4095) / 4096 + 1);
+    auto total = [&](int64_t m) {
+        int64_t t = 0;
+        d2h(&t, offs.p + runs_spans(m), 1, s);
+        MADAM_CHECK(hipStreamSynchronize(s));
+        return t;
+    };
+    const bool pol = c.nmap == 3;
+    // baseline side: the samples in time order
+    runs_mark(s, c.d_pixc.p, c.rec_layout, n, c.nsamp, dsh, maxrun, c.d_bstart.p, c.nbase, mask.p, words.p, counts.p,
+              offs.p, tmp.p);
+    c.n_rung = total(n);
+    c.d_rung.alloc(c.n_rung);
+    if (pol) c.d_rungw.alloc(c.n_rung);
+    runs_write(s, c.d_pixc.p, c.rec_layout, n, dsh, sh, words.p, offs.p, c.d_rung.p, pol ? c.d_rungw.p : nullptr);
+    c.d_rungst.alloc((size_t)c.ndet * (c.nbase + 1));
+    runs_base_starts(s, c.d_bstart.p, c.nbase, c.ndet, c.nsamp, words.p, offs.p, c.d_rungst.p);
+    // pixel side: the CSR entries
+    runs_mark(s, c.d_entc.p, c.rec_layout, nent, nent, 0, maxrun, c.d_segstart_s.p, c.nzpix, mask.p, words.p, counts.p,
+              offs.p, tmp.p);
+    c.n_runs = total(nent);
+    c.d_runs.alloc(c.n_runs);
+    if (pol) c.d_runsw.alloc(c.n_runs);
+    runs_write(s, c.d_entc.p, c.rec_layout, nent, 0, sh, words.p, offs.p, c.d_runs.p, pol ? c.d_runsw.p : nullptr);
+    seg.alloc(c.nzpix + 1);
+    runs_pixel_starts(s, c.d_segstart_s.p, c.nzpix, words.p, offs.p, seg.p);
+    segtiles_alloc(c.sr_r, c.n_runs);
+    segred_build(s, seg.p, c.nzpix, c.n_runs, c.sr_r.heads.p, c.sr_r.k0.p, c.sr_r.fix_end.p, c.sr_r.fix_ord.p);
+    MADAM_CHECK(hipStreamSynchronize(s));
+    c.run_sh = sh;
+    c.runs_ok = true;
+    c.stats[ST_RUN_RECORDS] = (double)c.n_rung;
+}
+
+void runs_prepare_fp32(Context &c)
+{
+    if (!runs_wanted<float>(c) || c.runs32_ok) return;
+    if (!c.runs_ok) build_runs(c);
+    if (!c.runs_ok) return;
+    if (c.nmap == 3) {
+        c.d_rungw32.alloc(c.n_rung);
+        c.d_runsw32.alloc(c.n_runs);
+        runs_cast(c.stream, c.d_rungw.p, c.d_rungw32.p, c.n_rung);
+        runs_cast(c.stream, c.d_runsw.p, c.d_runsw32.p, c.n_runs);
+    }
+    c.runs32_ok = true;
+}
+
+template <typename T>
+static RunView<T> run_view(Context &c)
+{
+    RunView<T> v;
+    v.sh = c.run_sh;
+    v.per_base = (double)c.n_rung / std::max<int64_t>(c.nbtot, 1);
+    v.gst = c.d_rungst.p;
+    v.gword = c.d_rung.p;
+    v.sword = c.d_runs.p;
+    if (sizeof(T) == 8) {
+        v.gw = c.d_rungw.p;
+        v.sw = c.d_runsw.p;
+    } else {
+        v.gw = c.d_rungw32.p;
+        v.sw = c.d_runsw32.p;
+    }
+    return v;
+}
+
+template <typename T>
+static bool use_runs(const Context &c)
+{
+    return (sizeof(T) == 8 ? c.runs_ok : c.runs32_ok) && runs_wanted<T>(c);
+}
+
+template <typename T>
+void project_to_map(Context &c, const T *pw, const T *cc_c, T *m4)
+{
+    if (use_runs<T>(c))
+        launch_scatter_run<T>(c.stream, c.nmap, c.n_runs, run_view<T>(c), pw, c.sr_r.heads.p, c.sr_r.k0.p,
+                              c.sr_r.fix_end.p, c.sr_r.fix_ord.p, c.d_nzq.p, c.nzpix, cc_c, m4, c.d_sr_part.p);
+    else
+        launch_scatter_seg<T>(c.stream, c.nmap, c.nactive, c.rec_layout == REC16 ? (const void *)c.d_ent.p : c.d_entc.p,
+                              c.rec_layout, pw, c.sr_s.heads.p, c.sr_s.k0.p, c.sr_s.fix_end.p, c.sr_s.fix_ord.p,
+                              c.d_nzq.p, c.nzpix, cc_c, m4, c.d_sr_part.p);
+}
+template void project_to_map<double>(Context &, const double *, const double *, double *);
+template void project_to_map<float>(Context &, const float *, const float *, float *);
+
+template <typename T>
+void project_to_baselines(Context &c, const T *m4, const T *dwb, const T *nna, const T *p, T *ap)
+{
+    if (use_runs<T>(c))
+        launch_gather_run<T>(c.stream, c.nmap, c.ndet, c.nbase, run_view<T>(c), m4, dwb, nna, p, ap);
+    else
+        launch_gather_flat<T>(c.stream, c.nmap, c.ndet, c.nsamp, c.nbase, c.d_bstart.p,
+                              c.rec_layout == REC16 ? (const void *)c.d_pixw.p : c.d_pixc.p, c.rec_layout, m4, c.ndeg,
+                              dwb, nna, p, ap);
+}
+template void project_to_baselines<double>(Context &, const double *, const double *, const double *, const double *,
+                                           double *);
+template void project_to_baselines<float>(Context &, const float *, const float *, const float *, const float *,
+                                          float *);
 
 // segment tables of the two projections; they depend on the pointing only
 static void build_segtiles(Context &c)
@@ -838,6 +984,7 @@ static void build_segtiles(Context &c)
     }
     int64_t nt = std::max(segred_ntiles(c.nactive), segred_ntiles((int64_t)c.ndet * c.nsamp));
     c.d_sr_part.alloc(2 * (nt > 0 ? nt : 1));
+    if (runs_wanted<double>(c)) build_runs(c);
 }
 
 
@@ -1187,7 +1334,9 @@ static int pcg_steps(Context &c, int nmax, bool converge)
         done++;
         c.pcg_steps_done++;
         if (prof) { t_it.start(s); t_sc.start(s); }
-        if ((c.kernel_variant & 15) == 0 || (c.kernel_variant & 15) == 3)   // segmented tiles (default)
+        if ((c.kernel_variant & 15) == 0)   // segmented tiles (default)
+            project_to_map<double>(c, c.d_pw.p, c.d_ccinv_c.p, c.d_m4x.p);
+        else if ((c.kernel_variant & 15) == 3)
             launch_scatter_seg(s, c.nmap, c.nactive, c.rec_layout == REC16 ? (const void *)c.d_ent.p : c.d_entc.p,
                                c.rec_layout, c.d_pw.p, c.sr_s.heads.p, c.sr_s.k0.p,
                                c.sr_s.fix_end.p, c.sr_s.fix_ord.p, c.d_nzq.p, c.nzpix, c.d_ccinv_c.p, c.d_m4x.p,
@@ -1207,6 +1356,8 @@ static int pcg_steps(Context &c, int nmax, bool converge)
             launch_gather_seg(s, c.nmap, (int64_t)c.ndet * c.nsamp, c.d_pixw.p, c.d_m4x.p, c.ndeg, c.sr_g.heads.p,
                               c.sr_g.k0.p, c.sr_g.fix_end.p, c.sr_g.fix_ord.p, c.d_dwb.p, c.d_nna.p, c.d_p.p,
                               c.d_ap.p, c.d_sr_part.p);
+        else if ((c.kernel_variant & 15) == 0)
+            project_to_baselines<double>(c, c.d_m4x.p, c.d_dwb.p, c.d_nna.p, c.d_p.p, c.d_ap.p);
         else if ((c.kernel_variant & 15) != 1)
             launch_gather_flat(s, c.nmap, c.ndet, c.nsamp, c.nbase, c.d_bstart.p,
                                c.rec_layout == REC16 ? (const void *)c.d_pixw.p : c.d_pixc.p, c.rec_layout,
@@ -1265,15 +1416,11 @@ static void apply_operator(Context &c, const double *x, double *y, double *pw)
     const Params &p = c.p;
     int64_t nb = c.nbtot;
     launch_pw_slots(s, x, c.d_bord.p, c.d_dwb_s.p, pw, nb);
-    launch_scatter_seg(s, c.nmap, c.nactive, c.rec_layout == REC16 ? (const void *)c.d_ent.p : c.d_entc.p,
-                       c.rec_layout, pw, c.sr_s.heads.p, c.sr_s.k0.p, c.sr_s.fix_end.p, c.sr_s.fix_ord.p,
-                       c.d_nzq.p, c.nzpix, c.d_ccinv_c.p, c.d_m4x.p, c.d_sr_part.p);
+    project_to_map<double>(c, pw, c.d_ccinv_c.p, c.d_m4x.p);
     if (p.kfilter) apply_prior(c, x, y);
     else if (p.diagfilter != 0) launch_axpby_nna(s, y, c.d_nna.p, x, p.diagfilter, nb);
     else launch_fill(s, y, 0.0, nb);
-    launch_gather_flat(s, c.nmap, c.ndet, c.nsamp, c.nbase, c.d_bstart.p,
-                       c.rec_layout == REC16 ? (const void *)c.d_pixw.p : c.d_pixc.p, c.rec_layout, c.d_m4x.p,
-                       c.ndeg, c.d_dwb.p, c.d_nna.p, x, y);
+    project_to_baselines<double>(c, c.d_m4x.p, c.d_dwb.p, c.d_nna.p, x, y);
 }
 
 // one operator of the last solve on a host vector of nbtot baselines:

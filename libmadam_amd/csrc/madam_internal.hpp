@@ -30,7 +30,7 @@ struct PixW {
 // of exactly 1 (the (1, cos 2psi, sin 2psi) convention), REC12 {index, w1, w2}
 // and, for temperature-only maps, REC4 {index} carry the same information in
 // fewer bytes (1.0f * x == x, so the results are the same bits).
-enum RecLayout { REC16 = 0, REC12 = 1, REC4 = 2 };
+enum RecLayout { REC16 = 0, REC12 = 1, REC4 = 2, REC_RUN = 3 };
 struct Rec12 {
     int32_t i;
     float w1, w2;
@@ -114,6 +114,35 @@ struct VecT<float> {
     using v4 = float4;
 };
 
+// Run records of the one-right-hand-side projections (madam_runs.hip), in the
+// operator's type: a word {number of samples, index} per run, the sums of w1
+// and w2 beside it (nmap 3).  g*: runs in time order, gst[ndet][nbase + 1] the
+// first run of each baseline; s*: runs of the CSR in pixel order.
+template <typename T>
+struct RunView {
+    int sh = 0;          // bits of the index
+    double per_base = 0;   // runs per baseline (mean)
+    const int64_t *gst = nullptr;
+    const uint32_t *gword = nullptr, *sword = nullptr;
+    const void *gw = nullptr, *sw = nullptr;
+};
+// weight sums of run i, read once per pass (non-temporal, as load_rec_nt)
+template <typename T>
+__device__ inline typename VecT<T>::v2 load_wsum_nt(const void *base, int64_t i)
+{
+    typename VecT<T>::v2 r;
+    if constexpr (sizeof(T) == 8) {
+        rec_v4i v = __builtin_nontemporal_load((const rec_v4i *)base + i);
+        r.x = __hiloint2double(v.y, v.x);
+        r.y = __hiloint2double(v.w, v.z);
+    } else {
+        long long v = __builtin_nontemporal_load((const long long *)base + i);
+        r.x = __int_as_float((int)v);
+        r.y = __int_as_float((int)(v >> 32));
+    }
+    return r;
+}
+
 struct CsrEnt {
     int32_t b;   // global baseline index
     float w0, w1, w2;
@@ -156,10 +185,12 @@ void launch_flag_intervals(hipStream_t s, int32_t *pix, int64_t nsamp, const int
 // same pass, the CSR sort keys (the pixel, flag_key for inactive samples), the
 // compact records (REC12 for nmap 3, REC4 for nmap 1; those of REC12 are only
 // valid when *nonunit stays 0) and *nonunit += the number of active samples
-// whose w0 is not exactly 1 (*nonunit must start at 0)
+// whose w0 is not exactly 1; of a 64th of the samples, nonunit[1] += the
+// active ones and nonunit[2] += those on the cross pixel (pixel >> dsh) of the
+// sample before (all three must start at 0)
 void launch_pack(hipStream_t s, const int32_t *pix, const float *w, int nnz, int nmap, int ndet, int64_t nsamp,
                  const int64_t *ival_start, int ninterval, const double *dw_ival, int nsubchunk, int pass,
-                 PixW *pixw, uint32_t *key, uint32_t flag_key, void *pixc, unsigned long long *nonunit);
+                 PixW *pixw, uint32_t *key, uint32_t flag_key, void *pixc, int dsh, unsigned long long *nonunit);
 void launch_exclusive_scan_i32_to_i64(hipStream_t s, const int32_t *in, int64_t n, int64_t *out, int64_t *tmp,
                                       int64_t tmp_len);
 // TT: the TOD's type (double, or float for the mixed-precision solves)
@@ -215,6 +246,11 @@ template <typename T>
 void launch_scatter_seg(hipStream_t s, int nmap, int64_t nent, const void *ent, int rl, const T *pw,
                         const uint8_t *heads, const int64_t *tile_k0, const int64_t *fix_end, const int64_t *fix_ord,
                         const int32_t *nzq, int64_t nzpix, const T *cc_c, T *m4, void *part);
+// the same over run records (the segment tables built over the runs)
+template <typename T>
+void launch_scatter_run(hipStream_t s, int nmap, int64_t nrun, const RunView<T> &rv, const T *pw, const uint8_t *heads,
+                        const int64_t *tile_k0, const int64_t *fix_end, const int64_t *fix_ord, const int32_t *nzq,
+                        int64_t nzpix, const T *cc_c, T *m4, void *part);
 // cc_c[k] = ccinv6[nzq[k]]: the inverse pixel matrices in the pixel side's ordinal order
 void segred_compact_cc(hipStream_t s, const int32_t *nzq, int64_t nseg, const double *ccinv6, double *cc_c);
 void launch_gather_seg(hipStream_t s, int nmap, int64_t nent, const PixW *pixw, const double *m4, int64_t ndeg,
@@ -276,6 +312,29 @@ void launch_cg_prec(hipStream_t s, const Segment *seg, int64_t nseg, const int *
                     const double *resid, double *zr);
 void launch_cg_p(hipStream_t s, const Segment *seg, int64_t nseg, const int *act, const double *beta, const double *zr,
                  double *p);
+
+// ------------------------------------------------------------------ runs.hip
+
+int64_t runs_spans(int64_t n);
+// start bits of the runs among n records (index >> dsh, a negative index takes
+// no part), cut at `starts` (positions inside a period) and at every multiple
+// of maxrun: words[n / 64 + 9], counts[runs_spans(n)], offs[runs_spans(n) + 1]
+// the exclusive scan of counts, mask[period / 32 + 1] scratch
+void runs_mark(hipStream_t s, const void *rec, int rl, int64_t n, int64_t period, int dsh, uint32_t maxrun,
+               const int64_t *starts, int64_t nstarts, uint32_t *mask, unsigned long long *words, int32_t *counts,
+               int64_t *offs, int64_t *scan_tmp);
+// the runs' words and (REC12) weight sums
+void runs_write(hipStream_t s, const void *rec, int rl, int64_t n, int dsh, int sh, const unsigned long long *words,
+                const int64_t *offs, uint32_t *out, double2 *w64);
+// first run of every baseline gst[ndet][nbase + 1], of every pixel seg[nz + 1]
+void runs_base_starts(hipStream_t s, const int64_t *bstart, int64_t nbase, int ndet, int64_t nsamp,
+                      const unsigned long long *words, const int64_t *offs, int64_t *gst);
+void runs_pixel_starts(hipStream_t s, const int64_t *segstart, int64_t nz, const unsigned long long *words,
+                       const int64_t *offs, int64_t *seg);
+void runs_cast(hipStream_t s, const double2 *in, float2 *out, int64_t n);
+template <typename T>
+void launch_gather_run(hipStream_t s, int nmap, int ndet, int64_t nbase, const RunView<T> &rv, const T *m4,
+                       const T *dwb, const T *nna, const T *p, T *ap);
 
 // ------------------------------------------------------------------ fft.hip
 

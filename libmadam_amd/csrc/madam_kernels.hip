@@ -156,10 +156,12 @@ void launch_flag_intervals(hipStream_t s, int32_t *pix, int64_t nsamp, const int
 
 __global__ void k_pack(const int32_t *pix, const float *w, int nnz, int nmap, int ndet, int64_t nsamp,
                        const int64_t *ivs, int nival, const double *dw_ival, int nsubchunk, int pass, PixW *out,
-                       uint32_t *key, uint32_t flag_key, void *pixc, unsigned long long *nonunit)
+                       uint32_t *key, uint32_t flag_key, void *pixc, int dsh, unsigned long long *nonunit)
 {
     int64_t n = (int64_t)ndet * nsamp;
     unsigned long long nu = 0;
+    unsigned same = 0, seen = 0;
+    const bool sampled = (blockIdx.x & 63) == 0;   // the run length is estimated from a 64th of the blocks
     for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < n; g += (int64_t)gridDim.x * blockDim.x) {
         int det = (int)(g / nsamp);
         int64_t i = g % nsamp;
@@ -187,6 +189,10 @@ __global__ void k_pack(const int32_t *pix, const float *w, int nnz, int nmap, in
         out[g] = r;
         key[g] = r.pix >= 0 ? (uint32_t)r.pix : flag_key;
         nu += (r.pix >= 0 && r.w0 != 1.0f) ? 1 : 0;
+        if (sampled && r.pix >= 0) {
+            seen++;
+            same += (i > 0 && pix[g - 1] >= 0 && pix[g - 1] >> dsh == r.pix >> dsh) ? 1 : 0;
+        }
         if (nmap == 3) {
             Rec12 c;
             c.i = r.pix;
@@ -199,15 +205,25 @@ __global__ void k_pack(const int32_t *pix, const float *w, int nnz, int nmap, in
     }
     for (int o = 32; o > 0; o >>= 1) nu += __shfl_xor(nu, o, 64);
     if ((threadIdx.x & 63) == 0 && nu) atomicAdd(nonunit, nu);
+    if (sampled) {
+        for (int o = 32; o > 0; o >>= 1) {
+            seen += __shfl_xor(seen, o, 64);
+            same += __shfl_xor(same, o, 64);
+        }
+        if ((threadIdx.x & 63) == 0) {
+            atomicAdd(nonunit + 1, (unsigned long long)seen);
+            atomicAdd(nonunit + 2, (unsigned long long)same);
+        }
+    }
 }
 
 void launch_pack(hipStream_t s, const int32_t *pix, const float *w, int nnz, int nmap, int ndet, int64_t nsamp,
                  const int64_t *ivs, int nival, const double *dw_ival, int nsubchunk, int pass, PixW *pixw,
-                 uint32_t *key, uint32_t flag_key, void *pixc, unsigned long long *nonunit)
+                 uint32_t *key, uint32_t flag_key, void *pixc, int dsh, unsigned long long *nonunit)
 {
     k_pack<<<grid_for((int64_t)ndet * nsamp, TPB), TPB, 0, s>>>(pix, w, nnz, nmap, ndet, nsamp, ivs, nival,
                                                                 dw_ival, nsubchunk, pass, pixw, key, flag_key, pixc,
-                                                                nonunit);
+                                                                dsh, nonunit);
 }
 
 // ---------------------------------------------------------------- CSR by pixel
@@ -869,19 +885,20 @@ static constexpr int FLAT_LANES = 4;     // lanes per item in the reduction phas
 // the same load instruction, one cache-line access for all of them; the loads
 // of the pointing stream stay in whole 256-byte runs.
 static constexpr int FG_D = 4;                    // detectors per block
-static constexpr int FG_ITEMS = 256;              // (detector, baseline) items per block
-static constexpr int FG_LANES = FG_ITEMS >= 256 ? 1 : 256 / FG_ITEMS;   // lanes per item (reduction)
-static constexpr int FG_IPT = FG_ITEMS >= 256 ? FG_ITEMS / 256 : 1;     // items per thread
-static constexpr int FG_K = FG_ITEMS / FG_D;      // baselines per detector per block
 static constexpr int FG_T = FLAT_TILE / FG_D;     // samples per detector per LDS tile
 
-template <typename T, int NMAP, int RL>
+// FG_K baselines per detector and block: 64 (one lane sums each), or 16 (four
+// lanes each) for few or long baselines.
+template <typename T, int NMAP, int RL, int FG_K>
 __global__ void __launch_bounds__(256) k_gather_flat(int ndet, int64_t nsamp, int64_t nbase,
                                                      const int64_t *bstart, const void *pixw, const T *m4,
                                                      int64_t ndeg, const T *dwb, const T *nna,
                                                      const T *p, T *ap)
 {
     using V2 = typename VecT<T>::v2;
+    constexpr int FG_ITEMS = FG_D * FG_K;                          // (detector, baseline) items per block
+    constexpr int FG_LANES = FG_ITEMS >= 256 ? 1 : 256 / FG_ITEMS;   // lanes per item (reduction)
+    constexpr int FG_IPT = FG_ITEMS >= 256 ? FG_ITEMS / 256 : 1;     // items per thread
     __shared__ T vals[FLAT_TILE + 1];    // vals[d * FG_T + t]
     __shared__ int64_t bs[FG_K + 1];      // sample starts of the block's baselines, bs[nk] = end
     int64_t ngrp = (ndet + FG_D - 1) / FG_D;
@@ -1195,12 +1212,24 @@ void launch_gather_flat(hipStream_t s, int nmap, int ndet, int64_t nsamp, int64_
                         const void *pixw, int rl, const T *m4, int64_t ndeg, const T *dwb, const T *nna, const T *p,
                         T *ap)
 {
-    int64_t grid = ((ndet + FG_D - 1) / FG_D) * ((nbase + FG_K - 1) / FG_K);
-    if (grid > 0)
+    if (ndet <= 0 || nbase <= 0) return;
+    int64_t ngrp = (ndet + FG_D - 1) / FG_D;
+    // 64 baselines per detector and block keep the start-up cost of a block
+    // small, 16 leave more blocks and four lanes per sum where baselines are
+    // few or long.  Measured, us per launch, K = 64 / 16: FP64 4 x 2^20 samples
+    // in baselines of 100 93 / 22; 8 x 2^22 of 50, own boresights 148 / 135;
+    // 4 x 2^22 of 25 49 / 48; FP32 16 x 2^23 of 25 349 / 368.
+    const bool wide = ngrp * ((nbase + 63) / 64) >= 1024 && nsamp <= 40 * nbase;
     {
 #define MADAM_GF(NM, RLV)                                                                                        \
-    k_gather_flat<T, NM, RLV><<<(unsigned)grid, 256, 0, s>>>(ndet, nsamp, nbase, bstart, pixw, m4, ndeg, dwb, nna, p, \
-                                                             ap)
+    do {                                                                                                         \
+        if (wide)                                                                                                \
+            k_gather_flat<T, NM, RLV, 64><<<(unsigned)(ngrp * ((nbase + 63) / 64)), 256, 0, s>>>(                \
+                ndet, nsamp, nbase, bstart, pixw, m4, ndeg, dwb, nna, p, ap);                                    \
+        else                                                                                                     \
+            k_gather_flat<T, NM, RLV, 16><<<(unsigned)(ngrp * ((nbase + 15) / 16)), 256, 0, s>>>(                \
+                ndet, nsamp, nbase, bstart, pixw, m4, ndeg, dwb, nna, p, ap);                                    \
+    } while (0)
         if (nmap == 1) {
             if (rl == REC4) MADAM_GF(1, REC4);
             else MADAM_GF(1, REC16);

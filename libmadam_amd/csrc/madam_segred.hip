@@ -260,8 +260,11 @@ __device__ inline unsigned sr_head_bits(const uint8_t *heads, int64_t e0, int64_
 // (compact ordinal order) and the pixel index that lane l loaded before the
 // reduction.  Only a tile that finishes more than 64 pixels reads the
 // finishing data of the rest where they complete.
+// RL = REC_RUN: the entries are run records, `ent` their words and `entw`
+// their weight sums; a run of n samples enters with weights (n, W1, W2).
 template <typename T, int NC, int WAVES, int RL>
-__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(5, 8))) k_sr_scatter(int64_t nent, const void *ent, const T *pw,
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(5, 8))) k_sr_scatter(int64_t nent, const void *ent,
+                                                           const void *entw, int sh, const T *pw,
                                                            const uint8_t *heads, const int64_t *tile_k0,
                                                            const int64_t *fix_end, const int32_t *nzq,
                                                            int64_t nzpix, const T *cc_c, T *m4,
@@ -273,7 +276,10 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     int64_t j = sr_xcd_block(blockIdx.x, gridDim.x) * WAVES + w;
     int64_t t0 = j * SR_TILE;
     if (t0 >= nent) return;   // uniform over the wave; waves synchronise only with themselves
-    PixW e[SR_PER_LANE];   // the entries as full records: .pix is the baseline slot
+    constexpr bool RUN = RL == REC_RUN;
+    PixW e[RUN ? 1 : SR_PER_LANE];   // the entries as full records: .pix is the baseline slot
+    uint32_t rw[RUN ? SR_PER_LANE : 1];
+    V2 rs[RUN && NC == 3 ? SR_PER_LANE : 1];
     T x[SR_PER_LANE];
     int64_t k0 = 0;
     bool head0 = false, cont_last = false;
@@ -288,16 +294,32 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         cont_last = sr_meta_cont(meta);
         // unconditional loads from clamped indices, so that they all issue
         // before the first wait; entries past the end are neutralised after
+        if constexpr (RUN) {
 #pragma unroll
-        for (int u = 0; u < SR_PER_LANE; ++u) {
-            int64_t idx = t0 + u * 64 + lane;
-            e[u] = load_rec_nt<RL>(ent, idx < nent ? idx : nent - 1);
-        }
+            for (int u = 0; u < SR_PER_LANE; ++u) {
+                int64_t idx = t0 + u * 64 + lane;
+                idx = idx < nent ? idx : nent - 1;
+                rw[u] = __builtin_nontemporal_load((const uint32_t *)ent + idx);
+                if (NC == 3) rs[u] = load_wsum_nt<T>(entw, idx);
+            }
+            const uint32_t qmask = (1u << sh) - 1u;
 #pragma unroll
-        for (int u = 0; u < SR_PER_LANE; ++u) {
-            bool ok = t0 + u * 64 + lane < nent && e[u].pix >= 0;
-            T v = pw[ok ? e[u].pix : 0];
-            x[u] = ok ? v : (T)0;
+            for (int u = 0; u < SR_PER_LANE; ++u) {
+                T v = pw[rw[u] & qmask];
+                x[u] = t0 + u * 64 + lane < nent ? v : (T)0;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < SR_PER_LANE; ++u) {
+                int64_t idx = t0 + u * 64 + lane;
+                e[u] = load_rec_nt<RL>(ent, idx < nent ? idx : nent - 1);
+            }
+#pragma unroll
+            for (int u = 0; u < SR_PER_LANE; ++u) {
+                bool ok = t0 + u * 64 + lane < nent && e[u].pix >= 0;
+                T v = pw[ok ? e[u].pix : 0];
+                x[u] = ok ? v : (T)0;
+            }
         }
     }
     T prod[SR_PER_LANE][NC];
@@ -305,8 +327,13 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     for (int c = 0; c < NC; ++c) {
 #pragma unroll
         for (int u = 0; u < SR_PER_LANE; ++u) {
-            float wc = NC == 1 ? 1.0f : (c == 0 ? e[u].w0 : (c == 1 ? e[u].w1 : e[u].w2));
-            tr[w][sr_col(u, lane)] = NC == 1 ? x[u] : (T)wc * x[u];
+            if constexpr (RUN) {
+                T wc = c == 0 ? (T)(rw[u] >> sh) : (c == 1 ? rs[NC == 3 ? u : 0].x : rs[NC == 3 ? u : 0].y);
+                tr[w][sr_col(u, lane)] = wc * x[u];
+            } else {
+                float wc = NC == 1 ? 1.0f : (c == 0 ? e[u].w0 : (c == 1 ? e[u].w1 : e[u].w2));
+                tr[w][sr_col(u, lane)] = NC == 1 ? x[u] : (T)wc * x[u];
+            }
         }
         sr_wave_sync();
 #pragma unroll
@@ -630,8 +657,8 @@ void launch_scatter_seg(hipStream_t s, int nmap, int64_t nent, const void *ent, 
     if (nt == 0) return;
     unsigned grid = (unsigned)((nt + SR_WAVES - 1) / SR_WAVES);
 #define MADAM_SC(NCV, RLV)                                                                                       \
-    k_sr_scatter<T, NCV, SR_WAVES, RLV><<<grid, SR_TPB, 0, s>>>(nent, ent, pw, heads, tile_k0, fix_end, nzq, nzpix,   \
-                                                                 cc_c, m4, part)
+    k_sr_scatter<T, NCV, SR_WAVES, RLV><<<grid, SR_TPB, 0, s>>>(nent, ent, nullptr, 0, pw, heads, tile_k0, fix_end,  \
+                                                                 nzq, nzpix, cc_c, m4, part)
     if (nmap == 1) {
         if (rl == REC4) MADAM_SC(1, REC4);
         else MADAM_SC(1, REC16);
@@ -650,6 +677,32 @@ template void launch_scatter_seg<double>(hipStream_t, int, int64_t, const void *
 template void launch_scatter_seg<float>(hipStream_t, int, int64_t, const void *, int, const float *, const uint8_t *,
                                         const int64_t *, const int64_t *, const int64_t *, const int32_t *, int64_t,
                                         const float *, float *, void *);
+
+template <typename T>
+void launch_scatter_run(hipStream_t s, int nmap, int64_t nrun, const RunView<T> &rv, const T *pw, const uint8_t *heads,
+                        const int64_t *tile_k0, const int64_t *fix_end, const int64_t *fix_ord, const int32_t *nzq,
+                        int64_t nzpix, const T *cc_c, T *m4, void *part_v)
+{
+    using V4 = typename VecT<T>::v4;
+    V4 *part = (V4 *)part_v;
+    int64_t nt = segred_ntiles(nrun);
+    if (nt == 0) return;
+    unsigned grid = (unsigned)((nt + SR_WAVES - 1) / SR_WAVES);
+    if (nmap == 1)
+        k_sr_scatter<T, 1, SR_WAVES, REC_RUN><<<grid, SR_TPB, 0, s>>>(nrun, rv.sword, rv.sw, rv.sh, pw, heads, tile_k0,
+                                                                      fix_end, nzq, nzpix, cc_c, m4, part);
+    else
+        k_sr_scatter<T, 3, SR_WAVES, REC_RUN><<<grid, SR_TPB, 0, s>>>(nrun, rv.sword, rv.sw, rv.sh, pw, heads, tile_k0,
+                                                                      fix_end, nzq, nzpix, cc_c, m4, part);
+    k_sr_scatter_fix<T><<<(unsigned)((nt + SR_TPB - 1) / SR_TPB), SR_TPB, 0, s>>>(nmap, nt, fix_end, fix_ord, nzq,
+                                                                               part, cc_c, m4);
+}
+template void launch_scatter_run<double>(hipStream_t, int, int64_t, const RunView<double> &, const double *,
+                                         const uint8_t *, const int64_t *, const int64_t *, const int64_t *,
+                                         const int32_t *, int64_t, const double *, double *, void *);
+template void launch_scatter_run<float>(hipStream_t, int, int64_t, const RunView<float> &, const float *,
+                                        const uint8_t *, const int64_t *, const int64_t *, const int64_t *,
+                                        const int32_t *, int64_t, const float *, float *, void *);
 
 void launch_gather_seg(hipStream_t s, int nmap, int64_t nent, const PixW *pixw, const double *m4, int64_t ndeg,
                        const uint8_t *heads, const int64_t *tile_k0, const int64_t *fix_end, const int64_t *fix_ord,
