@@ -67,7 +67,7 @@ struct BatchState {
     DBuf<Segment> d_segR;
     DBuf<double> fftwork;
     int64_t fft_nseg = 0;
-    int64_t fft_batch32 = 1;   // segments per FFT batch of the FP32 convolution
+    int64_t fft_batch64 = 1, fft_batch32 = 1;   // segments per FFT batch of the FP64 / FP32 convolution
     // per right-hand side results
     std::vector<BatchScal> hsc, hsc64;
     std::vector<int> inner_steps;
@@ -328,7 +328,7 @@ static void batch_operator(Context &c, BatchState &B, const T *x, T *y, T *pw, T
         if (!c.prior_covers_all) batch_copy<T>(s, y, x, nb * R);
         if (!B.segR.empty())
             fft_convolve_segments<T>(s, c.fft, B.d_segR.p, (int64_t)B.segR.size(), x, y, c.d_fcov.p, c.d_fcov_rows.p,
-                                     c.nof / 2 + 1, B.fftwork.p, Ops<T>::fcov32(B) ? B.fft_batch32 : c.fft_batch,
+                                     c.nof / 2 + 1, B.fftwork.p, Ops<T>::fcov32(B) ? B.fft_batch32 : B.fft_batch64,
                                      B.fft_nseg, B.segR.data(), Ops<T>::fcov32(B));
     } else {
         batch_fill<T>(s, y, (T)0, nb * R);
@@ -363,14 +363,14 @@ static void batch_precond(Context &c, BatchState &B, const T *r, T *z)
         if (!B.segR.empty())
             fft_convolve_segments<T>(s, c.fft, B.d_segR.p, (int64_t)B.segR.size(), r, z, c.d_fprec.p,
                                      c.d_fprec_rows.p, c.nof / 2 + 1, B.fftwork.p,
-                                     Ops<T>::fprec32(B) ? B.fft_batch32 : c.fft_batch, B.fft_nseg,
+                                     Ops<T>::fprec32(B) ? B.fft_batch32 : B.fft_batch64, B.fft_nseg,
                                      B.segR.data(),
                                      Ops<T>::fprec32(B));
         break;
     default:
         if (!c.prec_covers_all) batch_copy<T>(s, z, r, nb * R);
         c.band.chain_pack = band_chain_pack(c.kernel_variant);
-        band_apply<T>(s, c.band, r, z, R, nb);
+        band_apply<T>(s, c.band, r, z, B.nrhs, nb);   // (the padding right-hand sides are inactive)
         if (!c.segcg.empty()) {
             // the inner-CG fallback segments, one right-hand side at a time in FP64
             DBuf<double> r1, z1;
@@ -547,11 +547,18 @@ static void tune_pieces(Context &c, BatchState &B, const Vec<T> &v)
     build_items(c, B, bestp);
 }
 
+// The prior's segments of every right-hand side (the padding ones beyond nrhs
+// hold nothing to convolve), and how many one pass of the convolution takes:
+// as many as keep its work buffer within 128 MiB of the last-level
+// cache, in equal batches.  FP64, five right-hand sides
+// of four segments of 2^16 points: one batch of 20 takes 66 us where eight of
+// 4 (the single solve's batch) took 226; FP32, 128 segments of 2^18 points:
+// two batches of 64 514 us, eight of 16 640.
 static void make_segments(Context &c, BatchState &B)
 {
     B.segR.clear();
     int64_t ns = (int64_t)c.segconv.size();
-    for (int r = 0; r < B.R; ++r)
+    for (int r = 0; r < B.nrhs; ++r)
         for (int64_t i = 0; i < ns; ++i) {
             Segment g = c.segconv[i];
             g.b0 += (int64_t)r * c.nbtot;
@@ -562,12 +569,11 @@ static void make_segments(Context &c, BatchState &B)
         h2d(B.d_segR.p, B.segR.data(), B.segR.size(), c.stream);
     }
     B.fft_nseg = std::max<int64_t>((int64_t)B.segR.size(), 1);
-    // the FP32 work buffer holds twice the segments of the FP64 one in the
-    // same bytes (the batch stays resident in the last-level cache)
-    B.fft_batch32 = std::min<int64_t>(std::min<int64_t>(2 * c.fft_batch, 64), B.fft_nseg);
+    if (!c.p.kfilter) return;
+    B.fft_batch64 = fft_batch_segments(c.fft, B.fft_nseg, sizeof(double2));
+    B.fft_batch32 = fft_batch_segments(c.fft, B.fft_nseg, sizeof(float2));
     if (const char *e = getenv("MADAM_FFT_BATCH32")) B.fft_batch32 = std::max<int64_t>(std::min<int64_t>(atoi(e), 64), 1);
-    if (c.p.kfilter)
-        B.fftwork.alloc(fft_convolve_work_doubles(c.fft, std::max<int64_t>(c.fft_batch, B.fft_batch32), B.fft_nseg));
+    B.fftwork.alloc(fft_convolve_work_doubles(c.fft, std::max<int64_t>(B.fft_batch64, B.fft_batch32), B.fft_nseg));
 }
 
 // binned map and right-hand side of one signal (src/smadam_routines.f90:252-671),

@@ -982,6 +982,14 @@ template void fft_convolve_segments<float>(hipStream_t, const FftPlan &, const S
                                            float *, const double *, const double *, int64_t, double *, int64_t,
                                            int64_t, const Segment *, const float *);
 
+int64_t fft_batch_segments(const FftPlan &p, int64_t nseg, size_t elem)
+{
+    int64_t cap = std::max<int64_t>((128ll << 20) / ((int64_t)elem * p.N), 1);
+    cap = std::min<int64_t>(cap, 512);
+    int64_t nbatch = (nseg + cap - 1) / cap;
+    return (nseg + nbatch - 1) / nbatch;
+}
+
 size_t fft_convolve_work_doubles(const FftPlan &p, int64_t batch, int64_t nseg_max)
 {
     return (size_t)batch * 2 * p.N + (size_t)(batch + 1) / 2 + 1 + (size_t)std::max(batch, nseg_max) * SEG_NB +

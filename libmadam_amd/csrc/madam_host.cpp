@@ -1520,16 +1520,9 @@ void solve_setup(Context &c, const TT *tod)
         double tp = now();
         if (!reuse && p.kfilter) {
             build_filters(c);
-            // batches whose work buffer (16 B per complex point) stays within
-            // 128 MiB, so the row and inverse column passes re-read it from the
-            // 256 MB last-level cache (32 segments of 2^19 points: 2 x 16 is
-            // 6 % faster than 1 x 32; smaller batches leave the GPU underfilled)
             // the inner-CG preconditioner convolves its segments with the same buffers
             int64_t nsc = std::max<int64_t>((int64_t)std::max(c.segconv.size(), c.segp.size()), 1);
-            int64_t cap = std::max<int64_t>((128ll << 20) / (16 * c.fft.N), 1);
-            cap = std::min<int64_t>(cap, 64);
-            int64_t nbatch = (nsc + cap - 1) / cap;
-            c.fft_batch = (nsc + nbatch - 1) / nbatch;
+            c.fft_batch = fft_batch_segments(c.fft, nsc, sizeof(double2));
             // batch buffer, ipsd ints and the per-segment partial sums
             c.d_fftwork.alloc(fft_convolve_work_doubles(c.fft, c.fft_batch, nsc));
             c.fft_nseg_max = nsc;

@@ -365,6 +365,12 @@ void fft_convolve_segments(hipStream_t s, const FftPlan &p, const Segment *dseg,
                            int64_t nseg_max, const Segment *hseg, const float *fc_rows32 = nullptr);
 // fT = fc reordered for the fused row pass: f[r + L1 k2] at [r * L2 + k2], f[N] at [N]
 void fft_spectrum_rows(hipStream_t s, const FftPlan &p, const double *fc, int64_t nrow, int64_t stride, double *fT);
+// segments per batch of the convolution of nseg segments, elem bytes per
+// complex point: equal batches whose work buffer stays within 128 MiB, so that
+// the row and inverse column passes re-read it from the 256 MB last-level
+// cache (32 segments of 2^19 points: 2 x 16 is 6 % faster than 1 x 32; smaller
+// batches leave the GPU underfilled)
+int64_t fft_batch_segments(const FftPlan &p, int64_t nseg, size_t elem);
 // nseg_max: the most segments one fft_convolve_segments call takes
 size_t fft_convolve_work_doubles(const FftPlan &p, int64_t batch, int64_t nseg_max);
 // inverse real FFT of fcov rows (invcov = c2r(fcov) / nof)
