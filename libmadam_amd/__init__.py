@@ -214,19 +214,19 @@ class Madam:
     def maps(self):
         sz = self.sizes()
         npix, nmap = sz["npix"], sz["nmap"]
-        m = np.zeros((npix, nmap))
-        b = np.zeros((npix, nmap))
-        h = np.zeros(npix, np.int32)
-        cc = np.zeros((npix, nmap, nmap))
-        mk = np.zeros(npix, np.int32)
-        cr = np.zeros(npix)
+        m = np.empty((npix, nmap))
+        b = np.empty((npix, nmap))
+        h = np.empty(npix, np.int32)
+        cc = np.empty((npix, nmap, nmap))
+        mk = np.empty(npix, np.int32)
+        cr = np.empty(npix)
         _check(lib().madam_get_maps(self._h, _ptr(m), _ptr(b), _ptr(h), _ptr(cc), _ptr(mk), _ptr(cr)))
         return dict(map=m, binmap=b, hits=h, cc=cc, mask=mk, crit=cr)
 
     def baselines(self):
         sz = self.sizes()
         shape = (sz["ndet"], sz["nbase"])
-        aa, yba, nna = np.zeros(shape), np.zeros(shape), np.zeros(shape)
+        aa, yba, nna = np.empty(shape), np.empty(shape), np.empty(shape)
         _check(lib().madam_get_baselines(self._h, _ptr(aa), _ptr(yba), _ptr(nna)))
         return dict(aa=aa, yba=yba, nna=nna)
 
@@ -286,11 +286,11 @@ class Madam:
         """map, binmap [npix][nmap], aa, yba [ndet][nbase] and the solve info of right-hand side irhs."""
         sz = self.sizes()
         npix, nmap = sz["npix"], sz["nmap"]
-        m = np.zeros((npix, nmap))
-        b = np.zeros((npix, nmap))
+        m = np.empty((npix, nmap))
+        b = np.empty((npix, nmap))
         _check(lib().madam_get_batch_maps(self._h, int(irhs), _ptr(m), _ptr(b)))
-        aa = np.zeros((sz["ndet"], sz["nbase"]))
-        yba = np.zeros((sz["ndet"], sz["nbase"]))
+        aa = np.empty((sz["ndet"], sz["nbase"]))
+        yba = np.empty((sz["ndet"], sz["nbase"]))
         _check(lib().madam_get_batch_baselines(self._h, int(irhs), _ptr(aa), _ptr(yba)))
         keys = ["steps", "status", "rr_inner", "passes", "rr_final", "t_setup", "t_solve", "pcg_steps", "t_pcg",
                 "piece", "t_scatter", "t_prior", "t_gather", "t_prec", "t_step", "n_prof", "rle_records_gather",

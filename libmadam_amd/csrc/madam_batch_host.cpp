@@ -884,24 +884,21 @@ void batch_get_maps(Context &c, int irhs, double *map, double *binmap)
     BatchState &B = batch_of(c, irhs);
     int64_t np = c.npix_map;
     int nm = c.nmap;
-    std::vector<double> m4(np * 4), b4(np * 4);
-    d2h(m4.data(), B.map4.p + (int64_t)irhs * np * 4, np * 4, c.stream);
-    d2h(b4.data(), B.binmap4.p + (int64_t)irhs * np * 4, np * 4, c.stream);
-    MADAM_CHECK(hipStreamSynchronize(c.stream));
-    for (int64_t q = 0; q < np; ++q)
-        for (int a = 0; a < nm; ++a) {
-            if (map) map[q * nm + a] = m4[q * 4 + a];
-            if (binmap) binmap[q * nm + a] = b4[q * 4 + a];
-        }
+    std::vector<OutItem> out;
+    const int mk = nm == 1 ? OUT_MAP1 : OUT_MAP3;
+    if (map) out.push_back({mk, B.map4.p + (int64_t)irhs * np * 4, map, np * nm});
+    if (binmap) out.push_back({mk, B.binmap4.p + (int64_t)irhs * np * 4, binmap, np * nm});
+    copy_out(c, out);
 }
 
 void batch_get_baselines(Context &c, int irhs, double *aa, double *yba)
 {
     BatchState &B = batch_of(c, irhs);
     int64_t nb = c.nbtot;
-    if (aa) d2h(aa, B.a64.p + (int64_t)irhs * nb, nb, c.stream);
-    if (yba) d2h(yba, B.yba.p + (int64_t)irhs * nb, nb, c.stream);
-    MADAM_CHECK(hipStreamSynchronize(c.stream));
+    std::vector<OutItem> out;
+    if (aa) out.push_back({OUT_COPY8, B.a64.p + (int64_t)irhs * nb, aa, nb});
+    if (yba) out.push_back({OUT_COPY8, B.yba.p + (int64_t)irhs * nb, yba, nb});
+    copy_out(c, out);
 }
 
 // out: steps of the (last inner) PCG, its status, its rr / rr0, refinement

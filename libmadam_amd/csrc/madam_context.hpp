@@ -113,7 +113,22 @@ enum { ST_NITER, ST_RRINIT, ST_RZINIT, ST_T_POINTING, ST_T_BIN, ST_T_INIT, ST_T_
        ST_BAND_CHUNKS, ST_BAND_CHUNKS_UNIQUE, ST_BAND_BLOCKS, ST_BAND_BLOCKS_UNIQUE, ST_REC_BYTES,
        ST_BAND_ROWS_FACTORED, ST_PREC_REUSED, ST_POINTING_REUSED, ST_NWIDE, ST_RUN_RECORDS, ST_COUNT };
 
+// ------------------------------------------------------------------ products to the host (madam_out.hip)
+
+enum OutKind { OUT_COPY8, OUT_COPY4, OUT_MAP3, OUT_MAP1, OUT_CC9, OUT_CC1 };
+struct OutItem {
+    int kind;          // layout of the output: 8- or 4-byte values as they are, [npix][3] or [npix] of a map of four
+                       // doubles per pixel, [npix][9] or [npix] of six matrix values per pixel
+    const void *src;   // device
+    void *dst;         // host
+    int64_t n;         // output values
+};
 struct Context;
+// copies on the handle's stream into host memory, complete on return
+void copy_out(Context &c, const std::vector<OutItem> &items);
+void out_handle_made();
+void out_handle_gone();
+
 struct BatchState;
 void batch_release(Context &c);
 void batch_invalidate(Context &c);
@@ -251,12 +266,14 @@ struct Context {
     // batched / mixed-precision solves (madam_batch_host.cpp)
     BatchState *batch = nullptr;
 
+    Context() { out_handle_made(); }
     ~Context()
     {
         batch_release(*this);
         if (band_ready) band_free(band);
         if (fft_ready) fft_plan_free(fft);
         if (stream) (void)hipStreamDestroy(stream);
+        out_handle_gone();
     }
 };
 

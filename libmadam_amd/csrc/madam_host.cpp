@@ -1622,6 +1622,18 @@ static void get_maps(Context &c, double *map, double *binmap, int32_t *hits, dou
     hipStream_t s = c.stream;
     int64_t np = c.npix_map;
     int nm = c.nmap;
+    if (!c.p.rm_monopole) {
+        std::vector<OutItem> out;
+        const int mk = nm == 1 ? OUT_MAP1 : OUT_MAP3, ck = nm == 1 ? OUT_CC1 : OUT_CC9;
+        if (map) out.push_back({mk, c.d_map4.p, map, np * nm});
+        if (binmap) out.push_back({mk, c.d_binmap4.p, binmap, np * nm});
+        if (hits) out.push_back({OUT_COPY4, c.d_hits.p, hits, np});
+        if (cc) out.push_back({ck, c.d_ccinv6.p, cc, np * nm * nm});
+        if (mask) out.push_back({OUT_COPY4, c.d_mask.p, mask, np});
+        if (crit) out.push_back({OUT_COPY8, c.d_crit.p, crit, np});
+        copy_out(c, out);
+        return;
+    }
     std::vector<double> m4(np * 4), b4(np * 4), ci(np * 6);
     std::vector<int32_t> mk(np);
     d2h(m4.data(), c.d_map4.p, np * 4, s);
@@ -1631,17 +1643,15 @@ static void get_maps(Context &c, double *map, double *binmap, int32_t *hits, dou
     if (hits) d2h(hits, c.d_hits.p, np, s);
     if (crit) d2h(crit, c.d_crit.p, np, s);
     MADAM_CHECK(hipStreamSynchronize(s));
-    if (c.p.rm_monopole) {
-        // makemaps monopole removal (src/map_routines.f90:341-353)
-        int64_t cover = 0;
-        for (int64_t q = 0; q < np; ++q) cover += mk[q] > 0;
-        if (cover > 0) {
-            for (auto *v : {&m4, &b4}) {
-                double mono = 0;
-                for (int64_t q = 0; q < np; ++q) mono += (*v)[q * 4];
-                mono = mono / cover;
-                for (int64_t q = 0; q < np; ++q) if (mk[q] > 0) (*v)[q * 4] -= mono;
-            }
+    // makemaps monopole removal (src/map_routines.f90:341-353)
+    int64_t cover = 0;
+    for (int64_t q = 0; q < np; ++q) cover += mk[q] > 0;
+    if (cover > 0) {
+        for (auto *v : {&m4, &b4}) {
+            double mono = 0;
+            for (int64_t q = 0; q < np; ++q) mono += (*v)[q * 4];
+            mono = mono / cover;
+            for (int64_t q = 0; q < np; ++q) if (mk[q] > 0) (*v)[q * 4] -= mono;
         }
     }
     for (int64_t q = 0; q < np; ++q)
@@ -2507,15 +2517,16 @@ MADAM_API int madam_get_baselines(void *ctx, double *aa, double *yba, double *nn
         Context &c = *(Context *)ctx;
         if (!c.solved) fail("no solution available");
         int64_t nb = c.nbtot;
-        if (aa) d2h(aa, c.d_aa.p, nb, c.stream);
+        std::vector<OutItem> out;
+        if (aa) out.push_back({OUT_COPY8, c.d_aa.p, aa, nb});
         if (c.p.kfirst) {
-            if (yba) d2h(yba, c.d_yba.p, nb, c.stream);
-            if (nna) d2h(nna, c.d_nna.p, nb, c.stream);
+            if (yba) out.push_back({OUT_COPY8, c.d_yba.p, yba, nb});
+            if (nna) out.push_back({OUT_COPY8, c.d_nna.p, nna, nb});
         } else {
             if (yba) std::fill(yba, yba + nb, 0.0);
             if (nna) std::fill(nna, nna + nb, 0.0);
         }
-        MADAM_CHECK(hipStreamSynchronize(c.stream));
+        copy_out(c, out);
     });
 }
 
