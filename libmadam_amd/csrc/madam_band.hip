@@ -23,6 +23,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <cstring>
 #include <vector>
 
 #include "madam_internal.hpp"
@@ -306,11 +307,11 @@ struct BandRhs {
     int64_t s, g;
 };
 
-template <typename V>
+// PB: loads in flight per lane before their LDS stores
+template <typename V, int PB = 128 / sizeof(V)>
 __device__ inline void band_tile_in(const V *v, uint32_t b0, int n, V *tile)
 {
     const int lane = threadIdx.x;
-    constexpr int PB = 128 / sizeof(V);   // loads in flight per lane before their LDS stores
 #pragma unroll
     for (int k0 = 0; k0 < 64; k0 += PB) {
         V in[PB];
@@ -895,6 +896,315 @@ __global__ void __launch_bounds__(64) k_band_bwd1(const ChunkInfo *ch, int64_t n
     band_tile_out(z, b0, nc, tile);
 }
 
+// ---------------------------------------------------------------- one-pass solve
+//
+// The carry that leaves a chunk of 64 rows decays fast: for baselines of 0.25,
+// 0.5 and 1 s under a 0.05 Hz knee, T_c ... T_{c-7} is 5e-30, 3e-43 and 1e-65
+// of the state entering the first of the eight chunks (512 rows; 4e-28 with a
+// fifth of the baselines flagged).  Where that product is below BD_NEGLIGIBLE
+// on every window of the factor (checked when it is built, in both
+// directions), the state entering a chunk is, far below an FP64 rounding, a
+// function of the eight chunks before it, and the whole solve is one pass: a
+// wave takes 48 chunks, eight more before and eight after them, one per lane;
+// the zero-carry forward sweep gives every lane its partial state; three
+// doubling steps over the lanes, S_c += T_c S_{c-1}, S_c += T_c T_{c-1}
+// S_{c-2}, S_c += T_c ... T_{c-3} S_{c-4}, gather eight chunks; the second
+// forward sweep leaves y in the LDS tile, and the same goes backward.  r is
+// read once (4/3 times with the halo), z written once, and nothing else moves:
+// where the chains took seven dependent launches between the sweeps
+// (band_apply, the path kept for slower decay and wider bands) the solve is one.
+// Its cost is latency and FP64 issue while blocks are few (37 KB of LDS per
+// wave leave four per CU in FP64, seven in FP32) and, where the factor does not
+// repeat, reading it four times.  Measured, us per apply, chains / one pass:
+//   671 k rows, one right-hand side (repeating factor)      132 / 43
+//   10.7 M rows                                             318 / 153
+//   168 k rows, 5 right-hand sides                          125 / 44
+//   1.3 M rows, 16 right-hand sides, FP32 vectors           396 / 247
+//   1.3 M rows, flagged (no repeats)                        350 / 134
+//   2.4 M rows, flagged                                     400 / 260
+// A repeating factor comes from LDS: as scalar loads (scalar registers hold two
+// rows ahead at most) the first took 60 us, as vector loads of one address 44,
+// but the fourth 404.
+static constexpr int BD_KD = 9, BD_K = BD_KD + 1, BD_KK = BD_KD * BD_KD;
+static constexpr int BD_HALO = 8, BD_OWN = 64 - 2 * BD_HALO;   // chunks per wave on each side, and its own
+static constexpr int BD_LEV = 3;                                // log2(BD_HALO) doubling steps
+static constexpr double BD_NEGLIGIBLE = 5.0e-20;                // 2^-64
+
+// lane l of block b holds chunk base + l, if that lies in the segment's lo .. hi - 1
+struct BandBlk {
+    int32_t base, lo, hi;
+    int32_t uslot;   // >= 0: every chunk of the block has the factor Lu[uslot] and the products PU[uslot]
+};
+
+// products of the transfer matrices T over the 2^l chunks that end at chunk
+// list[t] (dir 0) or start there (dir 1), l = 0, 1, 2: out[(l BD_KK + e) es + t ss].
+// pure[t]: all of them are T of the chunk itself.  Chunks outside the segment
+// never carry a state, so any finite matrix serves for them.
+__global__ void __launch_bounds__(64) k_band_products(const int32_t *list, const uint8_t *pure, int64_t nl,
+                                                      const ChunkInfo *ch, const double *T, int dir, double *out,
+                                                      int64_t es, int64_t ss)
+{
+    int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    int64_t t = g / BD_KD;
+    int j = (int)(g % BD_KD);   // column j of the products
+    if (t >= nl) return;
+    int64_t c = list[t];
+    int64_t at[4];
+    at[0] = c;
+    for (int k = 1; k < 4; ++k) {
+        int64_t prev = at[k - 1];
+        bool end = pure[t] || (dir == 0 ? ch[prev].first : ch[prev].last);
+        at[k] = end ? prev : (dir == 0 ? prev - 1 : prev + 1);
+    }
+    double v[BD_KD];
+    // columns of T_{at[0]} ... T_{at[m - 1]} for m = 1, 2, 4
+    for (int l = 0; l < BD_LEV; ++l) {
+        for (int m = 0; m < BD_KD; ++m) v[m] = m == j ? 1.0 : 0.0;
+        for (int k = (1 << l) - 1; k >= 0; --k) {
+            const double *M = T + at[k] * BD_KK;
+            double w[BD_KD];
+            for (int m = 0; m < BD_KD; ++m) {
+                double a = 0;
+                for (int q = 0; q < BD_KD; ++q) a += M[m * BD_KD + q] * v[q];
+                w[m] = a;
+            }
+            for (int m = 0; m < BD_KD; ++m) v[m] = w[m];
+        }
+        for (int m = 0; m < BD_KD; ++m) out[(int64_t)(l * BD_KK + m * BD_KD + j) * es + t * ss] = v[m];
+    }
+}
+
+// *worst = the largest infinity norm of T over eight consecutive chunks (the
+// bits of a non-negative double compare like an integer)
+__global__ void __launch_bounds__(64) k_band_decay(const int32_t *pslot, int64_t nch, const ChunkInfo *ch,
+                                                   const double *P, int64_t es, int dir, unsigned long long *worst)
+{
+    int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (c >= nch) return;
+    int64_t o = c;
+    for (int k = 0; k < BD_HALO - 1; ++k) {   // the window must lie in the segment
+        if (dir == 0 ? ch[o].first : ch[o].last) return;
+        o += dir == 0 ? -1 : 1;
+    }
+    int64_t c4 = dir == 0 ? c - 4 : c + 4;
+    const double *A = P + 2 * BD_KK * es + pslot[c], *B = P + 2 * BD_KK * es + pslot[c4];
+    double worstv = 0;
+    for (int m = 0; m < BD_KD; ++m) {
+        double sum = 0;
+        for (int j = 0; j < BD_KD; ++j) {
+            double a = 0;
+            for (int q = 0; q < BD_KD; ++q) a += A[(m * BD_KD + q) * es] * B[(q * BD_KD + j) * es];
+            sum += fabs(a);
+        }
+        worstv = sum > worstv || !(sum == sum) ? sum : worstv;
+    }
+    atomicMax(worst, (unsigned long long)__double_as_longlong(worstv == worstv ? fabs(worstv) : 1e300));
+}
+
+// compact row-major copies [i][m] of the factor of chunks list[u]
+__global__ void k_band_compact_chunks(const double *Li, const int32_t *list, int64_t nu, double *Lu)
+{
+    int64_t tot = nu * BAND_CH * BD_K;
+    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < tot; t += (int64_t)gridDim.x * blockDim.x) {
+        int64_t u = t / (BAND_CH * BD_K), im = t % (BAND_CH * BD_K);
+        Lu[t] = li_chunk(Li, nullptr, list[u], BD_K)[im * 64];
+    }
+}
+
+// Factor rows i0 .. i0 + PF - 1 of the lane's chunk and its values there.
+// MS = 64: the interleaved factor, one load per lane; MS = 1: a compact copy,
+// the same for the whole wave, in LDS (broadcast reads).
+template <int MS, typename V>
+struct BdRows {
+    static constexpr int PF = 4;
+    double w[PF][BD_K], h[PF];
+    __device__ inline void load(const double *lic, const V *tl, int i0, int key)
+    {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+            if (MS == 1) {
+                const double2 *row = (const double2 *)(lic + (i0 + u) * BD_K);
+#pragma unroll
+                for (int m = 0; m < BD_K / 2; ++m) {
+                    double2 v = row[m];
+                    w[u][2 * m] = v.x;
+                    w[u][2 * m + 1] = v.y;
+                }
+            } else {
+                const double *row = lic + (int64_t)(i0 + u) * BD_K * MS;
+#pragma unroll
+                for (int m = 0; m < BD_K; ++m) w[u][m] = row[m * MS];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < PF; ++u) h[u] = (double)tl[(i0 + u) ^ key];
+    }
+};
+
+// The sweeps of one chunk, as fwd_sweep and bwd_sweep over all 64 rows (a
+// segment's last chunk has zero factor rows past its end: its rows there stay
+// zero, no state enters it from behind, and none that leaves it is used), with
+// the next rows' loads in flight during the arithmetic of the current ones.
+// The sums are split so that one row waits for the row before it through two
+// dependent operations forward and one backward.
+template <int MS, typename V, bool STORE>
+__device__ inline void bd_fwd(const double *lic, V *tl, double (&S)[BD_KD], int key)
+{
+    constexpr int PF = BdRows<MS, V>::PF;
+    auto rows = [&](const BdRows<MS, V> &R, int i0) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+            double v = fma(S[0], R.w[u][0], R.h[u] * R.w[u][0]);
+#pragma unroll
+            for (int m = 1; m < BD_KD; ++m) S[m - 1] = fma(-R.w[u][m], v, S[m]);
+            S[BD_KD - 1] = -R.w[u][BD_KD] * v;
+            if (STORE) tl[(i0 + u) ^ key] = (V)v;
+        }
+    };
+    BdRows<MS, V> A, B;
+    A.load(lic, tl, 0, key);
+#pragma unroll 1
+    for (int i0 = 0; i0 < BAND_CH; i0 += 2 * PF) {
+        B.load(lic, tl, i0 + PF, key);
+        __builtin_amdgcn_sched_barrier(0);
+        rows(A, i0);
+        A.load(lic, tl, i0 + 2 * PF < BAND_CH ? i0 + 2 * PF : 0, key);
+        __builtin_amdgcn_sched_barrier(0);
+        rows(B, i0 + PF);
+    }
+}
+
+template <int MS, typename V, bool STORE>
+__device__ inline void bd_bwd(const double *lic, V *tl, double (&X)[BD_KD], int key)
+{
+    constexpr int PF = BdRows<MS, V>::PF;
+    auto rows = [&](const BdRows<MS, V> &R, int i0) {
+#pragma unroll
+        for (int u = PF - 1; u >= 0; --u) {
+            const double d = R.w[u][0];
+            // the rows further on in two chains, the row just done last
+            double s = R.h[u], t = R.w[u][3] * X[2];
+            s = fma(-R.w[u][2], X[1], s);
+#pragma unroll
+            for (int m = 4; m <= BD_KD; m += 2) s = fma(-R.w[u][m], X[m - 1], s);
+#pragma unroll
+            for (int m = 5; m <= BD_KD; m += 2) t = fma(R.w[u][m], X[m - 1], t);
+            double xi = fma(-(R.w[u][1] * d), X[0], (s - t) * d);
+#pragma unroll
+            for (int m = BD_KD - 1; m > 0; --m) X[m] = X[m - 1];
+            X[0] = xi;
+            if (STORE) tl[(i0 + u) ^ key] = (V)xi;
+        }
+    };
+    BdRows<MS, V> A, B;
+    A.load(lic, tl, BAND_CH - PF, key);
+#pragma unroll 1
+    for (int i0 = BAND_CH - PF; i0 >= 0; i0 -= 2 * PF) {
+        B.load(lic, tl, i0 - PF, key);
+        __builtin_amdgcn_sched_barrier(0);
+        rows(A, i0);
+        A.load(lic, tl, i0 >= 2 * PF ? i0 - 2 * PF : 0, key);
+        __builtin_amdgcn_sched_barrier(0);
+        rows(B, i0 - PF);
+    }
+}
+
+// S += P_l (S of the lane 2^l before (dir 0) or after (dir 1)), l = 0, 1, 2;
+// then the state entering the lane's chunk.  P element e of level l at
+// P[(l BD_KK + e) es].
+template <int DIR>
+__device__ inline void bd_carry(double (&S)[BD_KD], const double *P, int64_t es)
+{
+    const int lane = threadIdx.x;
+#pragma unroll 1
+    for (int l = 0; l < BD_LEV; ++l) {
+        // every load of the level before the first use (left to the
+        // scheduler each product waits for its own: 138 us instead of 44 for
+        // one right-hand side of 671 k rows)
+        double M[BD_KK];
+#pragma unroll
+        for (int e = 0; e < BD_KK; ++e) M[e] = P[(int64_t)(l * BD_KK + e) * es];
+        __builtin_amdgcn_sched_barrier(0);
+        double o[BD_KD];
+#pragma unroll
+        for (int q = 0; q < BD_KD; ++q) {
+            double x = DIR == 0 ? __shfl_up(S[q], 1 << l, 64) : __shfl_down(S[q], 1 << l, 64);
+            o[q] = (DIR == 0 ? lane >= (1 << l) : lane + (1 << l) < 64) ? x : 0.0;
+        }
+#pragma unroll
+        for (int m = 0; m < BD_KD; ++m) {
+            double a = 0;
+#pragma unroll
+            for (int q = 0; q < BD_KD; ++q) a = fma(M[m * BD_KD + q], o[q], a);
+            S[m] += a;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < BD_KD; ++q) {
+        double x = DIR == 0 ? __shfl_up(S[q], 1, 64) : __shfl_down(S[q], 1, 64);
+        S[q] = (DIR == 0 ? lane > 0 : lane < 63) ? x : 0.0;
+    }
+}
+
+template <int MS, typename V>
+__device__ inline void bd_solve(const double *lic, const double *Pf, const double *Pb, int64_t es, bool valid, V *tl,
+                                int key)
+{
+    double S[BD_KD];
+#pragma unroll
+    for (int m = 0; m < BD_KD; ++m) S[m] = 0;
+    bd_fwd<MS, V, false>(lic, tl, S, key);
+    bd_carry<0>(S, Pf, es);
+    bd_fwd<MS, V, true>(lic, tl, S, key);
+#pragma unroll
+    for (int m = 0; m < BD_KD; ++m) S[m] = 0;
+    bd_bwd<MS, V, false>(lic, tl, S, key);
+    // lanes outside the segment send nothing back into it
+#pragma unroll
+    for (int m = 0; m < BD_KD; ++m) S[m] = valid ? S[m] : 0.0;
+    bd_carry<1>(S, Pb, es);
+    bd_bwd<MS, V, true>(lic, tl, S, key);
+}
+
+// z = M^-1 r (r and z do not overlap: the halo of one block is another's own)
+template <typename V>
+__global__ void __launch_bounds__(64) k_band_direct(const BandBlk *__restrict__ blk, const ChunkInfo *__restrict__ ch,
+                                                    const int32_t *bmap, const double *Li,
+                                                    const double *__restrict__ Lu, const double *__restrict__ Pf,
+                                                    const double *__restrict__ Pb, const int32_t *__restrict__ pslot,
+                                                    int64_t nslot, const double *__restrict__ PU,
+                                                    const V *__restrict__ r, V *__restrict__ z, int64_t vstride)
+{
+    __shared__ V tile[64 * 64];
+    __shared__ __align__(16) double fac[BAND_CH * BD_K];
+    r += blockIdx.y * vstride;
+    z += blockIdx.y * vstride;
+    const int lane = threadIdx.x;
+    const BandBlk b = blk[blockIdx.x];
+    const int c = b.base + lane;
+    const bool valid = c >= b.lo && c < b.hi;
+    const uint32_t b0 = valid ? (uint32_t)ch[c].b0 : 0u;
+    const int n = valid ? ch[c].n : 0;
+    if (b.uslot >= 0) {
+        const double2 *lu = (const double2 *)(Lu + (int64_t)b.uslot * BAND_CH * BD_K);
+#pragma unroll
+        for (int k = 0; k < BD_K / 2; ++k) ((double2 *)fac)[k * 64 + lane] = lu[k * 64 + lane];
+    }
+    band_tile_in<V, 32>(r, b0, n, tile);
+    V *tl = tile + lane * 64;
+    if (b.uslot >= 0) {
+        int vz;   // a zero the compiler takes for a lane's own value: vector loads (scalar ones wait one batch at a time)
+        asm volatile("v_mov_b32 %0, 0" : "=v"(vz));
+        const double *pu = PU + (int64_t)b.uslot * 2 * BD_LEV * BD_KK + vz;
+        bd_solve<1, V>(fac, pu, pu + BD_LEV * BD_KK, 1, valid, tl, lane);
+    } else {
+        const int cc = valid ? c : b.lo;
+        const int64_t sl = pslot[cc];
+        bd_solve<64, V>(li_chunk(Li, bmap, cc, BD_K), Pf + sl, Pb + sl, nslot, valid, tl, lane);
+    }
+    band_tile_out(z, b0, lane >= BD_HALO && lane < 64 - BD_HALO ? n : 0, tile);
+}
+
 // ---------------------------------------------------------------- host side
 
 struct BandImpl {
@@ -917,6 +1227,12 @@ struct BandImpl {
     int32_t *uidx = nullptr;
     double *Lu = nullptr;
     int rcap = 1;   // right-hand sides the carry-state buffers hold
+    // one-pass solve (k_band_direct): blocks, product slots of the chunks
+    bool direct = false;
+    int64_t nblk = 0, nslot = 0;
+    BandBlk *blk = nullptr;
+    int32_t *pslot = nullptr;
+    double *Pf = nullptr, *Pb = nullptr, *PU = nullptr, *LuD = nullptr;
 };
 
 static int kd_class(int kd)
@@ -935,6 +1251,9 @@ static int kd_class(int kd)
     case 39: { constexpr int KD = 39; STMT; } break;      \
     default: { constexpr int KD = 49; STMT; } break;      \
     }
+
+static void band_build_direct(hipStream_t s, const BandPrec &bp, BandImpl *im, const std::vector<int64_t> &first,
+                              const std::vector<int32_t> &cmap);
 
 // Returns 0 on success; fills info_out[s] (0 ok, >0 failing column) for each segment.
 int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *dseg, int64_t nseg,
@@ -1138,10 +1457,104 @@ int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *
         MADAM_CHECK(hipMalloc(&im->bmap, sizeof(int32_t) * bmap.size()));
         MADAM_CHECK(hipMemcpyAsync(im->cmap, cmap.data(), sizeof(int32_t) * cmap.size(), hipMemcpyHostToDevice, s));
         MADAM_CHECK(hipMemcpyAsync(im->bmap, bmap.data(), sizeof(int32_t) * bmap.size(), hipMemcpyHostToDevice, s));
+        MADAM_CHECK(hipStreamSynchronize(s));   // the host tables above
+        band_build_direct(s, bp, im, first, cmap);
     }
     bp.impl = im;
     MADAM_CHECK(hipStreamSynchronize(s));
     return 0;
+}
+
+// tables of the one-pass solve; leaves im->direct false where the carry
+// decays too slowly for it
+static void band_build_direct(hipStream_t s, const BandPrec &bp, BandImpl *im, const std::vector<int64_t> &first,
+                              const std::vector<int32_t> &cmap)
+{
+    const int64_t nch = bp.nchunk;
+    if (bp.kd != BD_KD || nch == 0 || nch > INT32_MAX - 128) return;
+    // A chunk whose neighbours up to three away (inside the segment) are all
+    // its equals shares the products of its run.
+    std::vector<int32_t> pslot(nch), list;
+    std::vector<uint8_t> pure;
+    std::vector<BandBlk> blk;
+    std::vector<int32_t> urep, uslot;   // chunks and product slots of the uniform blocks
+    for (int64_t si = 0; si < im->nseg_used; ++si) {
+        const int64_t lo = first[si], hi = first[si + 1];
+        for (int64_t c = lo; c < hi; ++c) {
+            bool pu = true;
+            for (int64_t k = std::max(lo, c - 3); k <= std::min(hi - 1, c + 3) && pu; ++k) pu = cmap[k] == cmap[c];
+            if (pu && c > lo && pure[pslot[c - 1]] && cmap[c] == cmap[c - 1]) {
+                pslot[c] = pslot[c - 1];
+                continue;
+            }
+            pslot[c] = (int32_t)list.size();
+            list.push_back((int32_t)c);
+            pure.push_back(pu ? 1 : 0);
+        }
+        for (int64_t c0 = lo; c0 < hi; c0 += BD_OWN) {
+            BandBlk b{(int32_t)(c0 - BD_HALO), (int32_t)lo, (int32_t)hi, -1};
+            int64_t a = std::max(lo, c0 - BD_HALO), e = std::min(hi, c0 - BD_HALO + 64);
+            bool uni = true;
+            for (int64_t c = a + 1; c < e && uni; ++c) uni = cmap[c] == cmap[a] && pslot[c] == pslot[a];
+            if (uni && pure[pslot[a]]) {
+                if (uslot.empty() || uslot.back() != pslot[a]) {
+                    urep.push_back((int32_t)a);
+                    uslot.push_back(pslot[a]);
+                }
+                b.uslot = (int32_t)uslot.size() - 1;
+            }
+            blk.push_back(b);
+        }
+    }
+    const int64_t ns = (int64_t)list.size(), nu = (int64_t)urep.size(), np = BD_LEV * BD_KK;
+    im->nblk = (int64_t)blk.size();
+    im->nslot = ns;
+    int32_t *dlist = nullptr, *durep = nullptr;
+    uint8_t *dpure = nullptr;
+    unsigned long long *dworst = nullptr, worst = 0;
+    MADAM_CHECK(hipMalloc(&im->blk, sizeof(BandBlk) * blk.size()));
+    MADAM_CHECK(hipMalloc(&im->pslot, sizeof(int32_t) * nch));
+    MADAM_CHECK(hipMalloc(&im->Pf, sizeof(double) * np * ns));
+    MADAM_CHECK(hipMalloc(&im->Pb, sizeof(double) * np * ns));
+    MADAM_CHECK(hipMalloc(&im->PU, sizeof(double) * 2 * np * std::max<int64_t>(nu, 1)));
+    MADAM_CHECK(hipMalloc(&im->LuD, sizeof(double) * BAND_CH * BD_K * std::max<int64_t>(nu, 1)));
+    MADAM_CHECK(hipMalloc(&dlist, sizeof(int32_t) * ns));
+    MADAM_CHECK(hipMalloc(&dpure, ns));
+    MADAM_CHECK(hipMalloc(&durep, sizeof(int32_t) * std::max<int64_t>(nu, 1)));
+    MADAM_CHECK(hipMalloc(&dworst, sizeof(unsigned long long)));
+    MADAM_CHECK(hipMemsetAsync(dworst, 0, sizeof(unsigned long long), s));
+    MADAM_CHECK(hipMemcpyAsync(im->blk, blk.data(), sizeof(BandBlk) * blk.size(), hipMemcpyHostToDevice, s));
+    MADAM_CHECK(hipMemcpyAsync(im->pslot, pslot.data(), sizeof(int32_t) * nch, hipMemcpyHostToDevice, s));
+    MADAM_CHECK(hipMemcpyAsync(dlist, list.data(), sizeof(int32_t) * ns, hipMemcpyHostToDevice, s));
+    MADAM_CHECK(hipMemcpyAsync(dpure, pure.data(), ns, hipMemcpyHostToDevice, s));
+    unsigned g = (unsigned)((ns * BD_KD + 63) / 64), gc = (unsigned)((nch + 63) / 64);
+    k_band_products<<<g, 64, 0, s>>>(dlist, dpure, ns, im->ch, bp.Tf, 0, im->Pf, ns, 1);
+    k_band_products<<<g, 64, 0, s>>>(dlist, dpure, ns, im->ch, bp.Tb, 1, im->Pb, ns, 1);
+    k_band_decay<<<gc, 64, 0, s>>>(im->pslot, nch, im->ch, im->Pf, ns, 0, dworst);
+    k_band_decay<<<gc, 64, 0, s>>>(im->pslot, nch, im->ch, im->Pb, ns, 1, dworst);
+    if (nu > 0) {
+        std::vector<uint8_t> one(nu, 1);
+        MADAM_CHECK(hipMemcpyAsync(durep, urep.data(), sizeof(int32_t) * nu, hipMemcpyHostToDevice, s));
+        MADAM_CHECK(hipMemcpyAsync(dpure, one.data(), nu, hipMemcpyHostToDevice, s));
+        unsigned gu = (unsigned)((nu * BD_KD + 63) / 64);
+        k_band_products<<<gu, 64, 0, s>>>(durep, dpure, nu, im->ch, bp.Tf, 0, im->PU, 1, 2 * np);
+        k_band_products<<<gu, 64, 0, s>>>(durep, dpure, nu, im->ch, bp.Tb, 1, im->PU + np, 1, 2 * np);
+        k_band_compact_chunks<<<(unsigned)std::min<int64_t>((nu * BAND_CH * BD_K + 255) / 256, 65535), 256, 0, s>>>(
+            im->Li, durep, nu, im->LuD);
+        MADAM_CHECK(hipGetLastError());
+        MADAM_CHECK(hipStreamSynchronize(s));   // one
+    }
+    MADAM_CHECK(hipGetLastError());
+    MADAM_CHECK(hipMemcpyAsync(&worst, dworst, sizeof(worst), hipMemcpyDeviceToHost, s));
+    MADAM_CHECK(hipStreamSynchronize(s));
+    (void)hipFree(dlist);
+    (void)hipFree(dpure);
+    (void)hipFree(durep);
+    (void)hipFree(dworst);
+    double w;
+    static_assert(sizeof w == sizeof worst, "");
+    memcpy(&w, &worst, sizeof w);
+    im->direct = w < BD_NEGLIGIBLE;
 }
 
 // grow the carry-state buffers to nrhs right-hand sides
@@ -1174,6 +1587,12 @@ void band_apply(hipStream_t s, const BandPrec &bp, const T *r, T *z, int nrhs, i
                        __FILE__, __LINE__);
     int KD = bp.kd;
     unsigned R = (unsigned)nrhs;
+    if (im->direct && bp.chain_pack < 0 && r != z) {
+        k_band_direct<T><<<dim3((unsigned)im->nblk, R), 64, 0, s>>>(im->blk, im->ch, im->bmap, im->Li, im->LuD, im->Pf,
+                                                                    im->Pb, im->pslot, im->nslot, im->PU, r, z,
+                                                                    vstride);
+        return;
+    }
     dim3 g((unsigned)((bp.nchunk + 63) / 64), R);
     dim3 gs((unsigned)im->nseg_used, R);   // one 64-lane wave per segment
     BandRhs st{bp.nchunk * KD, (im->ngrp > 0 ? im->ngrp : 1) * KD};
@@ -1235,6 +1654,10 @@ void band_free(BandPrec &bp)
         (void)hipFree(im->Gb);
         (void)hipFree(im->cg);
         (void)hipFree(im->Sg);
+        for (double *p : {im->Pf, im->Pb, im->PU, im->LuD})
+            if (p) (void)hipFree(p);
+        if (im->blk) (void)hipFree(im->blk);
+        if (im->pslot) (void)hipFree(im->pslot);
         delete im;
     }
     if (bp.L) (void)hipFree(bp.L);
