@@ -415,7 +415,11 @@ static void pcg_step(Context &c, BatchState &B, const Vec<T> &v, double lim, int
     if (tm) tm->pc.stop(s);
     batch_dots<T>(s, 1, R, v.r, v.z, lean ? v.ap : v.ro, c.d_rmask.p, nb, B.dots.p);
     batch_final(s, R, B.dots.p, lean ? 4 : 1, B.sc.p, B.active.p, lim, iter_min, iter_max, nullptr, stall);
-    batch_update_p_pw<T>(s, R, B.sc.p, B.active.p, v.p, v.z, nb, c.d_bslot.p, Ops<T>::dwb(c, B), v.pw);
+    if (R == 1)
+        launch_update_p_slots<T>(s, c.ndet, c.nbase, &B.sc.p->beta, nullptr, B.active.p, v.p, v.z, c.d_bslot.p,
+                                 Ops<T>::dwb(c, B), v.pw);
+    else
+        batch_update_p_pw<T>(s, R, B.sc.p, B.active.p, v.p, v.z, nb, c.d_bslot.p, Ops<T>::dwb(c, B), v.pw);
     if (tm) {
         tm->st.stop(s);
         B.t_scatter += tm->sc.ms() * 1e-3;

@@ -287,7 +287,11 @@ void launch_finalize_scalars(hipStream_t s, const double *partials, int nblocks,
 // PCG vector steps, scalars read from device memory
 void launch_pcg_update_r(hipStream_t s, const double *scal, double *aa, double *r, double *ro, const double *p,
                          const double *ap, int64_t n);
-void launch_pcg_update_p(hipStream_t s, const double *scal, double *p, const double *z, int64_t n);
+// p = z + *beta p, pw[bslot[b]] = p[b] dwb[b]; nothing where *done != 0 (null:
+// never); where *active == 0 (null: never) p stays and pw is zero
+template <typename T>
+void launch_update_p_slots(hipStream_t s, int ndet, int64_t nbase, const double *beta, const double *done,
+                           const int *active, T *p, const T *z, const int32_t *bslot, const T *dwb, T *pw);
 void launch_axpby_nna(hipStream_t s, double *ap, const double *nna, const double *p, double factor, int64_t n);
 
 void launch_minmax(hipStream_t s, const int32_t *pix, int64_t n, int *mn, int *mx);

@@ -1626,17 +1626,78 @@ void launch_pcg_update_r(hipStream_t s, const double *scal, double *aa, double *
     k_update_r<<<grid_for(n, TPB), TPB, 0, s>>>(scal, aa, r, ro, p, ap, n);
 }
 
-__global__ void k_update_p(const double *scal, double *p, const double *z, int64_t n)
+// p = z + beta p and the next step's pixel-side input pw[bslot[b]] = p[b]
+// dwb[b], in one pass.  A block takes US_K baselines of US_D detectors: p, z,
+// dwb and the slots are read in baseline order (coalesced), and the products
+// are written from LDS with the detectors fastest.  The slots of co-pointed
+// detectors at one time are neighbours (baseline_slots), so a wave's store
+// touches one cache line per baseline instead of one per (baseline, detector).
+// Bound by those scattered writes.  Measured: FP32, 21.5 M baselines of 32
+// detectors, 552 us in plain baseline order, 130 now (step 4.58 -> 4.04 ms);
+// FP64, 10.7 M of 16 detectors, 180 us as the update and a gather through the
+// slot order, 115 now (step 2.54 -> 2.47 ms).
+// active (null: on) zeroes pw and leaves p of a finished right-hand side.
+static constexpr int US_D = 4, US_K = TPB;
+static constexpr int US_ROW = US_K + 16;   // LDS row stride: two detectors' rows start half the banks apart
+
+template <typename T>
+__global__ void __launch_bounds__(TPB) k_update_p_slots(int ndet, int64_t nbase, const double *beta_p,
+                                                        const double *done, const int *active, T *__restrict__ p,
+                                                        const T *__restrict__ z, const int32_t *__restrict__ bslot,
+                                                        const T *__restrict__ dwb, T *__restrict__ pw)
 {
-    double beta = scal[5];
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = z[i] + beta * p[i];
+    if (done && *done != 0.0) return;
+    __shared__ T v[US_D * US_ROW];
+    __shared__ int32_t sl[US_D * US_ROW];
+    int64_t ngrp = (ndet + US_D - 1) / US_D;
+    int64_t lb = xcd_block(blockIdx.x, gridDim.x);
+    int64_t kb = lb / ngrp;
+    int d0 = (int)(lb - kb * ngrp) * US_D;
+    int nd = ndet - d0 < US_D ? ndet - d0 : US_D;
+    int64_t k0 = kb * US_K;
+    int nk = (int)(nbase - k0 < US_K ? nbase - k0 : US_K);
+    const bool on = !active || active[0] != 0;
+    const T beta = (T)*beta_p;
+    const int t = threadIdx.x;
+    if (t < nk) {
+        T pi[US_D], zi[US_D], wi[US_D];
+        int32_t si[US_D];
+#pragma unroll
+        for (int d = 0; d < US_D; ++d) {
+            int64_t b = (int64_t)(d0 + (d < nd ? d : 0)) * nbase + k0 + t;
+            pi[d] = p[b];
+            zi[d] = z[b];
+            wi[d] = dwb[b];
+            si[d] = bslot[b];
+        }
+#pragma unroll
+        for (int d = 0; d < US_D; ++d) {
+            T x = zi[d] + beta * pi[d];
+            if (d < nd && on) p[(int64_t)(d0 + d) * nbase + k0 + t] = x;
+            v[d * US_ROW + t] = on ? x * wi[d] : (T)0;
+            sl[d * US_ROW + t] = si[d];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < US_D; ++u) {
+        int i = u * TPB + t, k = i / US_D, d = i % US_D;
+        if (k < nk && d < nd) pw[sl[d * US_ROW + k]] = v[d * US_ROW + k];
+    }
 }
 
-void launch_pcg_update_p(hipStream_t s, const double *scal, double *p, const double *z, int64_t n)
+template <typename T>
+void launch_update_p_slots(hipStream_t s, int ndet, int64_t nbase, const double *beta, const double *done,
+                           const int *active, T *p, const T *z, const int32_t *bslot, const T *dwb, T *pw)
 {
-    k_update_p<<<grid_for(n, TPB), TPB, 0, s>>>(scal, p, z, n);
+    int64_t grid = ((ndet + US_D - 1) / US_D) * ((nbase + US_K - 1) / US_K);
+    if (grid > 0)
+        k_update_p_slots<T><<<(unsigned)grid, TPB, 0, s>>>(ndet, nbase, beta, done, active, p, z, bslot, dwb, pw);
 }
+template void launch_update_p_slots<double>(hipStream_t, int, int64_t, const double *, const double *, const int *,
+                                            double *, const double *, const int32_t *, const double *, double *);
+template void launch_update_p_slots<float>(hipStream_t, int, int64_t, const double *, const double *, const int *,
+                                           float *, const float *, const int32_t *, const float *, float *);
 
 __global__ void k_gather_order(const double *in, const int32_t *ord, double *out, int64_t n)
 {
