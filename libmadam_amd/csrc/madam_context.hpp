@@ -239,6 +239,8 @@ struct Context {
     bool fft_ready = false;
     int64_t fft_batch = 0, fft_nseg_max = 0;
     int precond_kind = 0;
+    DBuf<unsigned> d_dotcnt;      // block count of the dot products, 0 between launches
+    double *h_steps = nullptr;    // pinned: rz and rr of the last PCG steps
     // inner-CG preconditioner segments (band width criterion or Cholesky failed)
     std::vector<Segment> segcg;
     std::vector<double> ic0cg;
@@ -273,6 +275,7 @@ struct Context {
         if (band_ready) band_free(band);
         if (fft_ready) fft_plan_free(fft);
         if (stream) (void)hipStreamDestroy(stream);
+        if (h_steps) (void)hipHostFree(h_steps);
         out_handle_gone();
     }
 };
@@ -332,14 +335,14 @@ void solve_setup(Context &c, const TT *tod);
 void cg_apply(Context &c, const double *r, double *z);
 // the two projections of one right-hand side, from the run records where the
 // pointing has them: m4 = ccinv P^T W F p (pw = p dwb in slot order), and
-// ap += nna p - F^T W P m4
+// ap += nna p - F^T W P m4 (add 0: ap =)
 // the FP32 weight sums of the run records, before FP32 projections (allocates:
 // call outside graph capture)
 void runs_prepare_fp32(Context &c);
 template <typename T>
 void project_to_map(Context &c, const T *pw, const T *cc_c, T *m4);
 template <typename T>
-void project_to_baselines(Context &c, const T *m4, const T *dwb, const T *nna, const T *p, T *ap);
+void project_to_baselines(Context &c, const T *m4, const T *dwb, const T *nna, const T *p, T *ap, int add = 1);
 
 // batched and mixed-precision solves (madam_batch_host.cpp)
 void solve_batch(Context &c, int nrhs, const void *signals, int tod_f32, int on_device, int precision);

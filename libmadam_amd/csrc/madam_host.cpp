@@ -920,19 +920,19 @@ template void project_to_map<double>(Context &, const double *, const double *, 
 template void project_to_map<float>(Context &, const float *, const float *, float *);
 
 template <typename T>
-void project_to_baselines(Context &c, const T *m4, const T *dwb, const T *nna, const T *p, T *ap)
+void project_to_baselines(Context &c, const T *m4, const T *dwb, const T *nna, const T *p, T *ap, int add)
 {
     if (use_runs<T>(c))
-        launch_gather_run<T>(c.stream, c.nmap, c.ndet, c.nbase, run_view<T>(c), m4, dwb, nna, p, ap);
+        launch_gather_run<T>(c.stream, c.nmap, c.ndet, c.nbase, run_view<T>(c), m4, dwb, nna, p, ap, add);
     else
         launch_gather_flat<T>(c.stream, c.nmap, c.ndet, c.nsamp, c.nbase, c.d_bstart.p,
                               c.rec_layout == REC16 ? (const void *)c.d_pixw.p : c.d_pixc.p, c.rec_layout, m4, c.ndeg,
-                              dwb, nna, p, ap);
+                              dwb, nna, p, ap, add);
 }
 template void project_to_baselines<double>(Context &, const double *, const double *, const double *, const double *,
-                                           double *);
+                                           double *, int);
 template void project_to_baselines<float>(Context &, const float *, const float *, const float *, const float *,
-                                          float *);
+                                          float *, int);
 
 // segment tables of the two projections; they depend on the pointing only
 static void build_segtiles(Context &c)
@@ -1295,6 +1295,10 @@ static void pcg_init(Context &c)
     int64_t nb = c.nbtot;
     for (auto *b : {&c.d_r, &c.d_ro, &c.d_z, &c.d_p, &c.d_pw, &c.d_ap}) b->alloc(nb);
     c.d_scal.alloc(8);
+    if (!c.d_dotcnt.p) {
+        c.d_dotcnt.alloc(1);
+        MADAM_CHECK(hipMemsetAsync(c.d_dotcnt.p, 0, sizeof(unsigned), s));
+    }
     int nblk = dots_nblocks(nb);
     c.d_part.alloc((size_t)nblk * 3);
     launch_fill(s, c.d_aa.p, 0.0, nb);
@@ -1317,78 +1321,89 @@ static void pcg_init(Context &c)
 
 // PCG iterations (src/smadam_routines.f90:785-924).  With converge = false the
 // exit tests are skipped and exactly nmax iterations run (benchmark mode).
-static int pcg_steps(Context &c, int nmax, bool converge)
+//
+// The exit tests are made on the device, which leaves the solution and the
+// scalars of an ended solve alone, so a step is queued before the host has
+// seen the one before it: the device does not wait for the host between steps
+// (40 us of a 300 us step at 4 x 2^22 samples).  Only within SPECULATE of the
+// limit does the host look first, so that no whole step is spent in vain.
+static constexpr double SPECULATE = 30;
+
+static void pcg_step(Context &c, const PcgExit &exit, Timer *t_sc, Timer *t_pr, Timer *t_ga, Timer *t_pc)
 {
     hipStream_t s = c.stream;
     const Params &p = c.p;
     int64_t nb = c.nbtot;
-    int nblk = dots_nblocks(nb);
-    int grp = group_for(c);
-    double rrinit = c.stats[ST_RRINIT];
-    double hs[8];
-    Timer t_sc, t_ga, t_pr, t_pc, t_it;
-    int prof = c.profile;
-    int done = 0;
-    for (;;) {
-        if (done >= nmax) break;
-        done++;
-        c.pcg_steps_done++;
-        if (prof) { t_it.start(s); t_sc.start(s); }
-        if ((c.kernel_variant & 15) == 0)   // segmented tiles (default)
-            project_to_map<double>(c, c.d_pw.p, c.d_ccinv_c.p, c.d_m4x.p);
-        else if ((c.kernel_variant & 15) == 3)
-            launch_scatter_seg(s, c.nmap, c.nactive, c.rec_layout == REC16 ? (const void *)c.d_ent.p : c.d_entc.p,
-                               c.rec_layout, c.d_pw.p, c.sr_s.heads.p, c.sr_s.k0.p,
-                               c.sr_s.fix_end.p, c.sr_s.fix_ord.p, c.d_nzq.p, c.nzpix, c.d_ccinv_c.p, c.d_m4x.p,
-                               c.d_sr_part.p);
-        else if ((c.kernel_variant & 15) == 2)
-            launch_scatter_tiles(s, c.nmap, c.npix_cross, c.ndeg, c.d_off.p, c.nactive, c.d_ent.p, c.d_pw.p,
-                                 c.d_ccinv6x.p, c.d_m4x.p, c.d_tileinfo.p, c.d_tilescratch.p);
-        else
-            launch_scatter_pixels(s, c.nmap, c.npix_cross, c.ndeg, c.d_off.p, c.d_ent.p, c.d_pw.p, c.d_ccinv6x.p,
-                                  c.d_m4x.p);
-        if (prof) { t_sc.stop(s); t_pr.start(s); }
-        if (p.kfilter) apply_prior(c, c.d_p.p, c.d_ap.p);
-        else if (p.diagfilter != 0) launch_axpby_nna(s, c.d_ap.p, c.d_nna.p, c.d_p.p, p.diagfilter, nb);
-        else launch_fill(s, c.d_ap.p, 0.0, nb);
-        if (prof) { t_pr.stop(s); t_ga.start(s); }
-        if ((c.kernel_variant & 15) == 3 && c.sr_g.ok)
-            launch_gather_seg(s, c.nmap, (int64_t)c.ndet * c.nsamp, c.d_pixw.p, c.d_m4x.p, c.ndeg, c.sr_g.heads.p,
-                              c.sr_g.k0.p, c.sr_g.fix_end.p, c.sr_g.fix_ord.p, c.d_dwb.p, c.d_nna.p, c.d_p.p,
-                              c.d_ap.p, c.d_sr_part.p);
-        else if ((c.kernel_variant & 15) == 0)
-            project_to_baselines<double>(c, c.d_m4x.p, c.d_dwb.p, c.d_nna.p, c.d_p.p, c.d_ap.p);
-        else if ((c.kernel_variant & 15) != 1)
-            launch_gather_flat(s, c.nmap, c.ndet, c.nsamp, c.nbase, c.d_bstart.p,
-                               c.rec_layout == REC16 ? (const void *)c.d_pixw.p : c.d_pixc.p, c.rec_layout,
-                               c.d_m4x.p, c.ndeg, c.d_dwb.p, c.d_nna.p, c.d_p.p, c.d_ap.p);
-        else
-            launch_gather_baselines(s, c.nmap, c.ndet, c.nsamp, c.nbase, c.d_bstart.p, c.d_pixw.p, c.d_m4x.p, c.ndeg,
-                                    c.d_dwb.p, c.d_nna.p, c.d_p.p, c.d_ap.p, grp);
-        if (prof) t_ga.stop(s);
-        launch_dots(s, 0, c.d_p.p, c.d_ap.p, nullptr, nullptr, c.d_rmask.p, nb, c.d_part.p, nblk);
-        launch_finalize(s, c.d_part.p, nblk, 1, c.d_scal.p + 1);
+    const int variant = c.kernel_variant & 15;
+    if (t_sc) t_sc->start(s);
+    if (variant == 0)   // segmented tiles (default)
+        project_to_map<double>(c, c.d_pw.p, c.d_ccinv_c.p, c.d_m4x.p);
+    else if (variant == 3)
+        launch_scatter_seg(s, c.nmap, c.nactive, c.rec_layout == REC16 ? (const void *)c.d_ent.p : c.d_entc.p,
+                           c.rec_layout, c.d_pw.p, c.sr_s.heads.p, c.sr_s.k0.p, c.sr_s.fix_end.p, c.sr_s.fix_ord.p,
+                           c.d_nzq.p, c.nzpix, c.d_ccinv_c.p, c.d_m4x.p, c.d_sr_part.p);
+    else if (variant == 2)
+        launch_scatter_tiles(s, c.nmap, c.npix_cross, c.ndeg, c.d_off.p, c.nactive, c.d_ent.p, c.d_pw.p,
+                             c.d_ccinv6x.p, c.d_m4x.p, c.d_tileinfo.p, c.d_tilescratch.p);
+    else
+        launch_scatter_pixels(s, c.nmap, c.npix_cross, c.ndeg, c.d_off.p, c.d_ent.p, c.d_pw.p, c.d_ccinv6x.p,
+                              c.d_m4x.p);
+    if (t_sc) { t_sc->stop(s); t_pr->start(s); }
+    // the baseline side adds to the prior's (or diagfilter's) term; without
+    // one, the default kernels write ap themselves
+    bool add = true;
+    if (p.kfilter) apply_prior(c, c.d_p.p, c.d_ap.p);
+    else if (p.diagfilter != 0) launch_axpby_nna(s, c.d_ap.p, c.d_nna.p, c.d_p.p, p.diagfilter, nb);
+    else if (variant == 0) add = false;
+    else launch_fill(s, c.d_ap.p, 0.0, nb);
+    if (t_sc) { t_pr->stop(s); t_ga->start(s); }
+    if (variant == 3 && c.sr_g.ok)
+        launch_gather_seg(s, c.nmap, (int64_t)c.ndet * c.nsamp, c.d_pixw.p, c.d_m4x.p, c.ndeg, c.sr_g.heads.p,
+                          c.sr_g.k0.p, c.sr_g.fix_end.p, c.sr_g.fix_ord.p, c.d_dwb.p, c.d_nna.p, c.d_p.p, c.d_ap.p,
+                          c.d_sr_part.p);
+    else if (variant == 0)
+        project_to_baselines<double>(c, c.d_m4x.p, c.d_dwb.p, c.d_nna.p, c.d_p.p, c.d_ap.p, add ? 1 : 0);
+    else if (variant != 1)
+        launch_gather_flat(s, c.nmap, c.ndet, c.nsamp, c.nbase, c.d_bstart.p,
+                           c.rec_layout == REC16 ? (const void *)c.d_pixw.p : c.d_pixc.p, c.rec_layout, c.d_m4x.p,
+                           c.ndeg, c.d_dwb.p, c.d_nna.p, c.d_p.p, c.d_ap.p);
+    else
+        launch_gather_baselines(s, c.nmap, c.ndet, c.nsamp, c.nbase, c.d_bstart.p, c.d_pixw.p, c.d_m4x.p, c.ndeg,
+                                c.d_dwb.p, c.d_nna.p, c.d_p.p, c.d_ap.p, group_for(c));
+    if (t_sc) t_ga->stop(s);
+    launch_pcg_pap(s, c.d_p.p, c.d_ap.p, c.d_rmask.p, nb, c.d_part.p, c.d_scal.p, c.d_dotcnt.p);
+    if (c.precond_kind <= 1) {
+        if (t_sc) t_pc->start(s);
+        launch_pcg_update_r_diag(s, c.precond_kind == 1 ? c.d_prec.p : nullptr, c.d_aa.p, c.d_r.p, c.d_z.p, c.d_p.p,
+                                 c.d_ap.p, c.d_rmask.p, nb, c.d_part.p, c.d_scal.p, c.d_dotcnt.p, exit);
+        if (t_sc) t_pc->stop(s);
+    } else {
         launch_pcg_update_r(s, c.d_scal.p, c.d_aa.p, c.d_r.p, c.d_ro.p, c.d_p.p, c.d_ap.p, nb);
-        if (prof) t_pc.start(s);
+        if (t_sc) t_pc->start(s);
         apply_precond(c, c.d_r.p, c.d_z.p);
-        if (prof) t_pc.stop(s);
-        launch_dots(s, 1, c.d_r.p, c.d_z.p, c.d_ro.p, nullptr, c.d_rmask.p, nb, c.d_part.p, nblk);
-        launch_finalize_scalars(s, c.d_part.p, nblk, c.d_scal.p);
-        bool last = false;
-        if (converge) {
-            d2h(hs, c.d_scal.p, 8, s);
-            MADAM_CHECK(hipStreamSynchronize(s));
-            double rz = hs[0], rr = hs[4];
-            c.rr_hist.push_back(rr / rrinit);
-            if (rr / rrinit > 1e3) { c.stats[ST_NITER] = c.pcg_steps_done; fail("CG is diverging"); }
-            if (rr / rrinit < p.cglimit && c.pcg_steps_done > p.iter_min) last = true;
-            if (rz == 0) last = true;
-        }
-        if (!last) {
-            launch_update_p_slots<double>(s, c.ndet, c.nbase, c.d_scal.p + 5, nullptr, nullptr, c.d_p.p, c.d_z.p,
-                                          c.d_bslot.p, c.d_dwb.p, c.d_pw.p);
-        }
-        if (prof) {
+        if (t_sc) t_pc->stop(s);
+        launch_pcg_rz(s, c.d_r.p, c.d_z.p, c.d_ro.p, c.d_rmask.p, nb, c.d_part.p, c.d_scal.p, c.d_dotcnt.p, exit);
+    }
+    launch_update_p_slots<double>(s, c.ndet, c.nbase, c.d_scal.p + 5, c.d_scal.p + 7, nullptr, c.d_p.p, c.d_z.p,
+                                  c.d_bslot.p, c.d_dwb.p, c.d_pw.p);
+}
+
+static int pcg_steps(Context &c, int nmax, bool converge)
+{
+    hipStream_t s = c.stream;
+    const Params &p = c.p;
+    const double rrinit = c.stats[ST_RRINIT];
+    launch_fill(s, c.d_scal.p + 7, 0.0, 1);
+    if (c.profile) {
+        Timer t_sc, t_ga, t_pr, t_pc, t_it;
+        int done = 0;
+        for (; done < nmax;) {
+            done++;
+            c.pcg_steps_done++;
+            PcgExit exit;
+            if (converge) exit = PcgExit{1, c.pcg_steps_done > p.iter_min, rrinit, p.cglimit, nullptr};
+            t_it.start(s);
+            pcg_step(c, exit, &t_sc, &t_pr, &t_ga, &t_pc);
             t_it.stop(s);
             c.stats[ST_T_SCATTER] += t_sc.ms() * 1e-3;
             c.stats[ST_T_PRIOR] += t_pr.ms() * 1e-3;
@@ -1397,12 +1412,67 @@ static int pcg_steps(Context &c, int nmax, bool converge)
             c.stats[ST_T_STEP] += t_it.ms() * 1e-3;
             c.stats[ST_N_SCATTER] += 1;
             c.stats[ST_N_GATHER] += 1;
+            if (!converge) continue;
+            double hs[8];
+            d2h(hs, c.d_scal.p, 8, s);
+            MADAM_CHECK(hipStreamSynchronize(s));
+            double rz = hs[0], rr = hs[4];
+            c.rr_hist.push_back(rr / rrinit);
+            if (rr / rrinit > 1e3) { c.stats[ST_NITER] = c.pcg_steps_done; fail("CG is diverging"); }
+            if ((rr / rrinit < p.cglimit && c.pcg_steps_done > p.iter_min) || rz == 0) break;
         }
-        if (last) break;
+        MADAM_CHECK(hipStreamSynchronize(s));
+        c.stats[ST_NITER] = c.pcg_steps_done;
+        return done;
+    }
+    // (the inner-CG fallback waits for the host inside every step)
+    const bool ahead = converge && c.segcg.empty();
+    if (ahead && !c.h_steps)
+        MADAM_CHECK(hipHostMalloc((void **)&c.h_steps, sizeof(double) * 4, hipHostMallocDefault));
+    struct Event {
+        hipEvent_t e = nullptr;
+        Event() { MADAM_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming)); }
+        ~Event() { (void)hipEventDestroy(e); }
+    } ev[2];
+    int queued = 0, seen = 0;
+    const int step0 = c.pcg_steps_done;
+    bool ended = false, diverged = false;
+    double q = 1.0;   // the last rr / rrinit seen
+    while (!ended && (queued < nmax || seen < queued)) {
+        if (queued < nmax && (queued == seen || !converge || (ahead && queued == seen + 1 && q > SPECULATE * p.cglimit))) {
+            PcgExit exit;
+            if (converge)
+                exit = PcgExit{1, step0 + queued + 1 > p.iter_min, rrinit, p.cglimit,
+                               ahead ? c.h_steps + 2 * (queued & 1) : nullptr};
+            pcg_step(c, exit, nullptr, nullptr, nullptr, nullptr);
+            if (ahead) MADAM_CHECK(hipEventRecord(ev[queued & 1].e, s));
+            queued++;
+            if (!converge) seen = queued;
+            continue;
+        }
+        double rz, rr;
+        if (ahead) {
+            MADAM_CHECK(hipEventSynchronize(ev[seen & 1].e));
+            rz = c.h_steps[2 * (seen & 1)];
+            rr = c.h_steps[2 * (seen & 1) + 1];
+        } else {
+            double hs[8];
+            d2h(hs, c.d_scal.p, 8, s);
+            MADAM_CHECK(hipStreamSynchronize(s));
+            rz = hs[0];
+            rr = hs[4];
+        }
+        seen++;
+        q = rr / rrinit;
+        c.rr_hist.push_back(q);
+        if (q > 1e3) ended = diverged = true;
+        else if ((q < p.cglimit && step0 + seen > p.iter_min) || rz == 0) ended = true;
     }
     MADAM_CHECK(hipStreamSynchronize(s));
+    c.pcg_steps_done = step0 + seen;
     c.stats[ST_NITER] = c.pcg_steps_done;
-    return done;
+    if (diverged) fail("CG is diverging");
+    return seen;
 }
 
 // y = A x for the destriping operator of the last solve: FᵀZF x (pixel side,

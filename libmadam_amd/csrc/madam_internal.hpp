@@ -219,7 +219,7 @@ void launch_gather_baselines(hipStream_t s, int nmap, int ndet, int64_t nsamp, i
 template <typename T>
 void launch_gather_flat(hipStream_t s, int nmap, int ndet, int64_t nsamp, int64_t nbase, const int64_t *bstart,
                         const void *rec, int rl, const T *m4, int64_t ndeg, const T *dwb, const T *nna, const T *p,
-                        T *ap);
+                        T *ap, int add = 1);   // add 0: ap is overwritten
 void launch_scatter_flat(hipStream_t s, int nmap, int64_t npix_cross, int64_t ndeg, const int64_t *off,
                          const CsrEnt *ent, const double *pw, const double *ccinv6, double *m4);
 // entry-balanced pixel-side projection: tinfo from launch_tile_info (once per
@@ -280,11 +280,33 @@ void launch_dots(hipStream_t s, int which, const double *a, const double *b, con
                  const int8_t *mask, int64_t n, double *partials, int nblocks);
 int dots_nblocks(int64_t n);
 void launch_finalize(hipStream_t s, const double *partials, int nblocks, int nval, double *out);
-// launch_finalize of the three r/z dot products into scal[2..4], then, in the
-// same launch, beta = (scal[2] - scal[3]) / scal[0] into scal[5], the old rz
-// into scal[6] and the new rz into scal[0]
-void launch_finalize_scalars(hipStream_t s, const double *partials, int nblocks, double *scal);
-// PCG vector steps, scalars read from device memory
+// exit tests of one PCG step, made on the device (test 0: none): host[0..1]
+// (pinned, or null) receive rz and rr, scal[7] becomes 1 where the solve has ended
+struct PcgExit {
+    int test = 0, past_min = 0;
+    double rrinit = 0, limit = 0;
+    double *host = nullptr;
+};
+// what the last block of a dot-product launch does (count null: nothing)
+struct DotsEnd {
+    unsigned *count = nullptr;   // 0 between launches
+    double *pap = nullptr;       // p . ap goes here, or
+    double *scal = nullptr;      // the step's scalars end here
+    PcgExit exit;
+};
+// scal[1] = p . ap
+void launch_pcg_pap(hipStream_t s, const double *p, const double *ap, const int8_t *mask, int64_t n, double *partials,
+                    double *scal, unsigned *count);
+// r . z, r_old . z and r . r into scal[2..4], beta = (scal[2] - scal[3]) /
+// scal[0] into scal[5], the old rz into scal[6], the new rz into scal[0], and
+// the exit tests; nothing where scal[7] != 0
+void launch_pcg_rz(hipStream_t s, const double *r, const double *z, const double *ro, const int8_t *mask, int64_t n,
+                   double *partials, double *scal, unsigned *count, const PcgExit &exit);
+// launch_pcg_update_r, z = r pd (pd null: z = r) and launch_pcg_rz in one pass
+void launch_pcg_update_r_diag(hipStream_t s, const double *pd, double *aa, double *r, double *z, const double *p,
+                              const double *ap, const int8_t *mask, int64_t n, double *partials, double *scal,
+                              unsigned *count, const PcgExit &exit);
+// PCG vector steps, scalars read from device memory (nothing where scal[7] != 0)
 void launch_pcg_update_r(hipStream_t s, const double *scal, double *aa, double *r, double *ro, const double *p,
                          const double *ap, int64_t n);
 // p = z + *beta p, pw[bslot[b]] = p[b] dwb[b]; nothing where *done != 0 (null:
@@ -338,7 +360,7 @@ void runs_pixel_starts(hipStream_t s, const int64_t *segstart, int64_t nz, const
 void runs_cast(hipStream_t s, const double2 *in, float2 *out, int64_t n);
 template <typename T>
 void launch_gather_run(hipStream_t s, int nmap, int ndet, int64_t nbase, const RunView<T> &rv, const T *m4,
-                       const T *dwb, const T *nna, const T *p, T *ap);
+                       const T *dwb, const T *nna, const T *p, T *ap, int add);   // add 0: ap is overwritten
 
 // ------------------------------------------------------------------ fft.hip
 

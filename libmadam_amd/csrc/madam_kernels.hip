@@ -893,7 +893,7 @@ template <typename T, int NMAP, int RL, int FG_K>
 __global__ void __launch_bounds__(256) k_gather_flat(int ndet, int64_t nsamp, int64_t nbase,
                                                      const int64_t *bstart, const void *pixw, const T *m4,
                                                      int64_t ndeg, const T *dwb, const T *nna,
-                                                     const T *p, T *ap)
+                                                     const T *p, T *ap, int add)
 {
     using V2 = typename VecT<T>::v2;
     constexpr int FG_ITEMS = FG_D * FG_K;                          // (detector, baseline) items per block
@@ -1010,7 +1010,7 @@ __global__ void __launch_bounds__(256) k_gather_flat(int ndet, int64_t nsamp, in
         T a = group_sum<FG_LANES>(acc[i]);
         if (own[i] && sub == 0) {
             int64_t b = (int64_t)(d0 + id[i]) * nbase + k0 + ik[i];
-            ap[b] = ap[b] + (nna[b] * p[b] - a * dwb[b]);
+            ap[b] = (add ? ap[b] : (T)0) + (nna[b] * p[b] - a * dwb[b]);
         }
     }
 }
@@ -1210,7 +1210,7 @@ size_t scatter_tiles_scratch_bytes(int64_t nent)
 template <typename T>
 void launch_gather_flat(hipStream_t s, int nmap, int ndet, int64_t nsamp, int64_t nbase, const int64_t *bstart,
                         const void *pixw, int rl, const T *m4, int64_t ndeg, const T *dwb, const T *nna, const T *p,
-                        T *ap)
+                        T *ap, int add)
 {
     if (ndet <= 0 || nbase <= 0) return;
     int64_t ngrp = (ndet + FG_D - 1) / FG_D;
@@ -1225,10 +1225,10 @@ void launch_gather_flat(hipStream_t s, int nmap, int ndet, int64_t nsamp, int64_
     do {                                                                                                         \
         if (wide)                                                                                                \
             k_gather_flat<T, NM, RLV, 64><<<(unsigned)(ngrp * ((nbase + 63) / 64)), 256, 0, s>>>(                \
-                ndet, nsamp, nbase, bstart, pixw, m4, ndeg, dwb, nna, p, ap);                                    \
+                ndet, nsamp, nbase, bstart, pixw, m4, ndeg, dwb, nna, p, ap, add);                               \
         else                                                                                                     \
             k_gather_flat<T, NM, RLV, 16><<<(unsigned)(ngrp * ((nbase + 15) / 16)), 256, 0, s>>>(                \
-                ndet, nsamp, nbase, bstart, pixw, m4, ndeg, dwb, nna, p, ap);                                    \
+                ndet, nsamp, nbase, bstart, pixw, m4, ndeg, dwb, nna, p, ap, add);                               \
     } while (0)
         if (nmap == 1) {
             if (rl == REC4) MADAM_GF(1, REC4);
@@ -1242,9 +1242,10 @@ void launch_gather_flat(hipStream_t s, int nmap, int ndet, int64_t nsamp, int64_
 }
 template void launch_gather_flat<double>(hipStream_t, int, int, int64_t, int64_t, const int64_t *, const void *, int,
                                          const double *, int64_t, const double *, const double *, const double *,
-                                         double *);
+                                         double *, int);
 template void launch_gather_flat<float>(hipStream_t, int, int, int64_t, int64_t, const int64_t *, const void *, int,
-                                        const float *, int64_t, const float *, const float *, const float *, float *);
+                                        const float *, int64_t, const float *, const float *, const float *, float *,
+                                        int);
 
 void launch_scatter_flat(hipStream_t s, int nmap, int64_t npix_cross, int64_t ndeg, const int64_t *off,
                          const CsrEnt *ent, const double *pw, const double *ccinv6, double *m4)
@@ -1494,8 +1495,80 @@ int dots_nblocks(int64_t n)
 // and issues all of a chunk's loads (mask as one 8-byte word, the vectors as
 // 16-byte pairs) before the arithmetic; the block partials and their final
 // sum are in a fixed order, so the result depends on n alone.
+// The end of the step's scalars (t: rz, rz2, rr): scal[2..4], beta = (scal[2]
+// - scal[3]) / scal[0] into scal[5], the old rz into scal[6], the new one into
+// scal[0]; then the exit tests of src/smadam_routines.f90:905-918, whose
+// outcome goes into scal[7] and whose values go to the host's slot.  A solve
+// that has ended keeps its scalars whatever steps are still queued.
+__device__ inline void pcg_scalars(const double *t, double *scal, const PcgExit &x)
+{
+    if (scal[7] != 0.0) return;
+    for (int q = 0; q < 3; ++q) scal[2 + q] = t[q];
+    scal[5] = (t[0] - t[1]) / scal[0];
+    scal[6] = scal[0];
+    scal[0] = t[0];
+    if (!x.test) return;
+    double q = t[2] / x.rrinit;
+    if (q > 1e3 || (q < x.limit && x.past_min) || t[0] == 0) scal[7] = 1.0;
+    if (x.host) {
+        x.host[0] = t[0];
+        x.host[1] = t[2];
+    }
+}
+
+// Block sums of three dot products into the block's partials; with fin.count
+// the last block to finish adds the partials (thread t adds blocks t, t + TPB,
+// ..., then a tree: the same order whichever block that is) and ends the
+// step's scalars, so that a short vector takes one launch instead of two.
+__device__ inline void dots_tail(double s0, double s1, double s2, double *partials, const DotsEnd &fin)
+{
+    s0 = wave_sum(s0);
+    s1 = wave_sum(s1);
+    s2 = wave_sum(s2);
+    __shared__ double sh[3][TPB];
+    __shared__ bool last;
+    int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (lane == 0) { sh[0][wv] = s0; sh[1][wv] = s1; sh[2][wv] = s2; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t0 = 0, t1 = 0, t2 = 0;
+        for (int k = 0; k < TPB / 64; ++k) { t0 += sh[0][k]; t1 += sh[1][k]; t2 += sh[2][k]; }
+        partials[blockIdx.x * 3] = t0;
+        partials[blockIdx.x * 3 + 1] = t1;
+        partials[blockIdx.x * 3 + 2] = t2;
+        if (fin.count) {
+            __threadfence();   // the partials before the count
+            last = atomicAdd(fin.count, 1u) == gridDim.x - 1;
+        }
+    }
+    if (!fin.count) return;
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    double t[3] = {0, 0, 0};
+    const volatile double *P = partials;
+    for (int i = threadIdx.x; i < (int)gridDim.x; i += TPB)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) t[q] += P[i * 3 + q];
+    for (int q = 0; q < 3; ++q) sh[q][threadIdx.x] = t[q];
+    __syncthreads();
+    for (int o = TPB / 2; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o)
+            for (int q = 0; q < 3; ++q) sh[q][threadIdx.x] += sh[q][threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return;
+    *fin.count = 0;
+    if (fin.pap) {
+        *fin.pap = sh[0][0];
+    } else {
+        double v[3] = {sh[0][0], sh[1][0], sh[2][0]};
+        pcg_scalars(v, fin.scal, fin.exit);
+    }
+}
+
 __global__ void __launch_bounds__(TPB) k_dots(int which, const double *a, const double *b, const double *c,
-                                              const int8_t *mask, int64_t n, double *partials)
+                                              const int8_t *mask, int64_t n, double *partials, DotsEnd fin)
 {
     double s0 = 0, s1 = 0, s2 = 0;
     int64_t nch = n / DOT_CHUNK;
@@ -1533,36 +1606,22 @@ __global__ void __launch_bounds__(TPB) k_dots(int which, const double *a, const 
             s2 += ai * ai;
         }
     }
-    s0 = wave_sum(s0);
-    s1 = wave_sum(s1);
-    s2 = wave_sum(s2);
-    __shared__ double sh[3][TPB / 64];
-    int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 0) { sh[0][wv] = s0; sh[1][wv] = s1; sh[2][wv] = s2; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t0 = 0, t1 = 0, t2 = 0;
-        for (int k = 0; k < TPB / 64; ++k) { t0 += sh[0][k]; t1 += sh[1][k]; t2 += sh[2][k]; }
-        partials[blockIdx.x * 3] = t0;
-        partials[blockIdx.x * 3 + 1] = t1;
-        partials[blockIdx.x * 3 + 2] = t2;
-    }
+    dots_tail(s0, s1, s2, partials, fin);
 }
 
 void launch_dots(hipStream_t s, int which, const double *a, const double *b, const double *c, const double *d,
                  const int8_t *mask, int64_t n, double *partials, int nblocks)
 {
     (void)d;
-    k_dots<<<nblocks, TPB, 0, s>>>(which, a, b, c, mask, n, partials);
+    k_dots<<<nblocks, TPB, 0, s>>>(which, a, b, c, mask, n, partials, DotsEnd());
 }
 
 // sums the block partials in a fixed order into out[0..nval): thread t adds
 // blocks t, t + 1024, ... (eight loads in flight per value), then a tree
 static constexpr int FIN_TPB = 1024;
-// with scal (out = scal + 2): then beta = (scal[2] - scal[3]) / scal[0] into
-// scal[5], the old rz into scal[6] and the new rz into scal[0]
+// with scal: the end of the step's scalars (pcg_scalars) in place of out
 __global__ void __launch_bounds__(FIN_TPB) k_finalize(const double *partials, int nblocks, int nval, double *out,
-                                                      double *scal)
+                                                      double *scal, PcgExit exit)
 {
     __shared__ double sh[3][FIN_TPB];
     double t[3] = {0, 0, 0};
@@ -1587,30 +1646,98 @@ __global__ void __launch_bounds__(FIN_TPB) k_finalize(const double *partials, in
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        for (int q = 0; q < nval; ++q) out[q] = sh[q][0];
         if (scal) {
-            double beta = (scal[2] - scal[3]) / scal[0];
-            scal[5] = beta;
-            scal[6] = scal[0];
-            scal[0] = scal[2];
+            double v[3] = {sh[0][0], sh[1][0], sh[2][0]};
+            pcg_scalars(v, scal, exit);
+        } else {
+            for (int q = 0; q < nval; ++q) out[q] = sh[q][0];
         }
     }
 }
 
 void launch_finalize(hipStream_t s, const double *partials, int nblocks, int nval, double *out)
 {
-    k_finalize<<<1, FIN_TPB, 0, s>>>(partials, nblocks, nval, out, nullptr);
+    k_finalize<<<1, FIN_TPB, 0, s>>>(partials, nblocks, nval, out, nullptr, PcgExit());
 }
 
-void launch_finalize_scalars(hipStream_t s, const double *partials, int nblocks, double *scal)
+// Up to this many blocks the last of them finishes the sums; beyond it the
+// blocks' fences and counts cost more than the second launch: a step at 42 k
+// baselines (21 blocks) 39 -> 33 us, at 180 k (88) 57 -> 53, but at 671 k (328)
+// 197 -> 207.
+static constexpr int DOTS_ONE = 128;
+
+void launch_pcg_pap(hipStream_t s, const double *p, const double *ap, const int8_t *mask, int64_t n, double *partials,
+                    double *scal, unsigned *count)
 {
-    k_finalize<<<1, FIN_TPB, 0, s>>>(partials, nblocks, 3, scal + 2, scal);
+    int nblk = dots_nblocks(n);
+    DotsEnd fin;
+    if (nblk <= DOTS_ONE) {
+        fin.count = count;
+        fin.pap = scal + 1;
+    }
+    k_dots<<<nblk, TPB, 0, s>>>(0, p, ap, nullptr, mask, n, partials, fin);
+    if (nblk > DOTS_ONE) k_finalize<<<1, FIN_TPB, 0, s>>>(partials, nblk, 1, scal + 1, nullptr, PcgExit());
 }
 
-// scal: [0] rz, [1] pap, [2] rz_new, [3] rz2, [4] rr, [5] beta
+static DotsEnd pcg_end(int nblk, double *scal, unsigned *count, const PcgExit &exit)
+{
+    DotsEnd fin;
+    if (nblk <= DOTS_ONE) {
+        fin.count = count;
+        fin.scal = scal;
+        fin.exit = exit;
+    }
+    return fin;
+}
+
+void launch_pcg_rz(hipStream_t s, const double *r, const double *z, const double *ro, const int8_t *mask, int64_t n,
+                   double *partials, double *scal, unsigned *count, const PcgExit &exit)
+{
+    int nblk = dots_nblocks(n);
+    k_dots<<<nblk, TPB, 0, s>>>(1, r, z, ro, mask, n, partials, pcg_end(nblk, scal, count, exit));
+    if (nblk > DOTS_ONE) k_finalize<<<1, FIN_TPB, 0, s>>>(partials, nblk, 3, nullptr, scal, exit);
+}
+
+// The residual update, a diagonal preconditioner (pd null: none) and the three
+// dot products of the new r and z in one pass: r_old is only needed for r_old .
+// z and never leaves the registers.
+__global__ void __launch_bounds__(TPB) k_update_r_diag(const double *pd, double *aa, double *r, double *z,
+                                                       const double *p, const double *ap, const int8_t *mask,
+                                                       int64_t n, double *scal, double *partials, DotsEnd fin)
+{
+    const bool on = scal[7] == 0.0;
+    const double alpha = scal[0] / scal[1];
+    double s0 = 0, s1 = 0, s2 = 0;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n && on;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        double ri = r[i], pi = p[i], ai = ap[i], xi = aa[i], d = pd ? pd[i] : 1.0;
+        bool m = mask[i] != 0;
+        double rn = ri - alpha * ai, zi = pd ? rn * d : rn;
+        aa[i] = xi + alpha * pi;
+        r[i] = rn;
+        z[i] = zi;
+        s0 += m ? rn * zi : 0.0;
+        s1 += m ? ri * zi : 0.0;
+        s2 += m ? rn * rn : 0.0;
+    }
+    dots_tail(s0, s1, s2, partials, fin);
+}
+
+void launch_pcg_update_r_diag(hipStream_t s, const double *pd, double *aa, double *r, double *z, const double *p,
+                              const double *ap, const int8_t *mask, int64_t n, double *partials, double *scal,
+                              unsigned *count, const PcgExit &exit)
+{
+    int nblk = dots_nblocks(n);
+    k_update_r_diag<<<nblk, TPB, 0, s>>>(pd, aa, r, z, p, ap, mask, n, scal, partials,
+                                         pcg_end(nblk, scal, count, exit));
+    if (nblk > DOTS_ONE) k_finalize<<<1, FIN_TPB, 0, s>>>(partials, nblk, 3, nullptr, scal, exit);
+}
+
+// scal: [0] rz, [1] pap, [2] rz_new, [3] rz2, [4] rr, [5] beta, [6] old rz, [7] != 0: the solve has ended
 __global__ void k_update_r(const double *scal, double *aa, double *r, double *ro, const double *p, const double *ap,
                            int64_t n)
 {
+    if (scal[7] != 0.0) return;
     double alpha = scal[0] / scal[1];
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         double ri = r[i];

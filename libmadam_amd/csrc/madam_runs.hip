@@ -220,7 +220,8 @@ __global__ void __launch_bounds__(RUN_TPB) k_gather_run(int ndet, int64_t nbase,
                                                         const uint32_t *__restrict__ word,
                                                         const void *__restrict__ wsum, int sh,
                                                         const T *__restrict__ m4, const T *__restrict__ dwb,
-                                                        const T *__restrict__ nna, const T *__restrict__ p, T *ap)
+                                                        const T *__restrict__ nna, const T *__restrict__ p, T *ap,
+                                                        int add)
 {
     using V2 = typename VecT<T>::v2;
     constexpr int TD = RG_T / D;                                    // runs per detector and tile
@@ -334,27 +335,27 @@ __global__ void __launch_bounds__(RUN_TPB) k_gather_run(int ndet, int64_t nbase,
         int it = threadIdx.x / L + i * (RUN_TPB / L), d = it / K, k = it % K;
         if (d < nd && k < nk && sub == 0) {
             int64_t b = (int64_t)(d0 + d) * nbase + k0 + k;
-            ap[b] = ap[b] + (nna[b] * p[b] - s * dwb[b]);
+            ap[b] = (add ? ap[b] : (T)0) + (nna[b] * p[b] - s * dwb[b]);
         }
     }
 }
 
 template <typename T, int D, int K>
 static void gather_run(hipStream_t s, int nmap, int ndet, int64_t nbase, const RunView<T> &rv, const T *m4,
-                       const T *dwb, const T *nna, const T *p, T *ap)
+                       const T *dwb, const T *nna, const T *p, T *ap, int add)
 {
     unsigned grid = (unsigned)(((ndet + D - 1) / D) * ((nbase + K - 1) / K));
     if (nmap == 1)
         k_gather_run<T, 1, D, K><<<grid, RUN_TPB, 0, s>>>(ndet, nbase, rv.gst, rv.gword, rv.gw, rv.sh, m4, dwb, nna, p,
-                                                          ap);
+                                                          ap, add);
     else
         k_gather_run<T, 3, D, K><<<grid, RUN_TPB, 0, s>>>(ndet, nbase, rv.gst, rv.gword, rv.gw, rv.sh, m4, dwb, nna, p,
-                                                          ap);
+                                                          ap, add);
 }
 
 template <typename T>
 void launch_gather_run(hipStream_t s, int nmap, int ndet, int64_t nbase, const RunView<T> &rv, const T *m4,
-                       const T *dwb, const T *nna, const T *p, T *ap)
+                       const T *dwb, const T *nna, const T *p, T *ap, int add)
 {
     if (ndet <= 0 || nbase <= 0) return;
     // Four detectors per block where there are that many.  64 baselines per
@@ -364,18 +365,18 @@ void launch_gather_run(hipStream_t s, int nmap, int ndet, int64_t nbase, const R
     // with 13 (temperature) 19 / 23, 164 with 7 10.9 / 9.4.
     const bool wide = (int64_t)((ndet + 3) / 4) * ((nbase + 63) / 64) >= 512 && rv.per_base <= 32;
     if (ndet == 1) {
-        gather_run<T, 1, 64>(s, nmap, ndet, nbase, rv, m4, dwb, nna, p, ap);
+        gather_run<T, 1, 64>(s, nmap, ndet, nbase, rv, m4, dwb, nna, p, ap, add);
     } else if (ndet == 2) {
-        if (wide) gather_run<T, 2, 64>(s, nmap, ndet, nbase, rv, m4, dwb, nna, p, ap);
-        else gather_run<T, 2, 16>(s, nmap, ndet, nbase, rv, m4, dwb, nna, p, ap);
+        if (wide) gather_run<T, 2, 64>(s, nmap, ndet, nbase, rv, m4, dwb, nna, p, ap, add);
+        else gather_run<T, 2, 16>(s, nmap, ndet, nbase, rv, m4, dwb, nna, p, ap, add);
     } else {
-        if (wide) gather_run<T, 4, 64>(s, nmap, ndet, nbase, rv, m4, dwb, nna, p, ap);
-        else gather_run<T, 4, 16>(s, nmap, ndet, nbase, rv, m4, dwb, nna, p, ap);
+        if (wide) gather_run<T, 4, 64>(s, nmap, ndet, nbase, rv, m4, dwb, nna, p, ap, add);
+        else gather_run<T, 4, 16>(s, nmap, ndet, nbase, rv, m4, dwb, nna, p, ap, add);
     }
 }
 template void launch_gather_run<double>(hipStream_t, int, int, int64_t, const RunView<double> &, const double *,
-                                        const double *, const double *, const double *, double *);
+                                        const double *, const double *, const double *, double *, int);
 template void launch_gather_run<float>(hipStream_t, int, int, int64_t, const RunView<float> &, const float *,
-                                       const float *, const float *, const float *, float *);
+                                       const float *, const float *, const float *, float *, int);
 
 }  // namespace madam
