@@ -245,6 +245,214 @@ __global__ void __launch_bounds__(64) k_band_factor_w(const Segment *seg, int64_
     }
 }
 
+// ---- the factor in pieces, where it does not repeat
+//
+// A segment is a serial chain of columns (0.44 us each: 37 ms for 84 k rows
+// whatever the GPU's size), but the window forgets where it started: after a
+// few hundred columns two chains that started from different windows hold the
+// same bits.  Where flags keep the factor from repeating, pieces of BP_ROWS
+// columns are factored at the same time, each from a start BP_WARM columns
+// ahead of its own (as if the segment began there); they keep the window they
+// reached at their first column and at their end.  A second pass, one wave per
+// segment, compares each piece's first window with the one the piece before it
+// ended in.  Equal bits: the piece is what the serial chain gives.  Otherwise
+// (or where a pivot failed on the way) it factors the piece again from the
+// true window, so the factor always has the serial chain's bits.
+static constexpr int BP_ROWS = 1024, BP_WARM = 512;
+
+template <int KD>
+struct BandWin {
+    double W[KD + 1];
+
+    // rows j .. j + KD of A, as if the segment began at column j
+    __device__ inline void start(const double (&icv)[KD + 1], const double *nn, int64_t j, int64_t n, int lane)
+    {
+        constexpr int K = KD + 1;
+#pragma unroll
+        for (int bb = 0; bb < K; ++bb) {
+            double v = 0.0;
+            if (lane < K && bb <= lane && j + lane < n) {
+                int d = lane - bb;
+#pragma unroll
+                for (int m = 0; m < K; ++m) if (m == d) v = icv[m];
+                if (bb == lane) v += nn[j + lane];
+            }
+            W[bb] = v;
+        }
+    }
+
+    // column j: the steps of k_band_factor_w; false where the pivot fails.
+    // nni: nna of the row entering the window (j + K)
+    __device__ inline bool column(const double (&icv)[KD + 1], int64_t j, int64_t n, double nni, double *Lrow,
+                                  bool store, int lane)
+    {
+        constexpr int K = KD + 1;
+        constexpr bool DPP_SHIFT = K <= 15;
+        double ajj = readlane_d(W[0], 0);
+        if (!(ajj > 0)) return false;
+        double dinv = rsqrt_nr(ajj);
+        double l = (lane >= 1 && lane < K && j + lane < n) ? W[0] * dinv : 0.0;
+        if (store) {
+            if (lane == 0) Lrow[0] = dinv;
+            else if (lane < K) Lrow[lane] = l;
+        }
+#pragma unroll
+        for (int bb = 1; bb < K; ++bb) {
+            double lb = readlane_d(l, bb);
+            if (bb <= lane) W[bb] -= l * lb;
+        }
+        int64_t i = j + K;
+        double Wn[K];
+#pragma unroll
+        for (int bb = 0; bb < K - 1; ++bb)
+            Wn[bb] = DPP_SHIFT ? shift_down_row(W[bb + 1]) : __shfl(W[bb + 1], lane + 1, 64);
+        Wn[K - 1] = 0.0;
+        if (lane == K - 1) {
+#pragma unroll
+            for (int bb = 0; bb < K; ++bb) {
+                double v = 0.0;
+                if (i < n) {
+                    v = icv[K - 1 - bb];
+                    if (bb == K - 1) v += nni;
+                }
+                Wn[bb] = v;
+            }
+        }
+#pragma unroll
+        for (int bb = 0; bb < K; ++bb) W[bb] = Wn[bb];
+        return true;
+    }
+
+    // columns j0 .. j1 - 1, stored from column js on; the failing column or -1
+    __device__ inline int64_t columns(const double (&icv)[KD + 1], const double *nn, int64_t j0, int64_t js, int64_t j1,
+                                      int64_t n, double *L, int lane)
+    {
+        constexpr int K = KD + 1;
+        double nnext = j0 + K + lane < n ? nn[j0 + K + lane] : 0.0;
+        for (int64_t c0 = j0; c0 < j1; c0 += 64) {
+            double nbuf = nnext;
+            nnext = c0 + 64 + K + lane < n ? nn[c0 + 64 + K + lane] : 0.0;
+            int tn = j1 - c0 < 64 ? (int)(j1 - c0) : 64;
+            for (int t = 0; t < tn; ++t)
+                if (!column(icv, c0 + t, n, readlane_d(nbuf, t), L + (c0 + t) * K, c0 + t >= js, lane)) return c0 + t;
+        }
+        return -1;
+    }
+};
+
+// The window's entries below the diagonal are never written to or read back as
+// part of A's lower triangle, so only W[bb], bb <= lane, is compared.
+template <int KD>
+__device__ inline void band_win_store(const BandWin<KD> &w, double *to, int lane)
+{
+    constexpr int K = KD + 1;
+    if (lane < K)
+#pragma unroll
+        for (int bb = 0; bb < K; ++bb) to[bb * K + lane] = bb <= lane ? w.W[bb] : 0.0;
+}
+
+// grid: a wave per piece, the pieces of all segments one after another
+// (pfirst[s] the first of segment s); win[piece][2][K][K] the windows at the
+// piece's first column and past its last, bad[piece] != 0 where a pivot failed
+template <int KD>
+__global__ void __launch_bounds__(64) k_band_factor_pieces(const Segment *seg, int64_t nseg, const int *nband_seg,
+                                                           const int64_t *pfirst, const double *invcov, int64_t nof,
+                                                           const double *nna, double *Lb, double *win, int *bad)
+{
+    constexpr int K = KD + 1;
+    int lane = threadIdx.x & 63;
+    int64_t pc = blockIdx.x;
+    int64_t lo = 0, hi = nseg - 1;   // the segment with pfirst[s] <= pc < pfirst[s + 1]
+    while (lo < hi) {
+        int64_t mid = (lo + hi + 1) >> 1;
+        if (pfirst[mid] <= pc) lo = mid;
+        else hi = mid - 1;
+    }
+    const Segment sg = seg[lo];
+    const int nb = nband_seg[lo];
+    if (nb <= 0 || sg.skip) return;
+    const double *ic = invcov + (int64_t)sg.ipsd * nof;
+    const double *nn = nna + sg.b0;
+    const int64_t n = sg.noba, js = (pc - pfirst[lo]) * BP_ROWS;
+    if (js >= n) return;
+    const int64_t j1 = js + BP_ROWS < n ? js + BP_ROWS : n, j0 = js > BP_WARM ? js - BP_WARM : 0;
+    double icv[K];
+#pragma unroll
+    for (int m = 0; m < K; ++m) icv[m] = m < nb ? ic[m] : 0.0;
+    double *L = Lb + sg.b0 * K;
+    BandWin<KD> w;
+    w.start(icv, nn, j0, n, lane);
+    int64_t f = js > j0 ? w.columns(icv, nn, j0, js, js, n, L, lane) : -1;
+    if (f < 0) {
+        band_win_store<KD>(w, win + (pc * 2) * K * K, lane);
+        f = w.columns(icv, nn, js, js, j1, n, L, lane);
+    }
+    band_win_store<KD>(w, win + (pc * 2 + 1) * K * K, lane);
+    if (lane == 0) bad[pc] = f >= 0 ? 1 : 0;
+}
+
+// wave per segment: see above; info as k_band_factor_w
+template <int KD>
+__global__ void __launch_bounds__(64) k_band_factor_check(const Segment *seg, int64_t nseg, const int *nband_seg,
+                                                          const int64_t *pfirst, const double *invcov, int64_t nof,
+                                                          const double *nna, double *Lb, double *win, const int *bad,
+                                                          int *info)
+{
+    constexpr int K = KD + 1;
+    int lane = threadIdx.x & 63;
+    int64_t s = blockIdx.x;
+    if (s >= nseg) return;
+    const Segment sg = seg[s];
+    const int nb = nband_seg[s];
+    if (nb <= 0 || sg.skip) return;
+    const double *ic = invcov + (int64_t)sg.ipsd * nof;
+    const double *nn = nna + sg.b0;
+    const int64_t n = sg.noba, p0 = pfirst[s], np = (n + BP_ROWS - 1) / BP_ROWS;
+    double icv[K];
+#pragma unroll
+    for (int m = 0; m < K; ++m) icv[m] = m < nb ? ic[m] : 0.0;
+    for (int64_t t = 0; t < np; ++t) {
+        const int64_t pc = p0 + t, js = t * BP_ROWS, j1 = js + BP_ROWS < n ? js + BP_ROWS : n;
+        const double *mine = win + (pc * 2) * K * K, *before = win + (pc * 2 - 1) * K * K;
+        bool ok = bad[pc] == 0;
+        if (ok && t > 0) {
+            bool eq = true;
+            for (int e = lane; e < K * K; e += 64)
+                eq = eq && __double_as_longlong(mine[e]) == __double_as_longlong(before[e]);
+            ok = __ballot(!eq) == 0;
+        }
+        if (ok) continue;
+        // from the true window; a segment's first piece starts from its own
+        BandWin<KD> w;
+        if (t == 0) {
+            w.start(icv, nn, 0, n, lane);
+        } else {
+#pragma unroll
+            for (int bb = 0; bb < K; ++bb) w.W[bb] = lane < K ? before[bb * K + lane] : 0.0;
+        }
+        int64_t f = w.columns(icv, nn, js, js, j1, n, Lb + sg.b0 * K, lane);
+        if (f >= 0) {
+            if (lane == 0) info[s] = (int)(f + 1);
+            return;
+        }
+        band_win_store<KD>(w, win + (pc * 2 + 1) * K * K, lane);
+        __threadfence_block();   // the next piece reads it back
+    }
+}
+
+// changes[s] += rows of segment s whose nna differs from the row before
+__global__ void k_band_nna_changes(const Segment *seg, int64_t nseg, const double *nna, unsigned long long *changes)
+{
+    int64_t s = blockIdx.y;
+    const Segment sg = seg[s];
+    unsigned c = 0;
+    for (int64_t i = 1 + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < sg.noba;
+         i += (int64_t)gridDim.x * blockDim.x)
+        c += __double_as_longlong(nna[sg.b0 + i]) != __double_as_longlong(nna[sg.b0 + i - 1]) ? 1 : 0;
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+    if ((threadIdx.x & 63) == 0 && c) atomicAdd(changes + s, (unsigned long long)c);
+}
+
 // Lb rows of block src + 64 q' (q' = 1 .. q) = those of block src, for every
 // repeat the factorization recorded
 __global__ void k_band_fill_periodic(const Segment *seg, int64_t nseg, int K, const int64_t *per_src,
@@ -1278,34 +1486,86 @@ int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *
     MADAM_CHECK(hipMalloc(&dinfo, sizeof(int) * (nseg > 0 ? nseg : 1)));
     MADAM_CHECK(hipMemcpyAsync(dnb, nband_seg_host, sizeof(int) * nseg, hipMemcpyHostToDevice, s));
     MADAM_CHECK(hipMemsetAsync(dinfo, 0, sizeof(int) * (nseg > 0 ? nseg : 1), s));
-    int64_t *dper = nullptr;   // per_src[nseg][BAND_MAXJ], per_q[nseg][BAND_MAXJ]
-    int64_t ns1 = nseg > 0 ? nseg : 1, nj = ns1 * BAND_MAXJ;
-    MADAM_CHECK(hipMalloc(&dper, sizeof(int64_t) * 2 * nj));
-    MADAM_CHECK(hipMemsetAsync(dper, 0, sizeof(int64_t) * 2 * nj, s));
-    if (nseg > 0) {
-        BAND_DISPATCH(KD, (k_band_factor_w<KD><<<(unsigned)nseg, 64, 0, s>>>(dseg, nseg, dnb, invcov_dev, nof, nna,
-                                                                            bp.L, dinfo, periodic ? dper : nullptr,
-                                                                            dper + nj)));
-        if (periodic) {
-            unsigned gy = (unsigned)std::min<int64_t>(nseg, 65535);
-            unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>(256, 8192 / nseg));
-            k_band_fill_periodic<<<dim3(gx, gy), 256, 0, s>>>(dseg, nseg, K, dper, dper + nj, bp.L);
-        }
+    // A repeating factor is a few hundred columns after every change of nna and
+    // copies (k_band_factor_w); where that comes to more than BP_SERIAL columns
+    // in a segment the factor is made in pieces (8 detectors x 2^23 flagged
+    // samples, 16 segments of 84 k rows: the preconditioner 45 -> 7 ms, of which
+    // the serial chain had been 36.7).
+    const int64_t BP_SERIAL = 8192, PER_CHANGE = 256;
+    int64_t ns1 = nseg > 0 ? nseg : 1;
+    std::vector<int64_t> pfirst(nseg + 1, 0);
+    int64_t longest = 0;
+    for (int64_t i = 0; i < nseg; ++i) {
+        longest = std::max<int64_t>(longest, hseg[i].noba);
+        pfirst[i + 1] = pfirst[i] + (hseg[i].noba + BP_ROWS - 1) / BP_ROWS;
     }
-    MADAM_CHECK(hipGetLastError());
-    MADAM_CHECK(hipMemcpyAsync(info_out, dinfo, sizeof(int) * nseg, hipMemcpyDeviceToHost, s));
-    std::vector<int64_t> perq(nj, 0);
-    MADAM_CHECK(hipMemcpyAsync(perq.data(), dper + nj, sizeof(int64_t) * nj, hipMemcpyDeviceToHost, s));
-    MADAM_CHECK(hipStreamSynchronize(s));
+    bool pieces = false;
+    unsigned long long *dcnt = nullptr;   // nna changes per segment
+    MADAM_CHECK(hipMalloc(&dcnt, sizeof(unsigned long long) * ns1));
+    MADAM_CHECK(hipMemsetAsync(dcnt, 0, sizeof(unsigned long long) * ns1, s));
+    if (periodic && longest > BP_SERIAL && nseg <= 65535) {
+        k_band_nna_changes<<<dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(64, 8192 / nseg)), (unsigned)nseg), 256,
+                             0, s>>>(dseg, nseg, nna, dcnt);
+        std::vector<unsigned long long> ch(nseg);
+        MADAM_CHECK(hipMemcpyAsync(ch.data(), dcnt, sizeof(ch[0]) * nseg, hipMemcpyDeviceToHost, s));
+        MADAM_CHECK(hipStreamSynchronize(s));
+        for (int64_t i = 0; i < nseg; ++i)
+            pieces = pieces || std::min<int64_t>(hseg[i].noba, (int64_t)ch[i] * PER_CHANGE) > BP_SERIAL;
+    }
+    bp.nrows_factored = 0;
+    if (pieces) {
+        int64_t *dpf = nullptr;
+        double *win = nullptr;
+        int *bad = nullptr;
+        const int64_t npc = pfirst[nseg];
+        MADAM_CHECK(hipMalloc(&dpf, sizeof(int64_t) * (nseg + 1)));
+        MADAM_CHECK(hipMalloc(&win, sizeof(double) * 2 * K * K * npc));
+        MADAM_CHECK(hipMalloc(&bad, sizeof(int) * npc));
+        MADAM_CHECK(hipMemcpyAsync(dpf, pfirst.data(), sizeof(int64_t) * (nseg + 1), hipMemcpyHostToDevice, s));
+        BAND_DISPATCH(KD, ({
+            k_band_factor_pieces<KD><<<(unsigned)npc, 64, 0, s>>>(dseg, nseg, dnb, dpf, invcov_dev, nof, nna, bp.L, win,
+                                                                  bad);
+            k_band_factor_check<KD><<<(unsigned)nseg, 64, 0, s>>>(dseg, nseg, dnb, dpf, invcov_dev, nof, nna, bp.L, win,
+                                                                  bad, dinfo);
+        }));
+        MADAM_CHECK(hipGetLastError());
+        MADAM_CHECK(hipMemcpyAsync(info_out, dinfo, sizeof(int) * nseg, hipMemcpyDeviceToHost, s));
+        MADAM_CHECK(hipStreamSynchronize(s));
+        (void)hipFree(dpf);
+        (void)hipFree(win);
+        (void)hipFree(bad);
+        for (int64_t i = 0; i < nseg; ++i)
+            if (!hseg[i].skip && nband_seg_host[i] > 0) bp.nrows_factored += hseg[i].noba;
+    } else {
+        int64_t *dper = nullptr;   // per_src[nseg][BAND_MAXJ], per_q[nseg][BAND_MAXJ]
+        int64_t nj = ns1 * BAND_MAXJ;
+        MADAM_CHECK(hipMalloc(&dper, sizeof(int64_t) * 2 * nj));
+        MADAM_CHECK(hipMemsetAsync(dper, 0, sizeof(int64_t) * 2 * nj, s));
+        if (nseg > 0) {
+            BAND_DISPATCH(KD, (k_band_factor_w<KD><<<(unsigned)nseg, 64, 0, s>>>(dseg, nseg, dnb, invcov_dev, nof, nna,
+                                                                                bp.L, dinfo, periodic ? dper : nullptr,
+                                                                                dper + nj)));
+            if (periodic) {
+                unsigned gy = (unsigned)std::min<int64_t>(nseg, 65535);
+                unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>(256, 8192 / nseg));
+                k_band_fill_periodic<<<dim3(gx, gy), 256, 0, s>>>(dseg, nseg, K, dper, dper + nj, bp.L);
+            }
+        }
+        MADAM_CHECK(hipGetLastError());
+        MADAM_CHECK(hipMemcpyAsync(info_out, dinfo, sizeof(int) * nseg, hipMemcpyDeviceToHost, s));
+        std::vector<int64_t> perq(nj, 0);
+        MADAM_CHECK(hipMemcpyAsync(perq.data(), dper + nj, sizeof(int64_t) * nj, hipMemcpyDeviceToHost, s));
+        MADAM_CHECK(hipStreamSynchronize(s));
+        (void)hipFree(dper);
+        for (int64_t i = 0; i < nseg; ++i)
+            if (!hseg[i].skip && nband_seg_host[i] > 0) {
+                bp.nrows_factored += hseg[i].noba;
+                for (int k = 0; k < BAND_MAXJ; ++k) bp.nrows_factored -= 64 * perq[i * BAND_MAXJ + k];
+            }
+    }
     (void)hipFree(dnb);
     (void)hipFree(dinfo);
-    (void)hipFree(dper);
-    bp.nrows_factored = 0;
-    for (int64_t i = 0; i < nseg; ++i)
-        if (!hseg[i].skip && nband_seg_host[i] > 0) {
-            bp.nrows_factored += hseg[i].noba;
-            for (int k = 0; k < BAND_MAXJ; ++k) bp.nrows_factored -= 64 * perq[i * BAND_MAXJ + k];
-        }
+    (void)hipFree(dcnt);
     // chunk table over the segments that factored
     std::vector<ChunkInfo> ch;
     std::vector<int64_t> first;
