@@ -1015,6 +1015,36 @@ void fft_c2r_rows(hipStream_t s, const FftPlan &p, const double *fc, int64_t nro
 
 // ---------------------------------------------------------------- noise filter
 
+// one block per row: thread t adds values t, t + 1024, ... (eight loads in
+// flight), then a tree
+__global__ void __launch_bounds__(1024) k_row_power(const double *x, int64_t stride, int64_t n, double *out)
+{
+    const double *v = x + blockIdx.x * stride;
+    double s = 0;
+    for (int64_t i0 = threadIdx.x; i0 < n; i0 += 8 * 1024) {
+        double a[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) a[u] = i0 + u * 1024 < n ? v[i0 + u * 1024] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += a[u] * a[u];
+    }
+    __shared__ double sh[1024];
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    for (int o = 512; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[blockIdx.x] = sh[0];
+}
+
+void launch_row_power(hipStream_t s, const double *x, int64_t nrow, int64_t stride, int64_t n, double *out)
+{
+    if (nrow <= 0) return;
+    k_row_power<<<(unsigned)nrow, 1024, 0, s>>>(x, stride, n, out);
+    MADAM_CHECK(hipGetLastError());
+}
+
 // interpolate_psd for one target frequency (src/noise_routines.f90:130-190),
 // lf / lp are log(freq) / log(psd)
 __device__ double interp_psd(const double *freq, const double *psd, const double *lf, const double *lp, int64_t n_in,

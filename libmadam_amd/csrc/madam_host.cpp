@@ -1191,15 +1191,22 @@ static void build_preconditioner(Context &c)
     // invcov = c2r(fcov) / nof per PSD
     c.d_invcov.alloc((size_t)c.nof * c.npsdtot);
     fft_c2r_rows(s, c.fft, c.d_fcov.p, c.npsdtot, c.d_invcov.p, nullptr);
-    std::vector<double> ic((size_t)c.nof * c.npsdtot);
-    d2h(ic.data(), c.d_invcov.p, ic.size(), s);
-    MADAM_CHECK(hipStreamSynchronize(s));
+    // the host needs the power of the first half and the first values (the
+    // whole rows are 134 MB for 16 PSDs of 2^20)
+    const int64_t nic = std::min<int64_t>(c.nof, std::max(p.precond_width_max, 1));
+    std::vector<double> ic((size_t)nic * c.npsdtot), ptot(c.npsdtot, 0.0);
+    {
+        DBuf<double> dp;
+        dp.alloc(c.npsdtot);
+        launch_row_power(s, c.d_invcov.p, c.npsdtot, c.nof, c.nof / 2, dp.p);
+        d2h(ptot.data(), dp.p, c.npsdtot, s);
+        MADAM_CHECK(hipMemcpy2DAsync(ic.data(), sizeof(double) * nic, c.d_invcov.p, sizeof(double) * c.nof,
+                                     sizeof(double) * nic, c.npsdtot, hipMemcpyDeviceToHost, s));
+        MADAM_CHECK(hipStreamSynchronize(s));
+    }
     // band width per PSD and segment (src/noise_routines.f90:1071-1090)
     const double plim = F32(1 - 1e-5f);
     std::vector<int> nband(c.segp.size(), 0);
-    std::vector<double> ptot(c.npsdtot, 0.0);
-    for (int ip = 0; ip < c.npsdtot; ++ip)
-        for (int64_t i = 0; i < c.nof / 2; ++i) ptot[ip] += ic[(size_t)ip * c.nof + i] * ic[(size_t)ip * c.nof + i];
     std::vector<int> tries(c.segp.size(), 1);
     std::vector<char> use_cg(c.segp.size(), 0);
     // Segments whose band would be wider than the factor kernels take
@@ -1211,7 +1218,7 @@ static void build_preconditioner(Context &c)
         const Segment &g = c.segp[is];
         if (g.skip || g.ipsd < 0) continue;
         if (p.use_cgprecond) { use_cg[is] = 1; continue; }
-        const double *v = ic.data() + (size_t)g.ipsd * c.nof;
+        const double *v = ic.data() + (size_t)g.ipsd * nic;
         int tr = 1, nb = 0, ok = 0;
         for (;;) {
             nb = (int)std::min<int64_t>(g.noba, (int64_t)tr * p.precond_width_min);
@@ -1270,7 +1277,7 @@ static void build_preconditioner(Context &c)
     for (size_t is = 0; is < c.segp.size(); ++is)
         if (use_cg[is]) {
             c.segcg.push_back(c.segp[is]);
-            c.ic0cg.push_back(ic[(size_t)c.segp[is].ipsd * c.nof]);
+            c.ic0cg.push_back(ic[(size_t)c.segp[is].ipsd * nic]);
         }
     if (!c.segcg.empty()) {
         c.d_segcg.alloc(c.segcg.size());

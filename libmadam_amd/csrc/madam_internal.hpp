@@ -401,6 +401,8 @@ int64_t fft_batch_segments(const FftPlan &p, int64_t nseg, size_t elem);
 size_t fft_convolve_work_doubles(const FftPlan &p, int64_t batch, int64_t nseg_max);
 // inverse real FFT of fcov rows (invcov = c2r(fcov) / nof)
 void fft_c2r_rows(hipStream_t s, const FftPlan &p, const double *fc, int64_t nrows, double *out, double *work);
+// out[row] = sum of the squares of the first n values of each row
+void launch_row_power(hipStream_t s, const double *x, int64_t nrow, int64_t stride, int64_t n, double *out);
 // noise filter (build_filter) on the device
 void launch_build_filter(hipStream_t s, int64_t nof, double fsample, int nshort, int radiometers, double sigma,
                          double plateau, int64_t n_in, int64_t startbin, const double *tab, double *fcov, int *bad);
