@@ -97,7 +97,12 @@ struct BatchState {
         gexec_free = nullptr;
         graph_free = nullptr;
     }
-    ~BatchState() { drop_graphs(); }
+    int *h_active = nullptr;   // pinned: the active flags after the last two steps
+    ~BatchState()
+    {
+        drop_graphs();
+        if (h_active) (void)hipHostFree(h_active);
+    }
 };
 
 void batch_release(Context &c)
@@ -431,6 +436,8 @@ static void pcg_step(Context &c, BatchState &B, const Vec<T> &v, double lim, int
     }
 }
 
+static constexpr double AHEAD_STEP = 1e-3;   // steps shorter than this (s) are queued ahead
+
 static int count_active(Context &c, BatchState &B)
 {
     std::vector<int> a(B.R);
@@ -462,9 +469,7 @@ static int64_t batch_pcg(Context &c, BatchState &B, const Vec<T> &v, const T *b,
     // profiling times every part with events, so the steps run as launched
     bool graph = B.use_graph && c.segcg.empty() && !c.profile;
     StepTimers tmr;
-    int64_t steps = 0;
-    double t0 = now();
-    while (count_active(c, B) > 0) {
+    auto launch = [&] {
         if (c.profile) {
             pcg_step<T>(c, B, v, lim, iter_min, iter_max, stall, &tmr);
         } else if (graph) {
@@ -479,11 +484,44 @@ static int64_t batch_pcg(Context &c, BatchState &B, const Vec<T> &v, const T *b,
             pcg_step<T>(c, B, v, lim, iter_min, iter_max, stall);
         }
         MADAM_CHECK(hipGetLastError());
-        steps++;
+    };
+    // A step leaves right-hand sides that are done alone, so short steps are
+    // queued one ahead of the host's look at the active flags: the look costs
+    // some 30 us a step, a step too many at the end costs one step (448 steps
+    // of 38 us, 4 detectors x 2^19 samples: 27.2 -> 20.4 ms; steps of 0.3 ms:
+    // 11.7 -> 11.5 ms; longer than 1 ms: nothing).
+    int64_t queued = 0, seen = 0;
+    double t0 = now();
+    if (count_active(c, B) > 0) {
+        if (!B.h_active) MADAM_CHECK(hipHostMalloc((void **)&B.h_active, sizeof(int) * 2 * 64, hipHostMallocDefault));
+        struct Event {
+            hipEvent_t e = nullptr;
+            Event() { MADAM_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming)); }
+            ~Event() { (void)hipEventDestroy(e); }
+        } ev[2];
+        bool ahead = false;
+        double t1 = now();
+        for (bool on = true; on;) {
+            launch();
+            MADAM_CHECK(hipMemcpyAsync(B.h_active + 64 * (queued & 1), B.active.p, sizeof(int) * R,
+                                       hipMemcpyDeviceToHost, s));
+            MADAM_CHECK(hipEventRecord(ev[queued & 1].e, s));
+            queued++;
+            if (ahead && queued == seen + 1) continue;
+            MADAM_CHECK(hipEventSynchronize(ev[seen & 1].e));
+            const int *a = B.h_active + 64 * (seen & 1);
+            seen++;
+            on = false;
+            for (int k = 0; k < R; ++k) on = on || a[k] != 0;
+            // decided on the second and third step (the first may capture the graph)
+            if (seen == 1) t1 = now();
+            if (seen == 3) ahead = !c.profile && c.segcg.empty() && (now() - t1) / 2 < AHEAD_STEP;
+        }
+        MADAM_CHECK(hipStreamSynchronize(s));
     }
     B.t_inner += now() - t0;
-    B.n_inner += steps;
-    return steps;
+    B.n_inner += seen;
+    return seen;
 }
 
 // ------------------------------------------------------------------ set-up and solve
