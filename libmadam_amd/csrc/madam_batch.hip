@@ -1222,6 +1222,197 @@ __global__ void k_bmap_unpack(const T *m, int64_t npix, int nmap, int R, int r, 
     }
 }
 
+// ---------------------------------------------------------------- sums per pixel for several signals
+// Binning a signal (src/smadam_routines.f90:111-250) and subtracting baselines
+// from the binned signal (src/smadam_routines.f90:1489-1539) read every CSR
+// entry, and for each a value from somewhere else: the TOD sample, a cache line
+// per entry.  Done one signal at a time that line brings one value; here the
+// samples (or baselines) of GR signals lie side by side, so the entry and the
+// line are read once for all of them.  Lane (g, r) of a wave takes entries g, g
+// + G, ... (G = 64 / GR, four in flight) for signal r; the G sums meet over the
+// lanes.  A wave takes one pixel; pixels of more than BM_LONG entries (poles)
+// go to a list and to a block of 16 waves each.  Bound by the gathered lines.
+// Measured, 16 signals of 8 detectors x 2^22 FP32 samples at Nside 256, ms for
+// all: binning 16.8 -> 2.5 (the turning of the samples included), subtraction
+// 8.6 -> 1.6.
+static constexpr int BM_LONG = 2048, BM_U = 4, BM_LTPB = 1024;
+
+// out[i * GR + r] = sig[r * n + i] (0 for r >= nr)
+template <typename TT, int GR>
+__global__ void __launch_bounds__(BTPB) k_turn(const TT *__restrict__ sig, int64_t n, int nr, TT *__restrict__ out)
+{
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        TT v[GR];
+#pragma unroll
+        for (int r = 0; r < GR; ++r) v[r] = r < nr ? sig[(int64_t)r * n + i] : (TT)0;
+        using V = typename Quad<TT>::V;
+#pragma unroll
+        for (int r = 0; r < GR; r += 4) {
+            V q;
+            q.x = v[r];
+            q.y = v[r + 1];
+            q.z = v[r + 2];
+            q.w = v[r + 3];
+            *(V *)(out + i * GR + r) = q;
+        }
+    }
+}
+
+// sums over entries first, first + step, ... below end, BM_U at a time.  SUB:
+// val[slot * vstride + r] (baselines times weight), else val[src * vstride + r]
+// times the slot's weight
+template <typename TT, int GR, int NMAP, bool SUB>
+__device__ inline void bm_sum(double (&a)[3], int64_t first, int64_t end, int step, const CsrEnt *ent,
+                              const uint32_t *src, const TT *val, int64_t vstride, const double *dwb)
+{
+    const int lane = threadIdx.x & 63, r = lane % GR, g = lane / GR;
+    constexpr int G = 64 / GR;
+    for (int64_t j0 = first; j0 < end; j0 += step) {
+        CsrEnt e[BM_U];
+        uint32_t sr[BM_U];
+        bool ok[BM_U];
+#pragma unroll
+        for (int u = 0; u < BM_U; ++u) {
+            int64_t j = j0 + u * G + g;
+            ok[u] = j < end;
+            j = ok[u] ? j : end - 1;
+            e[u] = ent[j];
+            if (!SUB) sr[u] = src[j];
+        }
+        double v[BM_U];
+#pragma unroll
+        for (int u = 0; u < BM_U; ++u) {
+            if (SUB) v[u] = (double)val[(int64_t)e[u].b * vstride + r];
+            else v[u] = (double)val[(int64_t)sr[u] * vstride + r] * dwb[e[u].b];
+        }
+#pragma unroll
+        for (int u = 0; u < BM_U; ++u) {
+            double x = ok[u] ? v[u] : 0.0;
+            if (NMAP == 1) {
+                a[0] += x;
+            } else {
+                a[0] += (double)e[u].w0 * x;
+                a[1] += (double)e[u].w1 * x;
+                a[2] += (double)e[u].w2 * x;
+            }
+        }
+    }
+#pragma unroll
+    for (int o = GR; o < 64; o <<= 1)
+#pragma unroll
+        for (int m = 0; m < NMAP; ++m) a[m] += __shfl_xor(a[m], o, 64);
+}
+
+// out[r][q] = rhs[r][q] - sums (SUB) or the sums; maps of four doubles per
+// pixel, ostride doubles apart
+template <int NMAP, bool SUB>
+__device__ inline void bm_store(const double *a, int64_t q, int r, const double *rhs, double *out, int64_t ostride)
+{
+    double4 v = make_double4(a[0], NMAP == 3 ? a[1] : 0.0, NMAP == 3 ? a[2] : 0.0, 0.0);
+    if (SUB) {
+        double4 b = *(const double4 *)(rhs + r * ostride + q * 4);
+        v = make_double4(b.x - v.x, b.y - v.y, b.z - v.z, b.w);
+    }
+    *(double4 *)(out + r * ostride + q * 4) = v;
+}
+
+template <typename TT, int GR, int NMAP, bool SUB>
+__global__ void __launch_bounds__(BTPB) k_bin_multi(int64_t npix, const int64_t *off, const CsrEnt *ent,
+                                                    const uint32_t *src, const TT *val, int64_t vstride, int nr,
+                                                    const double *dwb, const double *rhs, double *out, int64_t ostride,
+                                                    int32_t *list, int *nlist)
+{
+    int lane = threadIdx.x & 63;
+    int64_t wave = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
+    int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
+    for (int64_t q = wave; q < npix; q += nwaves) {
+        int64_t j0 = off[q], j1 = off[q + 1];
+        if (j1 - j0 > BM_LONG) {
+            if (lane == 0) list[atomicAdd(nlist, 1)] = (int32_t)q;
+            continue;
+        }
+        double a[3] = {0, 0, 0};
+        bm_sum<TT, GR, NMAP, SUB>(a, j0, j1, BM_U * (64 / GR), ent, src, val, vstride, dwb);
+        if (lane < nr) bm_store<NMAP, SUB>(a, q, lane, rhs, out, ostride);
+    }
+}
+
+// a block per long pixel: wave w takes every 16th piece, the waves' sums in order
+template <typename TT, int GR, int NMAP, bool SUB>
+__global__ void __launch_bounds__(BM_LTPB) k_bin_long(const int64_t *off, const CsrEnt *ent, const uint32_t *src,
+                                                      const TT *val, int64_t vstride, int nr, const double *dwb,
+                                                      const double *rhs, double *out, int64_t ostride,
+                                                      const int32_t *list, const int *nlist)
+{
+    constexpr int NW = BM_LTPB / 64, PC = BM_U * (64 / GR);
+    __shared__ double sh[NW][3][GR];
+    int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int i = blockIdx.x; i < *nlist; i += gridDim.x) {
+        int64_t q = list[i];
+        double a[3] = {0, 0, 0};
+        bm_sum<TT, GR, NMAP, SUB>(a, off[q] + w * PC, off[q + 1], NW * PC, ent, src, val, vstride, dwb);
+        if (lane < GR)
+#pragma unroll
+            for (int m = 0; m < 3; ++m) sh[w][m][lane] = a[m];
+        __syncthreads();
+        if (threadIdx.x < (unsigned)nr) {
+            double t[3] = {0, 0, 0};
+            for (int k = 0; k < NW; ++k)
+                for (int m = 0; m < 3; ++m) t[m] += sh[k][m][threadIdx.x];
+            bm_store<NMAP, SUB>(t, q, (int)threadIdx.x, rhs, out, ostride);
+        }
+        __syncthreads();
+    }
+}
+
+template <typename TT>
+void batch_turn(hipStream_t s, int gr, const TT *sig, int64_t n, int nr, TT *out)
+{
+    if (n <= 0) return;
+    if (gr == 4) k_turn<TT, 4><<<bgrid(n, BTPB, 65535), BTPB, 0, s>>>(sig, n, nr, out);
+    else k_turn<TT, 8><<<bgrid(n, BTPB, 65535), BTPB, 0, s>>>(sig, n, nr, out);
+}
+
+template <typename TT>
+void batch_bin(hipStream_t s, int gr, int nmap, bool sub, int64_t npix, const int64_t *off, const CsrEnt *ent,
+               const uint32_t *src, const TT *val, int64_t vstride, int nr, const double *dwb, const double *rhs,
+               double *out, int64_t ostride, int32_t *list, int *nlist)
+{
+    if (npix <= 0) return;
+    MADAM_CHECK(hipMemsetAsync(nlist, 0, sizeof(int), s));
+    int g = bgrid(npix, BTPB / 64, 1 << 20);
+#define BM_RUN(GR, NM, SB)                                                                                        \
+    do {                                                                                                          \
+        k_bin_multi<TT, GR, NM, SB><<<g, BTPB, 0, s>>>(npix, off, ent, src, val, vstride, nr, dwb, rhs, out, ostride, \
+                                                       list, nlist);                                              \
+        k_bin_long<TT, GR, NM, SB><<<512, BM_LTPB, 0, s>>>(off, ent, src, val, vstride, nr, dwb, rhs, out, ostride,   \
+                                                           list, nlist);                                          \
+    } while (0)
+#define BM_NM(GR, SB)              \
+    do {                           \
+        if (nmap == 1) BM_RUN(GR, 1, SB); \
+        else BM_RUN(GR, 3, SB);    \
+    } while (0)
+    if (gr == 4) {
+        if (sub) BM_NM(4, true);
+        else BM_NM(4, false);
+    } else {
+        if (sub) BM_NM(8, true);
+        else BM_NM(8, false);
+    }
+#undef BM_NM
+#undef BM_RUN
+    MADAM_CHECK(hipGetLastError());
+}
+template void batch_turn<float>(hipStream_t, int, const float *, int64_t, int, float *);
+template void batch_turn<double>(hipStream_t, int, const double *, int64_t, int, double *);
+template void batch_bin<float>(hipStream_t, int, int, bool, int64_t, const int64_t *, const CsrEnt *, const uint32_t *,
+                               const float *, int64_t, int, const double *, const double *, double *, int64_t,
+                               int32_t *, int *);
+template void batch_bin<double>(hipStream_t, int, int, bool, int64_t, const int64_t *, const CsrEnt *, const uint32_t *,
+                                const double *, int64_t, int, const double *, const double *, double *, int64_t,
+                                int32_t *, int *);
+
 // ---------------------------------------------------------------- explicit instantiations
 
 #define BATCH_INST(T)                                                                                              \

@@ -103,4 +103,16 @@ void batch_fill(hipStream_t s, T *d, T v, int64_t n);
 // the map of right-hand side r from the RHS-minor layout into double4 per pixel
 void batch_map_unpack(hipStream_t s, const void *m, int is_float, int64_t npix, int nmap, int R, int r, double *out4);
 
+// gr (4 or 8) signals of n samples side by side: out[i * gr + r] = sig[r * n + i], 0 for r >= nr
+template <typename TT>
+void batch_turn(hipStream_t s, int gr, const TT *sig, int64_t n, int nr, TT *out);
+// per map pixel, the sums of weight x value over its CSR entries for nr <= gr
+// signals at once: sub = false: value = val[src * vstride + r] dwb[slot] into
+// out[r * ostride + q * 4 + c]; sub: out = rhs - sums of val[slot * vstride + r].
+// list [npix], nlist: scratch
+template <typename TT>
+void batch_bin(hipStream_t s, int gr, int nmap, bool sub, int64_t npix, const int64_t *off, const CsrEnt *ent,
+               const uint32_t *src, const TT *val, int64_t vstride, int nr, const double *dwb, const double *rhs,
+               double *out, int64_t ostride, int32_t *list, int *nlist);
+
 }  // namespace madam

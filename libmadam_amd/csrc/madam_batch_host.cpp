@@ -618,23 +618,82 @@ static void make_segments(Context &c, BatchState &B)
     B.fftwork.alloc(fft_convolve_work_doubles(c.fft, std::max<int64_t>(B.fft_batch64, B.fft_batch32), B.fft_nseg));
 }
 
-// binned map and right-hand side of one signal (src/smadam_routines.f90:252-671),
-// with the shared pixel matrices of the set-up
+// right-hand side of one binned signal (src/smadam_routines.f90:428-671), with
+// the shared pixel matrices of the set-up; cc6 is read where the map is degraded
 template <typename TT>
-static void bin_signal(Context &c, const TT *tod, double *rhs4, double *yba, DBuf<double> &cc6, DBuf<double> &rhs4x,
-                       DBuf<double> &m4x, DBuf<double> &nna)
+static void signal_rhs(Context &c, const TT *tod, const double *rhs4, double *yba, const double *cc6, double *cc6x,
+                       DBuf<double> &rhs4x, DBuf<double> &m4x, DBuf<double> &nna)
 {
     hipStream_t s = c.stream;
-    launch_bin<TT>(s, c.nmap, c.npix_map, c.d_off.p, c.d_ent.p, c.d_src.p, tod, c.d_dwb_s.p, c.d_sdwb_s.p, cc6.p,
-                   rhs4);
     const double *rx = rhs4;
     if (c.ndeg > 1) {
-        launch_degrade(s, c.nmap, c.npix_cross, c.ndeg, cc6.p, rhs4, cc6.p + c.npix_map * 6, rhs4x.p);
+        launch_degrade(s, c.nmap, c.npix_cross, c.ndeg, cc6, rhs4, cc6x, rhs4x.p);
         rx = rhs4x.p;
     }
     launch_ccmultiply(s, c.nmap, c.npix_cross, c.d_ccinv6x.p, rx, m4x.p);
     launch_init_a<TT>(s, c.nmap, c.ndet, c.nsamp, c.nbase, c.d_bstart.p, c.d_pixw.p, tod, m4x.p, c.ndeg, c.d_dwb.p,
                       yba, nna.p, group_for(c));
+}
+
+// signals per pass of the shared binning (and subtraction): 4 or 8
+static int bin_group(int n) { return n <= 4 ? 4 : 8; }
+
+// device memory that may not be there: false leaves the buffer empty
+template <typename T>
+static bool try_alloc(DBuf<T> &b, size_t n)
+{
+    try {
+        b.alloc(n);
+    } catch (const HipError &e) {
+        if (e.err != hipErrorOutOfMemory) throw;
+        (void)hipGetLastError();
+        b.p = nullptr;
+        b.n = 0;
+        return false;
+    }
+    return true;
+}
+
+// binned maps rhs4[k] and right-hand sides yba[k] of the signals k = 1 ..
+// nrhs - 1 (the set-up has made those of the first): signals on the device are
+// binned bin_group at a time, from a copy with their samples side by side (32
+// or 64 bytes a sample; without the memory for it, one at a time, as signals
+// from the host are)
+template <typename TT, typename F>
+static void bin_signals(Context &c, BatchState &B, int nrhs, int on_device, F &&signal)
+{
+    hipStream_t s = c.stream;
+    int64_t n = (int64_t)c.ndet * c.nsamp, nb = c.nbtot, np = c.npix_map;
+    DBuf<double> cc6, cc6x, rhs4x, m4x, nna;
+    cc6x.alloc((size_t)c.npix_cross * 6);
+    rhs4x.alloc((size_t)c.npix_cross * 4);
+    m4x.alloc((size_t)c.npix_cross * 4);
+    nna.alloc(std::max<int64_t>(nb, 1));
+    const int gr = bin_group(nrhs - 1);
+    DBuf<TT> turned;
+    DBuf<int32_t> list;
+    if (on_device && nrhs > 2 && try_alloc(turned, (size_t)std::max<int64_t>(n, 1) * gr)) {
+        list.alloc(np + 1);
+        for (int k0 = 1; k0 < nrhs; k0 += gr) {
+            int nr = std::min(gr, nrhs - k0);
+            batch_turn<TT>(s, gr, signal(k0), n, nr, turned.p);
+            batch_bin<TT>(s, gr, c.nmap, false, np, c.d_off.p, c.d_ent.p, c.d_src.p, turned.p, gr, nr, c.d_dwb_s.p,
+                          nullptr, B.rhs4.p + (int64_t)k0 * np * 4, np * 4, list.p, (int *)(list.p + np));
+            for (int k = k0; k < k0 + nr; ++k)
+                signal_rhs<TT>(c, signal(k), B.rhs4.p + (int64_t)k * np * 4, B.yba.p + (int64_t)k * nb, c.d_cc6.p,
+                               cc6x.p, rhs4x, m4x, nna);
+        }
+    } else {
+        cc6.alloc((size_t)np * 6);
+        for (int k = 1; k < nrhs; ++k) {
+            const TT *tod = signal(k);
+            launch_bin<TT>(s, c.nmap, np, c.d_off.p, c.d_ent.p, c.d_src.p, tod, c.d_dwb_s.p, c.d_sdwb_s.p, cc6.p,
+                           B.rhs4.p + (int64_t)k * np * 4);
+            signal_rhs<TT>(c, tod, B.rhs4.p + (int64_t)k * np * 4, B.yba.p + (int64_t)k * nb, cc6.p, cc6x.p, rhs4x, m4x,
+                           nna);
+        }
+    }
+    MADAM_CHECK(hipStreamSynchronize(s));
 }
 
 template <typename TT>
@@ -679,17 +738,7 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
     batch_fill<double>(s, B.yba.p, 0.0, nb * R);
     batch_copy<double>(s, B.yba.p, c.d_yba.p, nb);
     batch_copy<double>(s, B.rhs4.p, c.d_rhs4.p, np * 4);
-    {
-        DBuf<double> cc6, rhs4x, m4x, nna;
-        cc6.alloc((size_t)(np + c.npix_cross) * 6);
-        rhs4x.alloc((size_t)c.npix_cross * 4);
-        m4x.alloc((size_t)c.npix_cross * 4);
-        nna.alloc(std::max<int64_t>(nb, 1));
-        for (int k = 1; k < nrhs; ++k)
-            bin_signal<TT>(c, signal(k), B.rhs4.p + (int64_t)k * np * 4, B.yba.p + (int64_t)k * nb, cc6, rhs4x, m4x,
-                           nna);
-        MADAM_CHECK(hipStreamSynchronize(s));
-    }
+    if (nrhs > 1) bin_signals<TT>(c, B, nrhs, on_device, signal);
     if (c.precond_kind == 3) band_reserve(c.band, R);
     make_segments(c, B);
     // per-RHS state
@@ -828,7 +877,25 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
                   p.incomplete_matrices, p.allow_decoupling, nullptr);
     B.map4.alloc((size_t)np * 4 * R);
     B.binmap4.alloc((size_t)np * 4 * R);
-    {
+    if (nrhs > 2) {
+        // the baselines of all right-hand sides in slot order, side by side,
+        // subtracted bin_group at a time
+        double *pw = precision == 0 ? tp<double>(B.pw) : B.pw64.p;
+        batch_pw<double>(s, R, B.a64.p, nb, c.d_bord.p, c.d_bslot.p, c.d_dwb_s.p, c.d_dwb.p, B.ones.p, pw);
+        const int gr = std::min(R, bin_group(nrhs));
+        DBuf<int32_t> list;
+        list.alloc(np + 1);
+        for (int k0 = 0; k0 < nrhs; k0 += gr)
+            batch_bin<double>(s, gr, c.nmap, true, np, c.d_off.p, c.d_ent.p, c.d_src.p, pw + k0, R,
+                              std::min(gr, nrhs - k0), c.d_dwb_s.p, B.rhs4.p + (int64_t)k0 * np * 4,
+                              B.map4.p + (int64_t)k0 * np * 4, np * 4, list.p, (int *)(list.p + np));
+        for (int k = 0; k < nrhs; ++k) {
+            double *m = B.map4.p + (int64_t)k * np * 4;
+            launch_ccmultiply(s, c.nmap, np, c.d_ccinv6.p, m, m);
+            launch_ccmultiply(s, c.nmap, np, c.d_ccinv6.p, B.rhs4.p + (int64_t)k * np * 4,
+                              B.binmap4.p + (int64_t)k * np * 4);
+        }
+    } else {
         DBuf<double> aa_s, rhsd4;
         aa_s.alloc(std::max<int64_t>(nb, 1));
         rhsd4.alloc(np * 4);
