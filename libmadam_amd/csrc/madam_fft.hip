@@ -563,6 +563,57 @@ __device__ void lds_fft8_dif(C *s, int L, int logL, int logncol, const C *twL, b
     }
 }
 
+// One round (T <= 3 stages from stage ST on) of the FFTs above, for a length
+// 2^LOG known at compile time, so that every stride, mask and trip count is a
+// constant.  load(a, base, col) fetches the item's points base + m h (h =
+// 2^ST), store(a, base, col) puts them back: LDS between rounds, global memory
+// for a transform's first and last round, which saves two of its LDS round
+// trips.  The operations and their order are those of lds_fft8 / lds_fft8_dif
+// (multiplications by one left out), so the results have the same bits.
+// The passes had been bound by LDS round trips and index arithmetic.  Measured
+// on 64 segments of 2^18 points, FP32, us with lds_fft8 -> with these rounds:
+// rows 94 -> 61 (4.4 TB/s), forward columns 67 -> 50, inverse columns 52 -> 38;
+// 32 segments of 2^19, FP64: rows 111 -> 80, columns 55 -> 44 and 53 -> 35.
+template <typename C, int LOG, int ST, int T, int LOGNCOL, int TPB, bool INV, bool DIF, typename Load, typename Store>
+__device__ inline void fft_round(const C *twL, Load load, Store store)
+{
+    constexpr int h0 = 1 << ST, E = 1 << T, nitems = ((1 << LOG) >> T) << LOGNCOL;
+#pragma unroll
+    for (int t0 = 0; t0 < nitems; t0 += TPB) {
+        const int t = t0 + threadIdx.x;
+        if (nitems % TPB && t >= nitems) break;
+        const int col = t & ((1 << LOGNCOL) - 1), it = t >> LOGNCOL;
+        const int j = it & (h0 - 1), base = (it >> ST) * (E * h0) + j;
+        C a[E], w[3][4];
+        load(a, base, col);
+        item_twiddles(ST == 0 ? CxT<C>::mk(1, 0) : twL[j << (LOG - ST - T)], T, INV, w);
+#pragma unroll
+        for (int q = 0; q < T; ++q) {
+            const int tt = DIF ? T - 1 - q : q;
+#pragma unroll
+            for (int m0 = 0; m0 < E; ++m0) {
+                if (m0 & (1 << tt)) continue;
+                const int r = m0 & ((1 << tt) - 1);
+                const bool one = ST == 0 && r == 0;
+                C x = a[m0], y = a[m0 + (1 << tt)];
+                if (!DIF) {
+                    C b = one ? y : cmul(y, w[tt][r]);
+                    a[m0] = CxT<C>::mk(x.x + b.x, x.y + b.y);
+                    a[m0 + (1 << tt)] = CxT<C>::mk(x.x - b.x, x.y - b.y);
+                } else {
+                    a[m0] = CxT<C>::mk(x.x + y.x, x.y + y.y);
+                    C d = CxT<C>::mk(x.x - y.x, x.y - y.y);
+                    a[m0 + (1 << tt)] = one ? d : cmul(d, w[tt][r]);
+                }
+            }
+        }
+        store(a, base, col);
+    }
+}
+
+// bits of v reversed within LOG bits
+template <int LOG> __device__ inline int rev_c(int v) { return (int)(__brev((unsigned)v) >> (32 - LOG)); }
+
 // ---------------------------------------------------------------- fused convolution
 // Three passes instead of eight (load, 2 x column, 2 x row, spectral, store):
 //   pass 1  forward column FFTs read x - mean straight from the baseline
@@ -587,7 +638,11 @@ static_assert(CONV_COL_TPB % CONV_NCOL == 0, "a column pass thread keeps one col
 
 // grid = (L2 / CONV_NCOL, batch)
 // (C: the work type, double2 or float2; T: the type of x)
-template <typename T, typename C>
+// LOG: log2 of the column length L1 where it is 7 to 9 (0: any length, by
+// lds_fft8).  With it the first round takes its points from x and the last one
+// puts them into work; three rounds of which the last, whatever LOG, has one
+// item per thread.
+template <typename T, typename C, int LOG>
 __global__ void __launch_bounds__(CONV_COL_TPB) k_conv_col_fwd(const T *x, const Segment *seg, int64_t s0, const double *partial_in,
                                C *work, int64_t N, int L1, int logL1, int L2, FftPlan P)
 {
@@ -619,6 +674,62 @@ __global__ void __launch_bounds__(CONV_COL_TPB) k_conv_col_fwd(const T *x, const
     // the stage twiddles, read from LDS by every round of the FFT
     C *tw = s + conv_lds_elems(tot);
     for (int i = threadIdx.x; i < (L1 > 1 ? L1 / 2 : 1); i += blockDim.x) tw[i] = CxT<C>::sub1(P)[i];
+    if constexpr (LOG > 0) {
+        __syncthreads();   // the twiddles
+        const int64_t n2 = c0 + (threadIdx.x & 7);
+        auto lds_in = [&](C *a, int base, int col, int h) {
+#pragma unroll
+            for (int m = 0; m < 8; ++m) a[m] = s[lp((base + m * h) * ncol + col)];
+        };
+        fft_round<C, LOG, 0, 3, 3, CONV_COL_TPB, false, false>(
+            tw,
+            [&](C *a, int base, int col) {
+                // position base + m holds point rev(base + m), the zero padding past noba included
+                const int64_t j0 = 2 * ((int64_t)rev_c<LOG>(base) * L2 + c0 + col);
+                T u[8], v[8];
+#pragma unroll
+                for (int m = 0; m < 8; ++m) {
+                    int64_t jj = j0 + 2 * (int64_t)rev_c<LOG>(m) * L2;
+                    u[m] = jj < noba ? xs[jj] : (T)0;
+                    v[m] = jj + 1 < noba ? xs[jj + 1] : (T)0;
+                }
+#pragma unroll
+                for (int m = 0; m < 8; ++m) {
+                    int64_t jj = j0 + 2 * (int64_t)rev_c<LOG>(m) * L2;
+                    a[m] = CxT<C>::mk(jj < noba ? (S)((double)u[m] - mean) : (S)0,
+                                      jj + 1 < noba ? (S)((double)v[m] - mean) : (S)0);
+                }
+            },
+            [&](C *a, int base, int col) {
+#pragma unroll
+                for (int m = 0; m < 8; ++m) s[lp((base + m) * ncol + col)] = a[m];
+            });
+        __syncthreads();
+        fft_round<C, LOG, 3, 3, 3, CONV_COL_TPB, false, false>(
+            tw, [&](C *a, int base, int col) { lds_in(a, base, col, 8); },
+            [&](C *a, int base, int col) {
+#pragma unroll
+                for (int m = 0; m < 8; ++m) s[lp((base + 8 * m) * ncol + col)] = a[m];
+            });
+        __syncthreads();
+        // W_N^(n2 k1), k1 = base + 64 m: two table reads and the matching powers
+        fft_round<C, LOG, 6, LOG - 6, 3, CONV_COL_TPB, false, false>(
+            tw,
+            [&](C *a, int base, int col) {
+#pragma unroll
+                for (int m = 0; m < (1 << (LOG - 6)); ++m) a[m] = s[lp((base + 64 * m) * ncol + col)];
+            },
+            [&](C *a, int base, int) {
+                C w = tw2(CxT<C>::na(P), CxT<C>::nb(P), (n2 * (int64_t)base) & (N - 1));
+                C ws = tw2(CxT<C>::na(P), CxT<C>::nb(P), (n2 * 64) & (N - 1));
+#pragma unroll
+                for (int m = 0; m < (1 << (LOG - 6)); ++m) {
+                    d[(int64_t)(base + 64 * m) * L2 + n2] = cmul(a[m], w);
+                    w = cmul(w, ws);
+                }
+            });
+        return;
+    }
     // (FP32 work: eight points per thread at a time, every load issued before
     // the LDS stores; FP64 keeps one at a time, the registers of eight cost
     // it more occupancy than the loads gain)
@@ -697,10 +808,17 @@ __device__ inline void conv_pair(C *s, int ik, int im, int64_t k, int64_t N, con
 // k2 * 2 + r (padded).  fc holds the filter spectra in row order
 // (fft_spectrum_rows): f[r + L1 k2] at [r * L2 + k2], f[N] at [N], so a row
 // pair reads two contiguous rows.
-template <typename C>
-__global__ void k_conv_rows(C *work, int64_t N, int L1, int L2, int logL2, FftPlan P, const typename CxT<C>::S *fc,
-                            int64_t fc_stride, const Segment *seg, int64_t s0)
+// LOG: log2 of the row length L2 where it is 8 to 10 (0: any length).  With
+// it the first forward round and the last inverse one work on global memory,
+// and the block has one thread per 8-point item (L2 / 4; 256 left half of them
+// idle at L2 = 512).
+template <typename C, int LOG>
+__global__ void __launch_bounds__(LOG ? 1 << (LOG - 2) : FFT_TPB)
+    k_conv_rows(C *work, int64_t N, int L1, int L2_, int logL2_, FftPlan P, const typename CxT<C>::S *fc,
+                int64_t fc_stride, const Segment *seg, int64_t s0)
 {
+    constexpr int TPB = LOG ? 1 << (LOG - 2) : FFT_TPB;
+    const int logL2 = LOG ? LOG : logL2_, L2 = LOG ? 1 << LOG : L2_;
     using S = typename CxT<C>::S;
     extern __shared__ __align__(16) unsigned char conv_lds[];
     C *s = reinterpret_cast<C *>(conv_lds);
@@ -715,34 +833,72 @@ __global__ void k_conv_rows(C *work, int64_t N, int L1, int L2, int logL2, FftPl
     const C *tw = CxT<C>::sub2(P);
     if (TWL) {
         C *twl = s + conv_lds_elems(tot);
-        for (int i = threadIdx.x; i < (L2 > 1 ? L2 / 2 : 1); i += blockDim.x) twl[i] = tw[i];
+        for (int i = threadIdx.x; i < (L2 > 1 ? L2 / 2 : 1); i += TPB) twl[i] = tw[i];
         tw = twl;
     }
     // natural order in and out of LDS (no bank conflicts): the forward row
     // FFTs are DIF (bit-reversed output), the inverse ones DIT (bit-reversed
     // input), and the spectral step addresses the bit-reversed positions
-    constexpr int NB = sizeof(C) == 8 ? 8 : 1;   // as in k_conv_col_fwd
-    for (int t0 = threadIdx.x; t0 < tot; t0 += NB * blockDim.x) {
-        C in[NB];   // every load issued before the LDS stores
+    auto lds_in = [&](C *a, int base, int r, int h, int e) {
 #pragma unroll
-        for (int k = 0; k < NB; ++k) {
-            int t = t0 + k * blockDim.x;
-            if (t < tot) in[k] = d[(int64_t)((t >> logL2) == 0 ? ra : rb) * L2 + (t & (L2 - 1))];
-        }
+        for (int m = 0; m < 8; ++m)
+            if (m < e) a[m] = s[lp((base + m * h) * 2 + r)];
+    };
+    auto lds_out = [&](C *a, int base, int r, int h, int e) {
 #pragma unroll
-        for (int k = 0; k < NB; ++k) {
-            int t = t0 + k * blockDim.x;
-            if (t < tot) s[lp((t & (L2 - 1)) * 2 + (t >> logL2))] = in[k];
+        for (int m = 0; m < 8; ++m)
+            if (m < e) s[lp((base + m * h) * 2 + r)] = a[m];
+    };
+    if constexpr (LOG > 0) {
+        if (TWL) __syncthreads();
+        fft_round<C, LOG, LOG - 3, 3, 1, TPB, false, true>(
+            tw,
+            [&](C *a, int base, int r) {
+                const C *row = d + (int64_t)(r == 0 ? ra : rb) * L2 + base;
+#pragma unroll
+                for (int m = 0; m < 8; ++m) a[m] = row[m * (L2 / 8)];
+            },
+            [&](C *a, int base, int r) { lds_out(a, base, r, L2 / 8, 8); });
+        __syncthreads();
+        fft_round<C, LOG, LOG - 6, 3, 1, TPB, false, true>(
+            tw, [&](C *a, int base, int r) { lds_in(a, base, r, 1 << (LOG - 6), 8); },
+            [&](C *a, int base, int r) { lds_out(a, base, r, 1 << (LOG - 6), 8); });
+        __syncthreads();
+        constexpr int T3 = LOG - 6 < 3 ? LOG - 6 : 3, S3 = LOG - 6 - T3;
+        fft_round<C, LOG, S3, T3, 1, TPB, false, true>(
+            tw, [&](C *a, int base, int r) { lds_in(a, base, r, 1 << S3, 1 << T3); },
+            [&](C *a, int base, int r) { lds_out(a, base, r, 1 << S3, 1 << T3); });
+        __syncthreads();
+        if constexpr (S3 > 0) {
+            fft_round<C, LOG, 0, S3, 1, TPB, false, true>(
+                tw, [&](C *a, int base, int r) { lds_in(a, base, r, 1, 1 << S3); },
+                [&](C *a, int base, int r) { lds_out(a, base, r, 1, 1 << S3); });
+            __syncthreads();
         }
+    } else {
+        constexpr int NB = sizeof(C) == 8 ? 8 : 1;   // as in k_conv_col_fwd
+        for (int t0 = threadIdx.x; t0 < tot; t0 += NB * TPB) {
+            C in[NB];   // every load issued before the LDS stores
+    #pragma unroll
+            for (int k = 0; k < NB; ++k) {
+                int t = t0 + k * TPB;
+                if (t < tot) in[k] = d[(int64_t)((t >> logL2) == 0 ? ra : rb) * L2 + (t & (L2 - 1))];
+            }
+    #pragma unroll
+            for (int k = 0; k < NB; ++k) {
+                int t = t0 + k * TPB;
+                if (t < tot) s[lp((t & (L2 - 1)) * 2 + (t >> logL2))] = in[k];
+            }
+        }
+        __syncthreads();
+        lds_fft8_dif<C>(s, L2, logL2, 1, tw, false);   // 2 rows
     }
-    __syncthreads();
-    lds_fft8_dif<C>(s, L2, logL2, 1, tw, false);   // 2 rows
     // X[ra + L1 k2] is at bitrev(k2) * 2; X[rb + L1 k2] at bitrev(k2) * 2 + 1
     if (ra == 0) {
         // row 0: pairs {k2, L2 - k2} (k2 = 0 holds X[0] and X[N / 2]);
         // row L1 / 2: pairs {k2, L2 - 1 - k2}
         const int h = L1 / 2;
-        for (int t = threadIdx.x; t <= L2; t += blockDim.x) {
+        for (int t = threadIdx.x; t <= L2; t += TPB) {
             if (t == 0) {
                 C a = s[lp(0)];
                 S x0 = a.x + a.y, xn = a.x - a.y;
@@ -760,7 +916,7 @@ __global__ void k_conv_rows(C *work, int64_t N, int L1, int L2, int logL2, FftPl
             }
         }
     } else {
-        for (int k2 = threadIdx.x; k2 < L2; k2 += blockDim.x) {
+        for (int k2 = threadIdx.x; k2 < L2; k2 += TPB) {
             int64_t kA = (int64_t)ra + (int64_t)L1 * k2;
             int pp = lp(bitrev(k2, logL2) * 2), qq = lp(bitrev(L2 - 1 - k2, logL2) * 2 + 1);
             S fA = f[(int64_t)ra * L2 + k2], fB = f[(int64_t)rb * L2 + L2 - 1 - k2];   // f[kA], f[N - kA]
@@ -769,8 +925,33 @@ __global__ void k_conv_rows(C *work, int64_t N, int L1, int L2, int logL2, FftPl
         }
     }
     __syncthreads();
+    if constexpr (LOG > 0) {
+        constexpr int SL = LOG == 10 ? 9 : 6, TL = LOG - SL;   // the last round
+        fft_round<C, LOG, 0, 3, 1, TPB, true, false>(
+            tw, [&](C *a, int base, int r) { lds_in(a, base, r, 1, 8); },
+            [&](C *a, int base, int r) { lds_out(a, base, r, 1, 8); });
+        __syncthreads();
+        fft_round<C, LOG, 3, 3, 1, TPB, true, false>(
+            tw, [&](C *a, int base, int r) { lds_in(a, base, r, 8, 8); },
+            [&](C *a, int base, int r) { lds_out(a, base, r, 8, 8); });
+        __syncthreads();
+        if constexpr (SL == 9) {
+            fft_round<C, LOG, 6, 3, 1, TPB, true, false>(
+                tw, [&](C *a, int base, int r) { lds_in(a, base, r, 64, 8); },
+                [&](C *a, int base, int r) { lds_out(a, base, r, 64, 8); });
+            __syncthreads();
+        }
+        fft_round<C, LOG, SL, TL, 1, TPB, true, false>(
+            tw, [&](C *a, int base, int r) { lds_in(a, base, r, 1 << SL, 1 << TL); },
+            [&](C *a, int base, int r) {
+                C *row = d + (int64_t)(r == 0 ? ra : rb) * L2 + base;
+#pragma unroll
+                for (int m = 0; m < (1 << TL); ++m) row[m << SL] = a[m];
+            });
+        return;
+    }
     lds_fft8<C>(s, L2, logL2, 1, tw, true);
-    for (int t = threadIdx.x; t < tot; t += blockDim.x) {
+    for (int t = threadIdx.x; t < tot; t += TPB) {
         int r = t >> logL2, n = t & (L2 - 1);
         int row = r == 0 ? ra : rb;
         d[(int64_t)row * L2 + n] = s[lp(n * 2 + r)];
@@ -778,7 +959,8 @@ __global__ void k_conv_rows(C *work, int64_t N, int L1, int L2, int logL2, FftPl
 }
 
 // grid = (L2 / CONV_NCOL, batch)
-template <typename T, typename C>
+// LOG: as in k_conv_col_fwd, the first round from work and the last one into y
+template <typename T, typename C, int LOG>
 __global__ void __launch_bounds__(CONV_COL_TPB) k_conv_col_inv(const C *work, const Segment *seg, int64_t s0, T *y, double *partial_out,
                                int64_t N, int L1, int logL1, int L2, FftPlan P)
 {
@@ -794,37 +976,9 @@ __global__ void __launch_bounds__(CONV_COL_TPB) k_conv_col_inv(const C *work, co
     int tot = L1 * ncol;
     C *tw = s + conv_lds_elems(tot);   // the stage twiddles in LDS
     for (int i = threadIdx.x; i < (L1 > 1 ? L1 / 2 : 1); i += blockDim.x) tw[i] = CxT<C>::sub1(P)[i];
-    {
-        int col = threadIdx.x % ncol, kst = blockDim.x / ncol;
-        int64_t n2 = c0 + col;
-        C w = tw2(CxT<C>::na(P), CxT<C>::nb(P), (n2 * (int64_t)(threadIdx.x / ncol)) & (N - 1));
-        C ws = tw2(CxT<C>::na(P), CxT<C>::nb(P), (n2 * kst) & (N - 1));   /* N is a power of two */
-        constexpr int NB = sizeof(C) == 8 ? 8 : 1;   // as in k_conv_col_fwd
-        for (int k10 = threadIdx.x / ncol; k10 < L1; k10 += NB * kst) {
-            C in[NB];   // every load issued before the twiddle products and LDS stores
-#pragma unroll
-            for (int k = 0; k < NB; ++k) {
-                int k1 = k10 + k * kst;
-                if (k1 < L1) in[k] = d[(int64_t)k1 * L2 + n2];
-            }
-#pragma unroll
-            for (int k = 0; k < NB; ++k) {
-                int k1 = k10 + k * kst;
-                if (k1 < L1) {
-                    s[lp(bitrev(k1, logL1) * ncol + col)] = cmulc(in[k], w);
-                    w = cmul(w, ws);
-                }
-            }
-        }
-    }
-    __syncthreads();
-    lds_fft8<C>(s, L1, logL1, 3, tw, true);
     double acc = 0;
     T *ys = y + sg.b0;
-    for (int t = threadIdx.x; t < tot; t += blockDim.x) {
-        int col = t % ncol, n1 = t / ncol;
-        int64_t jj = 2 * ((int64_t)n1 * L2 + c0 + col);
-        C v = s[lp(n1 * ncol + col)];
+    auto put = [&](C v, int64_t jj) {
         if (jj < noba) {
             double a = (double)v.x * inv;
             ys[jj] = (T)a;
@@ -834,6 +988,88 @@ __global__ void __launch_bounds__(CONV_COL_TPB) k_conv_col_inv(const C *work, co
             double a = (double)v.y * inv;
             ys[jj + 1] = (T)a;
             acc += a;
+        }
+    };
+    if constexpr (LOG > 0) {
+        __syncthreads();   // the twiddles
+        const int64_t n2 = c0 + (threadIdx.x & 7);
+        fft_round<C, LOG, 0, 3, 3, CONV_COL_TPB, true, false>(
+            tw,
+            [&](C *a, int base, int) {
+                // position base + m holds point k1 = rev(base) + rev3(m) H, times W_N^-(n2 k1):
+                // chains of step 64 in k1, as in k_conv_col_fwd
+                constexpr int H = 1 << (LOG - 3), NCH = 64 / H;
+                const int kb = rev_c<LOG>(base);
+                const C *col0 = d + (int64_t)kb * L2 + n2;
+                C in[8];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) in[r] = col0[(int64_t)r * H * L2];
+                C ws = tw2(CxT<C>::na(P), CxT<C>::nb(P), (n2 * 64) & (N - 1));
+#pragma unroll
+                for (int ch = 0; ch < NCH; ++ch) {
+                    C w = tw2(CxT<C>::na(P), CxT<C>::nb(P), (n2 * (int64_t)(kb + ch * H)) & (N - 1));
+#pragma unroll
+                    for (int r = ch; r < 8; r += NCH) {
+                        a[((r & 1) << 2) | (r & 2) | (r >> 2)] = cmulc(in[r], w);
+                        w = cmul(w, ws);
+                    }
+                }
+            },
+            [&](C *a, int base, int col) {
+#pragma unroll
+                for (int m = 0; m < 8; ++m) s[lp((base + m) * ncol + col)] = a[m];
+            });
+        __syncthreads();
+        fft_round<C, LOG, 3, 3, 3, CONV_COL_TPB, true, false>(
+            tw,
+            [&](C *a, int base, int col) {
+#pragma unroll
+                for (int m = 0; m < 8; ++m) a[m] = s[lp((base + 8 * m) * ncol + col)];
+            },
+            [&](C *a, int base, int col) {
+#pragma unroll
+                for (int m = 0; m < 8; ++m) s[lp((base + 8 * m) * ncol + col)] = a[m];
+            });
+        __syncthreads();
+        fft_round<C, LOG, 6, LOG - 6, 3, CONV_COL_TPB, true, false>(
+            tw,
+            [&](C *a, int base, int col) {
+#pragma unroll
+                for (int m = 0; m < (1 << (LOG - 6)); ++m) a[m] = s[lp((base + 64 * m) * ncol + col)];
+            },
+            [&](C *a, int base, int) {
+#pragma unroll
+                for (int m = 0; m < (1 << (LOG - 6)); ++m) put(a[m], 2 * ((int64_t)(base + 64 * m) * L2 + n2));
+            });
+    } else {
+        {
+            int col = threadIdx.x % ncol, kst = blockDim.x / ncol;
+            int64_t n2 = c0 + col;
+            C w = tw2(CxT<C>::na(P), CxT<C>::nb(P), (n2 * (int64_t)(threadIdx.x / ncol)) & (N - 1));
+            C ws = tw2(CxT<C>::na(P), CxT<C>::nb(P), (n2 * kst) & (N - 1));   /* N is a power of two */
+            constexpr int NB = sizeof(C) == 8 ? 8 : 1;   // as in k_conv_col_fwd
+            for (int k10 = threadIdx.x / ncol; k10 < L1; k10 += NB * kst) {
+                C in[NB];   // every load issued before the twiddle products and LDS stores
+    #pragma unroll
+                for (int k = 0; k < NB; ++k) {
+                    int k1 = k10 + k * kst;
+                    if (k1 < L1) in[k] = d[(int64_t)k1 * L2 + n2];
+                }
+    #pragma unroll
+                for (int k = 0; k < NB; ++k) {
+                    int k1 = k10 + k * kst;
+                    if (k1 < L1) {
+                        s[lp(bitrev(k1, logL1) * ncol + col)] = cmulc(in[k], w);
+                        w = cmul(w, ws);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        lds_fft8<C>(s, L1, logL1, 3, tw, true);
+        for (int t = threadIdx.x; t < tot; t += blockDim.x) {
+            int col = t % ncol, n1 = t / ncol;
+            put(s[lp(n1 * ncol + col)], 2 * ((int64_t)n1 * L2 + c0 + col));
         }
     }
     for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
@@ -898,6 +1134,16 @@ static bool conv_fusable(const FftPlan &p)
     return p.L2 >= CONV_NCOL && p.L1 >= 2 && p.L1 * CONV_NCOL <= 8192 && p.L2 <= 2048;
 }
 
+// the pass of length 2^logl: three lengths compiled in (noise filters of 2^15
+// to 2^20 points), any other at run time
+#define CONV_LOG(logl, A, B, D, STMT)                     \
+    switch (logl) {                                       \
+    case A: { constexpr int LOG = A; STMT; } break;       \
+    case B: { constexpr int LOG = B; STMT; } break;       \
+    case D: { constexpr int LOG = D; STMT; } break;       \
+    default: { constexpr int LOG = 0; STMT; } break;      \
+    }
+
 template <typename T>
 void fft_convolve_segments(hipStream_t s, const FftPlan &p, const Segment *dseg, int64_t nseg, const T *x, T *y,
                            const double *fc, const double *fc_rows, int64_t fc_stride, double *work, int64_t batch,
@@ -931,23 +1177,19 @@ void fft_convolve_segments(hipStream_t s, const FftPlan &p, const Segment *dseg,
             size_t col_elems = conv_lds_elems((int)(p.L1 * CONV_NCOL)) + std::max<int64_t>(p.L1 / 2, 1),
                    row_elems = conv_lds_elems((int)(2 * p.L2)) + std::max<int64_t>(p.L2 / 2, 1),
                    row_elems64 = conv_lds_elems((int)(2 * p.L2));   // (FP64 rows: no twiddles in LDS)
-            if (f32) {
-                // FP32 work: the same passes on float2, half the bytes and LDS
-                float2 *w32 = (float2 *)work;
-                k_conv_col_fwd<T, float2><<<gc, CONV_COL_TPB, sizeof(float2) * col_elems, s>>>(
-                    x, dseg, s0, partial + s0 * SEG_NB, w32, p.N, (int)p.L1, logL1, (int)p.L2, p);
-                k_conv_rows<float2><<<gr, FFT_TPB, sizeof(float2) * row_elems, s>>>(
-                    w32, p.N, (int)p.L1, (int)p.L2, logL2, p, fc_rows32, fc_stride, dseg, s0);
-                k_conv_col_inv<T, float2><<<gc, CONV_COL_TPB, sizeof(float2) * col_elems, s>>>(
-                    w32, dseg, s0, y, partial_out + s0 * ncb, p.N, (int)p.L1, logL1, (int)p.L2, p);
-            } else {
-                k_conv_col_fwd<T, double2><<<gc, CONV_COL_TPB, sizeof(double2) * col_elems, s>>>(
-                    x, dseg, s0, partial + s0 * SEG_NB, (double2 *)work, p.N, (int)p.L1, logL1, (int)p.L2, p);
-                k_conv_rows<double2><<<gr, FFT_TPB, sizeof(double2) * row_elems64, s>>>(
-                    (double2 *)work, p.N, (int)p.L1, (int)p.L2, logL2, p, fc_rows, fc_stride, dseg, s0);
-                k_conv_col_inv<T, double2><<<gc, CONV_COL_TPB, sizeof(double2) * col_elems, s>>>(
-                    (const double2 *)work, dseg, s0, y, partial_out + s0 * ncb, p.N, (int)p.L1, logL1, (int)p.L2, p);
-            }
+            auto passes = [&](auto *w, const auto *fcr, size_t row_lds) {
+                using C = std::remove_pointer_t<decltype(w)>;
+                size_t col_lds = sizeof(C) * col_elems;
+                CONV_LOG(logL1, 7, 8, 9, (k_conv_col_fwd<T, C, LOG><<<gc, CONV_COL_TPB, col_lds, s>>>(
+                    x, dseg, s0, partial + s0 * SEG_NB, w, p.N, (int)p.L1, logL1, (int)p.L2, p)));
+                CONV_LOG(logL2, 8, 9, 10, (k_conv_rows<C, LOG><<<gr, LOG ? 1 << (LOG - 2) : FFT_TPB, row_lds, s>>>(
+                    w, p.N, (int)p.L1, (int)p.L2, logL2, p, fcr, fc_stride, dseg, s0)));
+                CONV_LOG(logL1, 7, 8, 9, (k_conv_col_inv<T, C, LOG><<<gc, CONV_COL_TPB, col_lds, s>>>(
+                    w, dseg, s0, y, partial_out + s0 * ncb, p.N, (int)p.L1, logL1, (int)p.L2, p)));
+            };
+            // (FP32 work: the same passes on float2, half the bytes and LDS)
+            if (f32) passes((float2 *)work, fc_rows32, sizeof(float2) * row_elems);
+            else passes((double2 *)work, fc_rows, sizeof(double2) * row_elems64);
             continue;
         }
         k_seg_partial<T><<<gp, FFT_TPB, 0, s>>>(x, 0, 1, dseg, s0, 1.0, partial);
