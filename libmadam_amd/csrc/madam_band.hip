@@ -1224,7 +1224,7 @@ __global__ void k_band_compact_chunks(const double *Li, const int32_t *list, int
 // the same for the whole wave, in LDS (broadcast reads).
 template <int MS, typename V>
 struct BdRows {
-    static constexpr int PF = 4;
+    static constexpr int PF = 2;   // four rows ahead take the registers of a second FP32 wave per SIMD and gain nothing
     double w[PF][BD_K], h[PF];
     __device__ inline void load(const double *lic, const V *tl, int i0, int key)
     {
@@ -1320,32 +1320,40 @@ __device__ inline void bd_bwd(const double *lic, V *tl, double (&X)[BD_KD], int 
 // S += P_l (S of the lane 2^l before (dir 0) or after (dir 1)), l = 0, 1, 2;
 // then the state entering the lane's chunk.  P element e of level l at
 // P[(l BD_KK + e) es].
-template <int DIR>
+template <int DIR, int NR>
 __device__ inline void bd_carry(double (&S)[BD_KD], const double *P, int64_t es)
 {
     const int lane = threadIdx.x;
 #pragma unroll 1
     for (int l = 0; l < BD_LEV; ++l) {
-        // every load of the level before the first use (left to the
-        // scheduler each product waits for its own: 138 us instead of 44 for
-        // one right-hand side of 671 k rows)
-        double M[BD_KK];
-#pragma unroll
-        for (int e = 0; e < BD_KK; ++e) M[e] = P[(int64_t)(l * BD_KK + e) * es];
-        __builtin_amdgcn_sched_barrier(0);
-        double o[BD_KD];
+        double o[BD_KD], sum[BD_KD];
 #pragma unroll
         for (int q = 0; q < BD_KD; ++q) {
             double x = DIR == 0 ? __shfl_up(S[q], 1 << l, 64) : __shfl_down(S[q], 1 << l, 64);
             o[q] = (DIR == 0 ? lane >= (1 << l) : lane + (1 << l) < 64) ? x : 0.0;
         }
 #pragma unroll
-        for (int m = 0; m < BD_KD; ++m) {
-            double a = 0;
+        for (int m0 = 0; m0 < BD_KD; m0 += NR) {
+            // every load of NR rows before the first use (left to the
+            // scheduler each product waits for its own: 138 us instead of 44
+            // for one right-hand side of 671 k rows)
+            double M[NR * BD_KD];
 #pragma unroll
-            for (int q = 0; q < BD_KD; ++q) a = fma(M[m * BD_KD + q], o[q], a);
-            S[m] += a;
+            for (int e = 0; e < NR * BD_KD; ++e)
+                if (m0 * BD_KD + e < BD_KK) M[e] = P[(int64_t)(l * BD_KK + m0 * BD_KD + e) * es];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < NR; ++m) {
+                if (m0 + m >= BD_KD) continue;
+                double a = 0;
+#pragma unroll
+                for (int q = 0; q < BD_KD; ++q) a = fma(M[m * BD_KD + q], o[q], a);
+                sum[m0 + m] = a;
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
+#pragma unroll
+        for (int m = 0; m < BD_KD; ++m) S[m] += sum[m];
     }
 #pragma unroll
     for (int q = 0; q < BD_KD; ++q) {
@@ -1362,7 +1370,8 @@ __device__ inline void bd_solve(const double *lic, const double *Pf, const doubl
 #pragma unroll
     for (int m = 0; m < BD_KD; ++m) S[m] = 0;
     bd_fwd<MS, V, false>(lic, tl, S, key);
-    bd_carry<0>(S, Pf, es);
+    constexpr int NR = sizeof(V) == 8 ? BD_KD : (BD_KD + 1) / 2;   // matrix rows per load round
+    bd_carry<0, NR>(S, Pf, es);
     bd_fwd<MS, V, true>(lic, tl, S, key);
 #pragma unroll
     for (int m = 0; m < BD_KD; ++m) S[m] = 0;
@@ -1370,13 +1379,19 @@ __device__ inline void bd_solve(const double *lic, const double *Pf, const doubl
     // lanes outside the segment send nothing back into it
 #pragma unroll
     for (int m = 0; m < BD_KD; ++m) S[m] = valid ? S[m] : 0.0;
-    bd_carry<1>(S, Pb, es);
+    bd_carry<1, NR>(S, Pb, es);
     bd_bwd<MS, V, true>(lic, tl, S, key);
 }
 
 // z = M^-1 r (r and z do not overlap: the halo of one block is another's own)
+// Registers: two FP32 waves per SIMD (256 registers each; 21.5 KB of LDS let
+// seven blocks on a CU), so that one computes while the other waits; one wave
+// per SIMD took 244 us for 16 right-hand sides of 1.34 M rows, two 185 (one of
+// 21.5 M rows: 266 -> 211).  FP64 tiles (38 KB) leave one wave per SIMD whatever
+// the registers: each matrix of bd_carry is then loaded whole (154 us for 10.7 M
+// rows, 157 in halves).
 template <typename V>
-__global__ void __launch_bounds__(64) k_band_direct(const BandBlk *__restrict__ blk, const ChunkInfo *__restrict__ ch,
+__global__ void __launch_bounds__(64, sizeof(V) == 8 ? 1 : 2) k_band_direct(const BandBlk *__restrict__ blk, const ChunkInfo *__restrict__ ch,
                                                     const int32_t *bmap, const double *Li,
                                                     const double *__restrict__ Lu, const double *__restrict__ Pf,
                                                     const double *__restrict__ Pb, const int32_t *__restrict__ pslot,
