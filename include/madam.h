@@ -132,8 +132,8 @@ int madam_get_filter(void *ctx, int ipsd, double *fcov);
 /* projection kernels (low 4 bits): 0 = segmented 512-entry tiles on the pixel
  * side and LDS tiles on the baseline side (default), 1 = wave per pixel / lane
  * group per baseline, 2 = LDS tiles on both sides, 3 = segmented tiles on both
- * sides; + 16 = band factorization computes every row (no periodic
- * continuation of repeating 64-row blocks); + 32 / + 64 = band carry chains
+ * sides; + 16 = band factorization computes every row in one chain (no periodic
+ * continuation of repeating 64-row blocks, no pieces); + 32 / + 64 = band carry chains
  * always / never several per wave (default: several when there are enough
  * of them), + 128 (before the first solve on a pointing) = run records of the
  * projections whatever the number of samples */
