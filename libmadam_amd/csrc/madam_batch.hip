@@ -979,22 +979,9 @@ __global__ void k_bupdate_r(const BatchScal *sc, const int *active, T *__restric
     }
 }
 
-// p = z + beta p (active right-hand sides)
-template <typename T>
-__global__ void k_bupdate_p(const BatchScal *sc, const int *active, T *p, const T *z, int64_t n)
-{
-    int y = blockIdx.y;
-    if (!active[y]) return;
-    T beta = (T)sc[y].beta;
-    int64_t off = (int64_t)y * n;
-    for (int64_t i = off + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < off + n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = z[i] + beta * p[i];
-}
-
 // p = z + beta p on a tile of BPW_TB baselines x R (RHS-major rows), and the
 // next operator's pw[bslot[b] * R + r] = p[r][b] * dwb[b] from the same tile
-// (0 for finished right-hand sides): k_bupdate_p and k_bpw in one pass
+// (0 for finished right-hand sides): the p update and k_bpw in one pass
 template <typename T, int R>
 __global__ void __launch_bounds__(BTPB) k_bupdate_p_pw(const BatchScal *sc, const int *active, T *__restrict__ p,
                                                        const T *__restrict__ z, int64_t nbtot,
@@ -1111,13 +1098,6 @@ void batch_update_r(hipStream_t s, int R, const BatchScal *sc, const int *active
 {
     dim3 g((unsigned)bgrid(n, BTPB, 4096), (unsigned)R);
     k_bupdate_r<T><<<g, BTPB, 0, s>>>(sc, active, x, r, ro, p, ap, n);
-}
-
-template <typename T>
-void batch_update_p(hipStream_t s, int R, const BatchScal *sc, const int *active, T *p, const T *z, int64_t n)
-{
-    dim3 g((unsigned)bgrid(n, BTPB, 4096), (unsigned)R);
-    k_bupdate_p<T><<<g, BTPB, 0, s>>>(sc, active, p, z, n);
 }
 
 // ---------------------------------------------------------------- elementwise helpers
@@ -1429,7 +1409,6 @@ template void batch_bin<double>(hipStream_t, int, int, bool, int64_t, const int6
                                 double *);                                                                         \
     template void batch_update_r<T>(hipStream_t, int, const BatchScal *, const int *, T *, T *, T *, const T *,     \
                                     const T *, int64_t);                                                           \
-    template void batch_update_p<T>(hipStream_t, int, const BatchScal *, const int *, T *, const T *, int64_t);     \
     template void batch_accumulate<T>(hipStream_t, int, double *, const T *, const int *, int64_t);                \
     template void batch_diag<T>(hipStream_t, int, const T *, const double *, T *, int64_t);                        \
     template void batch_copy<T>(hipStream_t, T *, const T *, int64_t);                                             \

@@ -87,8 +87,6 @@ size_t batch_partials_doubles(int R);
 template <typename T>
 void batch_update_r(hipStream_t s, int R, const BatchScal *sc, const int *active, T *x, T *r, T *ro, const T *p,
                     const T *ap, int64_t n);
-template <typename T>
-void batch_update_p(hipStream_t s, int R, const BatchScal *sc, const int *active, T *p, const T *z, int64_t n);
 template <typename TI, typename TO>
 void batch_cast(hipStream_t s, const TI *in, TO *out, int64_t n);
 template <typename T>
