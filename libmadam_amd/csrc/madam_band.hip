@@ -1832,6 +1832,8 @@ static void band_build_direct(hipStream_t s, const BandPrec &bp, BandImpl *im, c
     im->direct = w < BD_NEGLIGIBLE;
 }
 
+int band_capacity(const BandPrec &bp) { return bp.impl ? ((const BandImpl *)bp.impl)->rcap : 0; }
+
 // grow the carry-state buffers to nrhs right-hand sides
 void band_reserve(const BandPrec &bp, int nrhs)
 {

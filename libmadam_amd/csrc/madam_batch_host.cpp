@@ -15,21 +15,40 @@
 //   r = yba - A64 a; solve A32 d = r to the reduction the tolerance still
 //   needs; a += d; until rr / rrinit < cglimit on the FP64 residual.
 //
-// One PCG step is the same sequence of launches every time, so it is
-// captured once into a HIP graph and replayed (unless the inner-CG
-// preconditioner fallback, which synchronises with the host, is in use).
+// One PCG step of a batch is the same sequence of launches every time, so it
+// is captured into a HIP graph and replayed, also by later batches whose
+// launches would be the same (unless the inner-CG preconditioner fallback,
+// which synchronises with the host, is in use).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <type_traits>
 #include <vector>
 
 #include "madam_context.hpp"
 
 namespace madam {
+
+// A captured PCG step: its launches replay with the grids and arguments they
+// were captured with, so it serves only while every one of them is what a
+// launch would use now (key, from step_key).
+struct StepGraph {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    std::vector<uint64_t> key;
+    void drop()
+    {
+        if (exec) (void)hipGraphExecDestroy(exec);
+        if (graph) (void)hipGraphDestroy(graph);
+        exec = nullptr;
+        graph = nullptr;
+    }
+};
 
 struct BatchState {
     int nrhs = 0, R = 0, prec = 0;
@@ -71,12 +90,9 @@ struct BatchState {
     // per right-hand side results
     std::vector<BatchScal> hsc, hsc64;
     std::vector<int> inner_steps;
-    // the captured PCG step, per vector type
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
-    hipGraph_t graph[2] = {nullptr, nullptr};
-    // the same step without exit tests, for madam_iterate_batch
-    hipGraphExec_t gexec_free = nullptr;
-    hipGraph_t graph_free = nullptr;
+    // the captured PCG step, per vector type, and the same step without exit
+    // tests, for madam_iterate_batch
+    StepGraph step[2], step_free;
     bool use_graph = true;
     double t_setup = 0, t_solve = 0, t_inner = 0;
     int64_t n_inner = 0, n_outer = 0;
@@ -86,16 +102,7 @@ struct BatchState {
 
     void drop_graphs()
     {
-        for (int i = 0; i < 2; ++i) {
-            if (gexec[i]) (void)hipGraphExecDestroy(gexec[i]);
-            if (graph[i]) (void)hipGraphDestroy(graph[i]);
-            gexec[i] = nullptr;
-            graph[i] = nullptr;
-        }
-        if (gexec_free) (void)hipGraphExecDestroy(gexec_free);
-        if (graph_free) (void)hipGraphDestroy(graph_free);
-        gexec_free = nullptr;
-        graph_free = nullptr;
+        for (StepGraph *g : {&step[0], &step[1], &step_free}) g->drop();
     }
     int *h_active = nullptr;   // pinned: the active flags after the last two steps
     ~BatchState()
@@ -436,6 +443,65 @@ static void pcg_step(Context &c, BatchState &B, const Vec<T> &v, double lim, int
     }
 }
 
+// What pcg_step's launches depend on.  Tables of the pointing and of the
+// preconditioner are rebuilt in place of the old ones: set_up counts them.
+// Everything else is listed: sizes of grids and loops, branches, scalar
+// arguments, and the buffers that a later batch may allocate anew.
+template <typename T>
+static std::vector<uint64_t> step_key(Context &c, BatchState &B, const Vec<T> &v, double lim, int iter_min,
+                                      int iter_max, int stall)
+{
+    uint64_t lim_bits;
+    static_assert(sizeof lim_bits == sizeof lim, "");
+    memcpy(&lim_bits, &lim, sizeof lim);
+    std::vector<uint64_t> k{lim_bits,
+                            c.set_up,
+                            (uint64_t)c.kernel_variant,
+                            (uint64_t)B.nrhs,
+                            (uint64_t)B.R,
+                            (uint64_t)iter_min,
+                            (uint64_t)iter_max,
+                            (uint64_t)stall,
+                            (uint64_t)B.segR.size(),
+                            (uint64_t)B.fft_nseg,
+                            (uint64_t)B.fft_batch64,
+                            (uint64_t)B.fft_batch32,
+                            (uint64_t)B.rle_ok,
+                            (uint64_t)B.bt.nitems,
+                            (uint64_t)B.bt.nfix,
+                            (uint64_t)B.bt.nparts,
+                            (uint64_t)B.bt_c.nitems,
+                            (uint64_t)B.bt_c.nfix,
+                            (uint64_t)B.bt_c.nparts,
+                            (uint64_t)c.runs_ok,
+                            (uint64_t)c.runs32_ok,
+                            (uint64_t)band_capacity(c.band)};
+    for (const void *p : std::initializer_list<const void *>{
+             v.x, v.r, v.ro, v.z, v.p, v.ap, v.pw, v.m, v.part, B.dots.p, B.sc.p, B.active.p, B.d_segR.p, B.fftwork.p,
+             Ops<T>::dwb(c, B), Ops<T>::nna(c, B), Ops<T>::cc(c, B), Ops<T>::m4(c, B), Ops<T>::fcov32(B),
+             Ops<T>::fprec32(B), B.bt.items, B.bt.fix, B.bt_c.items, B.bt_c.fix, B.rg_rec.p, B.rg_st.p, B.rg_base.p,
+             B.rs_rec.p, c.d_rung.p, c.d_rungw.p, c.d_rungw32.p, c.d_runs.p, c.d_runsw.p, c.d_runsw32.p})
+        k.push_back((uint64_t)(uintptr_t)p);
+    return k;
+}
+
+// one PCG step from its graph, captured where the one there is another step's
+template <typename T>
+static void launch_step(Context &c, BatchState &B, StepGraph &g, const Vec<T> &v, double lim, int iter_min,
+                        int iter_max, int stall)
+{
+    std::vector<uint64_t> key = step_key<T>(c, B, v, lim, iter_min, iter_max, stall);
+    if (!g.exec || g.key != key) {
+        g.drop();
+        MADAM_CHECK(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
+        pcg_step<T>(c, B, v, lim, iter_min, iter_max, stall);
+        MADAM_CHECK(hipStreamEndCapture(c.stream, &g.graph));
+        MADAM_CHECK(hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
+        g.key = std::move(key);
+    }
+    MADAM_CHECK(hipGraphLaunch(g.exec, c.stream));
+}
+
 static constexpr double AHEAD_STEP = 1e-3;   // steps shorter than this (s) are queued ahead
 
 static int count_active(Context &c, BatchState &B)
@@ -465,7 +531,7 @@ static int64_t batch_pcg(Context &c, BatchState &B, const Vec<T> &v, const T *b,
     batch_final(s, R, B.dots.p, 2, B.sc.p, B.active.p, lim, iter_min, iter_max, allow);
     // the first step's pixel-side input (the steps leave it for the next one)
     batch_pw<T>(s, R, v.p, nb, c.d_bord.p, c.d_bslot.p, Ops<T>::dwb_s(c, B), Ops<T>::dwb(c, B), B.active.p, v.pw);
-    int gi = std::is_same<T, float>::value ? 1 : 0;
+    StepGraph &graph_of = B.step[std::is_same<T, float>::value ? 1 : 0];
     // profiling times every part with events, so the steps run as launched
     bool graph = B.use_graph && c.segcg.empty() && !c.profile;
     StepTimers tmr;
@@ -473,13 +539,7 @@ static int64_t batch_pcg(Context &c, BatchState &B, const Vec<T> &v, const T *b,
         if (c.profile) {
             pcg_step<T>(c, B, v, lim, iter_min, iter_max, stall, &tmr);
         } else if (graph) {
-            if (!B.gexec[gi]) {
-                MADAM_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-                pcg_step<T>(c, B, v, lim, iter_min, iter_max, stall);
-                MADAM_CHECK(hipStreamEndCapture(s, &B.graph[gi]));
-                MADAM_CHECK(hipGraphInstantiate(&B.gexec[gi], B.graph[gi], nullptr, nullptr, 0));
-            }
-            MADAM_CHECK(hipGraphLaunch(B.gexec[gi], s));
+            launch_step<T>(c, B, graph_of, v, lim, iter_min, iter_max, stall);
         } else {
             pcg_step<T>(c, B, v, lim, iter_min, iter_max, stall);
         }
@@ -710,7 +770,6 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
     int64_t n = (int64_t)c.ndet * c.nsamp, nb = c.nbtot, np = c.npix_map;
     if (!c.batch) c.batch = new BatchState();
     BatchState &B = *c.batch;
-    if (B.R != R || B.prec != precision || !B.tables_ok || B.tables_ent != ent_records(c)) B.drop_graphs();
     B.nrhs = nrhs;
     B.prec = precision;
     B.t_inner = 0;
@@ -730,8 +789,6 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
     };
     // shared set-up with the first signal
     solve_setup<TT>(c, signal(0));
-    bool rebuilt_prec = c.stats[ST_PREC_REUSED] == 0;
-    if (rebuilt_prec || B.R != R) B.drop_graphs();
     B.R = R;
     B.yba.alloc((size_t)std::max<int64_t>(nb, 1) * R);
     B.rhs4.alloc((size_t)np * 4 * R);
@@ -764,10 +821,9 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
             v.part = tp<double>(B.part);
             B.tables_ok = true;
             B.tables_ent = ent_records(c);
-            B.drop_graphs();
         }
         v.x = B.a64.p;
-        B.drop_graphs();   // the solution vector is bound into the captured step
+        B.step[0].drop();   // (every FP64 batch captures its step)
         double t0 = now();
         batch_pcg<double>(c, B, v, B.yba.p, B.ones.p, p.cglimit, p.iter_min, p.iter_max, 0);
         B.hsc.resize(R);
@@ -792,7 +848,6 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
         const char *e32 = getenv("MADAM_FFT32");
         bool fft32 = !(e32 && atoi(e32) == 0);
         int64_t nspec = (int64_t)(c.nof / 2 + 1) * c.npsdtot;
-        const float *old_f = B.fcov_rows32.p, *old_p = B.fprec_rows32.p;
         if (fft32 && c.p.kfilter && c.d_fcov_rows.p) {
             B.fcov_rows32.alloc((size_t)nspec);
             batch_cast<double, float>(s, c.d_fcov_rows.p, B.fcov_rows32.p, nspec);
@@ -805,7 +860,6 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
         } else {
             B.fprec_rows32.release();
         }
-        if (B.fcov_rows32.p != old_f || B.fprec_rows32.p != old_p) B.drop_graphs();   // bound into the captured step
         if (R == 1) runs_prepare_fp32(c);
         Vec<float> v = alloc_vectors<float>(c, B);
         B.m4f.alloc((size_t)std::max<int64_t>(c.npix_cross, 1) * 4);
@@ -813,12 +867,8 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
             tune_pieces<float>(c, B, v);
             B.tables_ok = true;
             B.tables_ent = ent_records(c);
-            B.drop_graphs();
         }
-        if (R >= 8 && !B.rle_ok) {
-            build_rle(c, B);
-            B.drop_graphs();
-        }
+        if (R >= 8 && !B.rle_ok) build_rle(c, B);
         int64_t nparts = std::max<int64_t>(B.bt.nparts, B.rle_ok ? B.bt_c.nparts : 0);
         B.part.alloc((size_t)std::max<int64_t>(nparts, 1) * c.nmap * R * sizeof(float));
         v.part = tp<float>(B.part);
@@ -944,13 +994,7 @@ static void iterate_t(Context &c, BatchState &B, const T *b, int niter)
         if (c.profile) {
             pcg_step<T>(c, B, v, 0.0, 0, big, 0, &tmr);
         } else if (graph) {
-            if (!B.gexec_free) {
-                MADAM_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-                pcg_step<T>(c, B, v, 0.0, 0, big, 0);
-                MADAM_CHECK(hipStreamEndCapture(s, &B.graph_free));
-                MADAM_CHECK(hipGraphInstantiate(&B.gexec_free, B.graph_free, nullptr, nullptr, 0));
-            }
-            MADAM_CHECK(hipGraphLaunch(B.gexec_free, s));
+            launch_step<T>(c, B, B.step_free, v, 0.0, 0, big, 0);
         } else {
             pcg_step<T>(c, B, v, 0.0, 0, big, 0);
         }

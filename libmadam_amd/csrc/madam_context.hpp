@@ -253,6 +253,7 @@ struct Context {
     // configuration, pointing and kernel choice stay and reused when nna is
     // bitwise the same (they are functions of those alone)
     bool prec_cached = false;
+    uint64_t set_up = 0;   // builds of the pointing's and the preconditioner's tables so far
     int prec_cached_variant = 0;
     DBuf<double> d_nna_key;
     DBuf<int> d_flag;

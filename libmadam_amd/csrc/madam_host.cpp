@@ -650,6 +650,7 @@ static void build_filters(Context &c)
 static void set_pointing(Context &c, int32_t *pix, float *w, int on_device, bool dummy_is_flag = false)
 {
     if (!c.configured) fail("madam_set_pointing called before configure");
+    c.set_up++;
     hipStream_t s = c.stream;
     double t0 = now();
     int64_t n = (int64_t)c.ndet * c.nsamp;
@@ -1588,7 +1589,10 @@ void solve_setup(Context &c, const TT *tod)
             MADAM_CHECK(hipStreamSynchronize(s));
             reuse = differ == 0;
         }
-        if (!reuse) build_segments(c);
+        if (!reuse) {
+            c.set_up++;
+            build_segments(c);
+        }
         c.stats[ST_PREC_REUSED] = reuse ? 1 : 0;
         tm.stop(s);
         c.stats[ST_T_INIT] = tm.ms() * 1e-3;

@@ -442,6 +442,8 @@ template <typename T>
 void band_apply(hipStream_t s, const BandPrec &bp, const T *r, T *z, int nrhs = 1, int64_t vstride = 0);
 // make room for nrhs right-hand sides in band_apply (allocates; call outside graph capture)
 void band_reserve(const BandPrec &bp, int nrhs);
+// the right-hand sides there is room for (the buffers move when that grows)
+int band_capacity(const BandPrec &bp);
 void band_free(BandPrec &bp);
 
 // ------------------------------------------------------------------ pointing.hip
