@@ -87,8 +87,10 @@ struct BatchState {
     DBuf<double> fftwork;
     int64_t fft_nseg = 0;
     int64_t fft_batch64 = 1, fft_batch32 = 1;   // segments per FFT batch of the FP64 / FP32 convolution
-    // per right-hand side results
+    // per right-hand side results: the scalars once the batch's PCG has ended
+    // (empty before), then the maps
     std::vector<BatchScal> hsc, hsc64;
+    bool maps_ok = false;
     std::vector<int> inner_steps;
     // the captured PCG step, per vector type, and the same step without exit
     // tests, for madam_iterate_batch
@@ -118,7 +120,8 @@ void batch_release(Context &c)
     c.batch = nullptr;
 }
 
-// a new pointing: the work items and the captured steps refer to the old one
+// a new configuration or pointing: the work items, the captured steps and the
+// results refer to the old one
 void batch_invalidate(Context &c)
 {
     if (!c.batch) return;
@@ -771,6 +774,8 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
     if (!c.batch) c.batch = new BatchState();
     BatchState &B = *c.batch;
     B.nrhs = nrhs;
+    B.hsc.clear();
+    B.maps_ok = false;
     B.prec = precision;
     B.t_inner = 0;
     B.n_inner = 0;
@@ -911,10 +916,10 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
             batch_final(s, R, B.dots.p, 3, B.sc64.p, B.active64.p, p.cglimit, 0, max_outer);
             B.n_outer++;
         }
-        B.hsc.resize(R);
         B.hsc64.resize(R);
-        d2h(B.hsc.data(), B.sc.p, R, s);
         d2h(B.hsc64.data(), B.sc64.p, R, s);
+        B.hsc.resize(R);
+        d2h(B.hsc.data(), B.sc.p, R, s);
         MADAM_CHECK(hipStreamSynchronize(s));
         B.t_solve = now() - t0;
     }
@@ -960,6 +965,7 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
     }
     MADAM_CHECK(hipGetLastError());
     MADAM_CHECK(hipStreamSynchronize(s));
+    B.maps_ok = true;
     B.t_setup = now() - tstart - B.t_solve;
 }
 
@@ -1003,9 +1009,13 @@ static void iterate_t(Context &c, BatchState &B, const T *b, int niter)
     MADAM_CHECK(hipStreamSynchronize(s));
 }
 
+// The last batch's PCG has ended, so its vectors and scalars are there (its
+// maps, unless a right-hand side was diverging: maps_ok).
+static bool batch_ended(const Context &c) { return c.batch && c.batch->nrhs > 0 && !c.batch->hsc.empty(); }
+
 void batch_iterate(Context &c, int niter)
 {
-    if (!c.batch || c.batch->nrhs == 0) fail("madam_iterate_batch needs a completed madam_solve_batch");
+    if (!batch_ended(c)) fail("madam_iterate_batch needs a completed madam_solve_batch");
     BatchState &B = *c.batch;
     if (B.prec == 0) {
         iterate_t<double>(c, B, B.yba.p, niter);
@@ -1027,7 +1037,7 @@ void batch_reset_timers(Context &c)
 
 static BatchState &batch_of(Context &c, int irhs)
 {
-    if (!c.batch || c.batch->nrhs == 0) fail("no batched solution available");
+    if (!batch_ended(c)) fail("no batched solution available");
     if (irhs < 0 || irhs >= c.batch->nrhs) fail("right-hand side %d outside 0..%d", irhs, c.batch->nrhs - 1);
     return *c.batch;
 }
@@ -1035,6 +1045,7 @@ static BatchState &batch_of(Context &c, int irhs)
 void batch_get_maps(Context &c, int irhs, double *map, double *binmap)
 {
     BatchState &B = batch_of(c, irhs);
+    if (!B.maps_ok) fail("the last madam_solve_batch failed before it made maps");
     int64_t np = c.npix_map;
     int nm = c.nmap;
     std::vector<OutItem> out;

@@ -349,6 +349,10 @@ static void configure(Context &c, const char *parstring, long ndet, const char *
     if (nnz != 1 && nnz != 3) fail("nnz=%ld is not supported (nmap must be 1 or 3)", nnz);
     if (p.has_inmask || p.has_spectrum || p.has_covmat) fail("file_inmask / file_spectrum / file_covmat are not supported");
     if ((uint64_t)ndet * (uint64_t)nsamp >= (1ULL << 32)) fail("ndet * nsamp must be below 2^32");
+    // the sizes change from here on, also where the configuration is refused
+    // further down: no set-up or result of the old one may be used with them
+    c.configured = c.pointed = c.solved = c.prec_cached = false;
+    batch_invalidate(c);
     c.ndet = (int)ndet;
     c.nsamp = nsamp;
     c.nnz = (int)nnz;
@@ -575,9 +579,6 @@ static void configure(Context &c, const char *parstring, long ndet, const char *
         MADAM_CHECK(hipStreamSynchronize(s));
     }
     c.configured = true;
-    c.pointed = false;
-    c.solved = false;
-    c.prec_cached = false;
 }
 
 // ------------------------------------------------------------------ noise filter on the device
