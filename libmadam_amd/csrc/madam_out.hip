@@ -17,10 +17,10 @@
 #include <cstdint>
 #include <cstring>
 #include <mutex>
-#include <thread>
 #include <vector>
 
 #include "madam_context.hpp"
+#include "madam_workers.hpp"
 
 namespace madam {
 
@@ -114,6 +114,7 @@ static void *slot_take()
         return p;
     }
     if (g_out_made >= OUT_SLOTS) return nullptr;
+    g_out_free.reserve(OUT_SLOTS);   // giving a slot back cannot fail
     void *p = nullptr;
     if (hipHostMalloc(&p, OUT_SLOT, hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError();
@@ -123,11 +124,27 @@ static void *slot_take()
     return p;
 }
 
-static void slot_give(void *p)
-{
-    std::lock_guard<std::mutex> lk(g_out_mu);
-    g_out_free.push_back(p);
-}
+// up to `want` slots, given back once the kernels on the stream that write them have ended
+struct SlotLease {
+    std::vector<void *> p;
+    hipStream_t s;
+    SlotLease(int want, hipStream_t st) : s(st)
+    {
+        p.reserve(want);
+        while ((int)p.size() < want) {
+            void *q = slot_take();
+            if (!q) break;
+            p.push_back(q);
+        }
+    }
+    ~SlotLease()
+    {
+        if (p.empty()) return;
+        (void)hipStreamSynchronize(s);
+        std::lock_guard<std::mutex> lk(g_out_mu);
+        for (void *q : p) g_out_free.push_back(q);
+    }
+};
 
 // ------------------------------------------------------------------ copies
 
@@ -204,13 +221,8 @@ void copy_out(Context &c, const std::vector<OutItem> &items)
     // a thread per 8 MB: 685 MB take 63 / 34 / 20 / 15 ms with 1 / 2 / 4 / 8
     // threads, 36 MB 2.0 / 1.3 / 1.0 / 1.1
     int want = (int)std::min<size_t>((total + 2 * OUT_SLOT - 1) / (2 * OUT_SLOT), OUT_SLOTS);
-    std::vector<void *> slots;
-    while ((int)slots.size() < want) {
-        void *p = slot_take();
-        if (!p) break;
-        slots.push_back(p);
-    }
-    if (slots.empty()) {
+    SlotLease slots(want, s);
+    if (slots.p.empty()) {
         // every slot is lent: lay out in device scratch and let the runtime copy
         DBuf<char> d;
         d.alloc(OUT_SLOT);
@@ -225,15 +237,9 @@ void copy_out(Context &c, const std::vector<OutItem> &items)
         MADAM_CHECK(hipStreamSynchronize(s));
         return;
     }
-    std::vector<std::thread> th;
-    for (size_t i = 1; i < slots.size(); ++i) th.emplace_back(work, slots[i]);
-    work(slots[0]);
-    for (auto &t : th) t.join();
-    // the kernels that write a slot have ended once the stream has
-    hipError_t e = hipStreamSynchronize(s);
-    for (void *p : slots) slot_give(p);
+    run_workers((int)slots.p.size(), [&](int i) { work(slots.p[i]); });
     MADAM_CHECK(err);
-    MADAM_CHECK(e);
+    MADAM_CHECK(hipStreamSynchronize(s));
 }
 
 }  // namespace madam
