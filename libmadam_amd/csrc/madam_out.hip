@@ -153,6 +153,8 @@ static constexpr size_t OUT_SMALL = 1 << 20;   // one launch and one copy up to 
 void copy_out(Context &c, const std::vector<OutItem> &items)
 {
     hipStream_t s = c.stream;
+    // an error that an earlier call of the caller's left is not one of the launches below
+    (void)hipGetLastError();
     size_t total = 0;
     for (const OutItem &it : items) total += (size_t)it.n * elem_bytes(it.kind) + 8;
     if (total <= OUT_SMALL) {

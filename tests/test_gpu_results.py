@@ -78,3 +78,23 @@ def test_results_of_another_configuration_are_refused(accepted):
         with pytest.raises(libmadam_amd.MadamError):
             call()
     m.close()
+
+
+def test_products_after_an_error_of_the_callers():
+    """A refused runtime call of the caller's own (a device that is not there)
+    leaves an error behind; reading products must not take it for its own."""
+    import ctypes
+    import libmadam_amd
+    case = ring(prior=False, nside=64, nsamp=20000)   # maps of 10 MB: the threaded path, the baselines the small one
+    m = libmadam_amd.Madam(0)
+    a = configure(m, case)
+    m.set_pointing(a[4], a[5])
+    m.solve(case["signal"].copy())
+    want = m.maps(), m.baselines()
+    hip = ctypes.CDLL(libmadam_amd.lib()._name)   # the runtime that the library is linked with
+    for k, call in enumerate((m.maps, m.baselines)):
+        assert hip.hipSetDevice(9999) != 0
+        got = call()
+        for name in got:
+            assert np.array_equal(got[name], want[k][name]), name
+    m.close()
