@@ -242,7 +242,8 @@ def run_cfg3(a):
     nprof = max(prof["n_prof"], 1)
     times = dict(scatter=prof["t_scatter"] / nprof, gather=prof["t_gather"] / nprof)
     # one right-hand side runs the FP32 instantiations of the FP64 path's kernels
-    roof, kern = roofline_from(times, bytes_fp64(st, ndet, nsamp, npix_hit, nbtot, 4),
+    st32 = dict(st, run_records=prof.get("run_records"))
+    roof, kern = roofline_from(times, bytes_fp64(st32, ndet, nsamp, npix_hit, nbtot, 4),
                                dict(scatter="k_sr_scatter<float, 3, 4, 1>", gather="k_gather_flat<float, 3, 1>"),
                                "cfg3")
     value = N / t_mixed

@@ -83,8 +83,8 @@ int madam_get_baselines(void *ctx, double *aa, double *yba, double *nna);
  * nactive, t_total, t_step, ncg, band_chunks, band_chunks_unique, band_blocks,
  * band_blocks_unique, rec_bytes, band_rows_factored, prec_reused,
  * pointing_reused, nwide, run_records (the order of STAT_NAMES in
- * libmadam_amd/__init__.py; run_records: runs of samples that the baseline
- * side of the one-right-hand-side projections reads, 0 where it reads samples) */
+ * libmadam_amd/__init__.py; run_records: runs of samples that the baseline side
+ * of the FP64 one-right-hand-side projections reads, 0 where it reads samples) */
 int madam_get_stats(void *ctx, double *out, int n);
 int madam_get_rr_history(void *ctx, double *out, int n);
 int madam_set_profiling(void *ctx, int on);
@@ -119,7 +119,9 @@ int madam_get_batch_baselines(void *ctx, int irhs, double *aa, double *yba);
  * madam_set_profiling on, the summed HIP-event times of the steps' pixel
  * side, prior, baseline side, preconditioner and whole step, and the number
  * of steps timed; the run-length records of the FP32 operator on the baseline
- * and pixel sides (0 when it reads the sample records) (n <= 18) */
+ * and pixel sides (0 when it reads the sample records); for one right-hand
+ * side, the run records that its operator's baseline side reads (0: samples)
+ * (n <= 19) */
 int madam_get_batch_info(void *ctx, int irhs, double *out, int n);
 /* one operator of the last madam_solve on host vectors x, y of ndet * nbase
  * baselines: which 0 = noise prior y = C_a^-1 x (cinvmul, src/noise_routines.f90:745-913),

@@ -294,7 +294,7 @@ class Madam:
         _check(lib().madam_get_batch_baselines(self._h, int(irhs), _ptr(aa), _ptr(yba)))
         keys = ["steps", "status", "rr_inner", "passes", "rr_final", "t_setup", "t_solve", "pcg_steps", "t_pcg",
                 "piece", "t_scatter", "t_prior", "t_gather", "t_prec", "t_step", "n_prof", "rle_records_gather",
-                "rle_records_scatter"]
+                "rle_records_scatter", "run_records"]
         info = np.zeros(len(keys))
         _check(lib().madam_get_batch_info(self._h, int(irhs), _ptr(info), len(keys)))
         return dict(map=m, binmap=b, aa=aa, yba=yba, info=dict(zip(keys, info.tolist())))

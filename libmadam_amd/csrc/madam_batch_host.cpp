@@ -1074,7 +1074,7 @@ void batch_get_info(Context &c, int irhs, double *out, int n)
 {
     BatchState &B = batch_of(c, irhs);
     const BatchScal &S = B.hsc[irhs];
-    double v[18];
+    double v[19];
     v[0] = S.steps;
     v[1] = S.status;
     v[2] = S.rr0 > 0 ? S.rr / S.rr0 : 0;
@@ -1100,7 +1100,9 @@ void batch_get_info(Context &c, int irhs, double *out, int n)
     // run-length records of the FP32 operator (0: sample records)
     v[16] = B.rle_ok ? (double)B.n_rg : 0;
     v[17] = B.rle_ok ? (double)B.n_rs : 0;
-    for (int i = 0; i < n && i < 18; ++i) out[i] = v[i];
+    // run records of one right-hand side's operator (FP32 for precision 1)
+    v[18] = B.R == 1 ? (double)runs_read(c, B.prec == 1) : 0;
+    for (int i = 0; i < n && i < 19; ++i) out[i] = v[i];
 }
 
 }  // namespace madam

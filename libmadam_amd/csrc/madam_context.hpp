@@ -204,8 +204,8 @@ struct Context {
         bool ok = false;
     } sr_s, sr_g;
     // run records of the one-right-hand-side projections (madam_runs.hip):
-    // mean_run is the estimated samples per run, runs_ok whether the records
-    // of this pointing exist (word and FP64 sums; the FP32 sums on demand)
+    // mean_run is the estimated samples per run, runs_ok / runs32_ok whether
+    // the records of this pointing exist with FP64 / FP32 weight sums
     double mean_run = 0;
     bool runs_ok = false;
     int run_sh = 0;
@@ -340,6 +340,8 @@ void cg_apply(Context &c, const double *r, double *z);
 // the FP32 weight sums of the run records, before FP32 projections (allocates:
 // call outside graph capture)
 void runs_prepare_fp32(Context &c);
+// runs that the baseline side reads in FP64 / FP32 (0: it reads samples)
+int64_t runs_read(const Context &c, bool fp32);
 template <typename T>
 void project_to_map(Context &c, const T *pw, const T *cc_c, T *m4);
 template <typename T>

@@ -814,15 +814,17 @@ static bool runs_wanted(const Context &c)
     return c.mean_run >= (sizeof(T) == 8 ? 2.0 : 1.3);
 }
 
-// run records of both projections, and the pixel side's segment tables over them
-static void build_runs(Context &c)
+// run records of both projections with weight sums of type W, and the pixel
+// side's segment tables over them; false where the word cannot hold the indices
+template <typename W>
+static bool build_runs(Context &c, DBuf<W> &gw, DBuf<W> &sw)
 {
     hipStream_t s = c.stream;
     int dsh = 0;
     while ((1ll << dsh) < c.ndeg) ++dsh;
     int sh = 1;
     while ((1ll << sh) < std::max(c.npix_cross, c.nbtot)) ++sh;
-    if (sh > 28) return;
+    if (sh > 28) return false;
     uint32_t maxrun = (1u << (32 - sh)) - 1u;
     int64_t n = (int64_t)c.ndet * c.nsamp, nent = c.nactive, nmax = std::max(n, nent);
     DBuf<uint32_t> mask;
@@ -847,8 +849,8 @@ static void build_runs(Context &c)
               offs.p, tmp.p);
     c.n_rung = total(n);
     c.d_rung.alloc(c.n_rung);
-    if (pol) c.d_rungw.alloc(c.n_rung);
-    runs_write(s, c.d_pixc.p, c.rec_layout, n, dsh, sh, words.p, offs.p, c.d_rung.p, pol ? c.d_rungw.p : nullptr);
+    if (pol) gw.alloc(c.n_rung);
+    runs_write<W>(s, c.d_pixc.p, c.rec_layout, n, dsh, sh, words.p, offs.p, c.d_rung.p, gw.p);
     c.d_rungst.alloc((size_t)c.ndet * (c.nbase + 1));
     runs_base_starts(s, c.d_bstart.p, c.nbase, c.ndet, c.nsamp, words.p, offs.p, c.d_rungst.p);
     // pixel side: the CSR entries
@@ -856,23 +858,26 @@ static void build_runs(Context &c)
               offs.p, tmp.p);
     c.n_runs = total(nent);
     c.d_runs.alloc(c.n_runs);
-    if (pol) c.d_runsw.alloc(c.n_runs);
-    runs_write(s, c.d_entc.p, c.rec_layout, nent, 0, sh, words.p, offs.p, c.d_runs.p, pol ? c.d_runsw.p : nullptr);
+    if (pol) sw.alloc(c.n_runs);
+    runs_write<W>(s, c.d_entc.p, c.rec_layout, nent, 0, sh, words.p, offs.p, c.d_runs.p, sw.p);
     seg.alloc(c.nzpix + 1);
     runs_pixel_starts(s, c.d_segstart_s.p, c.nzpix, words.p, offs.p, seg.p);
     segtiles_alloc(c.sr_r, c.n_runs);
     segred_build(s, seg.p, c.nzpix, c.n_runs, c.sr_r.heads.p, c.sr_r.k0.p, c.sr_r.fix_end.p, c.sr_r.fix_ord.p);
     MADAM_CHECK(hipStreamSynchronize(s));
     c.run_sh = sh;
-    c.runs_ok = true;
-    c.stats[ST_RUN_RECORDS] = (double)c.n_rung;
+    return true;
 }
 
+// Below two samples per run the FP64 operator reads samples, and the records
+// hold FP32 sums alone.
 void runs_prepare_fp32(Context &c)
 {
     if (!runs_wanted<float>(c) || c.runs32_ok) return;
-    if (!c.runs_ok) build_runs(c);
-    if (!c.runs_ok) return;
+    if (!c.runs_ok) {
+        c.runs32_ok = build_runs(c, c.d_rungw32, c.d_runsw32);
+        return;
+    }
     if (c.nmap == 3) {
         c.d_rungw32.alloc(c.n_rung);
         c.d_runsw32.alloc(c.n_runs);
@@ -880,6 +885,19 @@ void runs_prepare_fp32(Context &c)
         runs_cast(c.stream, c.d_runsw.p, c.d_runsw32.p, c.n_runs);
     }
     c.runs32_ok = true;
+}
+
+static void release_runs(Context &c)
+{
+    c.runs_ok = c.runs32_ok = false;
+    c.d_rung.release();
+    c.d_runs.release();
+    c.d_rungw.release();
+    c.d_runsw.release();
+    c.d_rungw32.release();
+    c.d_runsw32.release();
+    c.d_rungst.release();
+    c.sr_r = Context::SegTiles();
 }
 
 template <typename T>
@@ -905,6 +923,11 @@ template <typename T>
 static bool use_runs(const Context &c)
 {
     return (sizeof(T) == 8 ? c.runs_ok : c.runs32_ok) && runs_wanted<T>(c);
+}
+
+int64_t runs_read(const Context &c, bool fp32)
+{
+    return (fp32 ? use_runs<float>(c) : use_runs<double>(c)) ? c.n_rung : 0;
 }
 
 template <typename T>
@@ -986,7 +1009,14 @@ static void build_segtiles(Context &c)
     }
     int64_t nt = std::max(segred_ntiles(c.nactive), segred_ntiles((int64_t)c.ndet * c.nsamp));
     c.d_sr_part.alloc(2 * (nt > 0 ? nt : 1));
-    if (runs_wanted<double>(c)) build_runs(c);
+    // (buffers of the pointing before are kept only where this one's solves can use them)
+    if (runs_wanted<double>(c)) {
+        c.runs_ok = build_runs(c, c.d_rungw, c.d_runsw);
+    } else {
+        c.d_rungw.release();
+        c.d_runsw.release();
+        if (!runs_wanted<float>(c)) release_runs(c);
+    }
 }
 
 
@@ -1618,6 +1648,7 @@ void solve_setup(Context &c, const TT *tod)
         c.stats[ST_T_PRECOND] = now() - tp;
         c.stats[ST_PRECOND_KIND] = c.precond_kind;
         c.stats[ST_NOF] = (double)c.nof;
+        c.stats[ST_RUN_RECORDS] = (double)runs_read(c, false);
     }
 }
 

@@ -349,9 +349,10 @@ int64_t runs_spans(int64_t n);
 void runs_mark(hipStream_t s, const void *rec, int rl, int64_t n, int64_t period, int dsh, uint32_t maxrun,
                const int64_t *starts, int64_t nstarts, uint32_t *mask, unsigned long long *words, int32_t *counts,
                int64_t *offs, int64_t *scan_tmp);
-// the runs' words and (REC12) weight sums
+// the runs' words and (REC12) weight sums (W: double2 or float2)
+template <typename W>
 void runs_write(hipStream_t s, const void *rec, int rl, int64_t n, int dsh, int sh, const unsigned long long *words,
-                const int64_t *offs, uint32_t *out, double2 *w64);
+                const int64_t *offs, uint32_t *out, W *wsum);
 // first run of every baseline gst[ndet][nbase + 1], of every pixel seg[nz + 1]
 void runs_base_starts(hipStream_t s, const int64_t *bstart, int64_t nbase, int ndet, int64_t nsamp,
                       const unsigned long long *words, const int64_t *offs, int64_t *gst);

@@ -72,11 +72,12 @@ __global__ void __launch_bounds__(RUN_TPB) k_run_flags(const void *rec, int64_t 
     if (lane == 0) counts[w] = cnt;
 }
 
-// the runs: word and FP64 weight sums (w64 null: no weights)
-template <int RL>
+// the runs: word and weight sums, added in FP64 and stored as W (double2, or
+// float2 where only the FP32 operator reads them)
+template <int RL, typename W>
 __global__ void __launch_bounds__(RUN_TPB) k_run_write(const void *rec, int64_t n, int dsh, int sh,
                                                        const unsigned long long *words, const int64_t *offs,
-                                                       uint32_t *out, double2 *w64)
+                                                       uint32_t *out, W *wsum)
 {
     int lane = threadIdx.x & 63;
     int64_t w = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
@@ -101,7 +102,12 @@ __global__ void __launch_bounds__(RUN_TPB) k_run_write(const void *rec, int64_t 
             }
             int64_t o = at + __popcll(b & ((1ull << lane) - 1ull));
             out[o] = q | (m << sh);
-            if (RL == REC12) w64[o] = s;
+            if (RL == REC12) {
+                W v;
+                v.x = (decltype(v.x))s.x;
+                v.y = (decltype(v.y))s.y;
+                wsum[o] = v;
+            }
         }
         at += __popcll(b);
     }
@@ -169,14 +175,19 @@ void runs_mark(hipStream_t s, const void *rec, int rl, int64_t n, int64_t period
     MADAM_CHECK(hipGetLastError());
 }
 
+template <typename W>
 void runs_write(hipStream_t s, const void *rec, int rl, int64_t n, int dsh, int sh, const unsigned long long *words,
-                const int64_t *offs, uint32_t *out, double2 *w64)
+                const int64_t *offs, uint32_t *out, W *wsum)
 {
     unsigned g = run_grid(runs_spans(n) * 64, INT32_MAX);
-    if (rl == REC12) k_run_write<REC12><<<g, RUN_TPB, 0, s>>>(rec, n, dsh, sh, words, offs, out, w64);
-    else k_run_write<REC4><<<g, RUN_TPB, 0, s>>>(rec, n, dsh, sh, words, offs, out, w64);
+    if (rl == REC12) k_run_write<REC12, W><<<g, RUN_TPB, 0, s>>>(rec, n, dsh, sh, words, offs, out, wsum);
+    else k_run_write<REC4, W><<<g, RUN_TPB, 0, s>>>(rec, n, dsh, sh, words, offs, out, wsum);
     MADAM_CHECK(hipGetLastError());
 }
+template void runs_write<double2>(hipStream_t, const void *, int, int64_t, int, int, const unsigned long long *,
+                                  const int64_t *, uint32_t *, double2 *);
+template void runs_write<float2>(hipStream_t, const void *, int, int64_t, int, int, const unsigned long long *,
+                                 const int64_t *, uint32_t *, float2 *);
 
 void runs_base_starts(hipStream_t s, const int64_t *bstart, int64_t nbase, int ndet, int64_t nsamp,
                       const unsigned long long *words, const int64_t *offs, int64_t *gst)

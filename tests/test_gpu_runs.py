@@ -105,3 +105,44 @@ def test_mixed_solve_from_runs():
     res = r["yba"].reshape(-1) - m.apply(2, r["aa"])
     m.close()
     assert np.linalg.norm(res) <= 1.01e-10 * np.linalg.norm(r["yba"])
+
+
+@pytest.mark.parametrize("nnz", [3, 1])
+def test_runs_that_only_fp32_reads(nnz):
+    """Between 1.3 and 2 samples per run the FP64 operator reads samples and a mixed solve's FP32 operator
+    runs: the records hold FP32 sums alone (12 bytes a run and side, not 28), each precision reports what it
+    reads, and the solution meets the limit on the FP64 residual in as many steps as from samples."""
+    import torch
+    import libmadam_amd
+    scan = dict(fsample=100.0, spin_period=7.5, prec_period=4000.0, opening_turns=85.0 / 360.0, lon0_turns=0.0)
+    m, steps = None, {}
+    for nsamp in (2 ** 20, 2 ** 16 - 1):     # the shorter scan is below the 2^18 samples from which runs are used
+        c = mc.ring_case(ndet=4, nsamp=nsamp, nside=64, base_first=1.0, nnz=nnz, seed=nnz, fsample=100.0,
+                         pointing=lambda d, n: oracle.expand_pointing(scan, dict(psi_turns=0.125 * d), 64, 0, n),
+                         extra_pars=dict(cglimit=1e-14))
+        for variant in ((0,) if nsamp > 2 ** 18 else (0, 128)):
+            m = libmadam_amd.Madam(0)
+            args = mc.call_args(c)
+            m.configure(*args[:4], *args[7:], c["nnz"])
+            m.set_kernel_variant(variant)
+            m.set_pointing(c["pixels"], c["pixweights"])
+            m.solve(c["signal"].copy())
+            assert m.stats()["run_records"] == 0
+            free = torch.cuda.mem_get_info()[0]
+            m.solve_batch(c["signal"].reshape(1, 4, -1), precision=1)
+            r = m.batch_result(0)
+            used = free - torch.cuda.mem_get_info()[0]
+            runs = r["info"]["run_records"]
+            assert m.stats()["run_records"] == 0
+            if nsamp < 2 ** 18 and variant == 0:
+                assert runs == 0
+            else:
+                assert 1.3 <= m.stats()["nactive"] / runs < 2.0
+            if nsamp > 2 ** 18:
+                # both sides' records and segment tables, and the batch's own vectors and maps (under 40 MB)
+                assert used <= 30 * runs + 40e6
+            res = r["yba"].reshape(-1) - m.apply(2, r["aa"])
+            assert np.linalg.norm(res) <= 1.01e-7 * np.linalg.norm(r["yba"])
+            steps[nsamp, variant] = r["info"]["pcg_steps"]
+            m.close()
+    assert abs(steps[2 ** 16 - 1, 0] - steps[2 ** 16 - 1, 128]) <= 0.1 * steps[2 ** 16 - 1, 0] + 2
