@@ -135,10 +135,12 @@ int madam_get_filter(void *ctx, int ipsd, double *fcov);
  * side and LDS tiles on the baseline side (default), 1 = wave per pixel / lane
  * group per baseline, 2 = LDS tiles on both sides, 3 = segmented tiles on both
  * sides; + 16 = band factorization computes every row in one chain (no periodic
- * continuation of repeating 64-row blocks, no pieces); + 32 / + 64 = band carry chains
- * always / never several per wave (default: several when there are enough
- * of them), + 128 (before the first solve on a pointing) = run records of the
- * projections whatever the number of samples */
+ * continuation of repeating 64-row blocks, no pieces); + 32 / + 64 = the
+ * chained band solve in place of the one-pass one, its carry chains always /
+ * never several per wave (default: one pass where the carries decay fast
+ * enough, else chains, several per wave when there are enough of them); + 128
+ * (before the first solve on a pointing) = run records of the projections
+ * whatever the number of samples */
 int madam_set_kernel_variant(void *ctx, int variant);
 /* pointing expansion of the synthetic ring scan: scan5 = {fsample, spin_period,
  * prec_period, opening_turns, lon0_turns}, dets3[ndet][3] = {psi_turns,

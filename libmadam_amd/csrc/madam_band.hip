@@ -1481,7 +1481,7 @@ static void band_build_direct(hipStream_t s, const BandPrec &bp, BandImpl *im, c
 // Returns 0 on success; fills info_out[s] (0 ok, >0 failing column) for each segment.
 int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *dseg, int64_t nseg,
                     const int *nband_seg_host, const double *invcov_dev, int64_t nof, const double *nna,
-                    int *info_out, bool periodic)
+                    int *info_out, bool periodic, bool direct)
 {
     int kdmax = 0;
     for (int64_t i = 0; i < nseg; ++i)
@@ -1733,15 +1733,29 @@ int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *
         MADAM_CHECK(hipMemcpyAsync(im->cmap, cmap.data(), sizeof(int32_t) * cmap.size(), hipMemcpyHostToDevice, s));
         MADAM_CHECK(hipMemcpyAsync(im->bmap, bmap.data(), sizeof(int32_t) * bmap.size(), hipMemcpyHostToDevice, s));
         MADAM_CHECK(hipStreamSynchronize(s));   // the host tables above
-        band_build_direct(s, bp, im, first, cmap);
+        if (direct) band_build_direct(s, bp, im, first, cmap);
     }
     bp.impl = im;
     MADAM_CHECK(hipStreamSynchronize(s));
     return 0;
 }
 
-// tables of the one-pass solve; leaves im->direct false where the carry
-// decays too slowly for it
+// the tables of the one-pass solve go
+static void band_drop_direct(BandImpl *im)
+{
+    im->direct = false;
+    for (double **p : {&im->Pf, &im->Pb, &im->PU, &im->LuD}) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+    }
+    if (im->blk) (void)hipFree(im->blk);
+    if (im->pslot) (void)hipFree(im->pslot);
+    im->blk = nullptr;
+    im->pslot = nullptr;
+}
+
+// tables of the one-pass solve (3.9 KB per 64 rows where the factor does not
+// repeat); none, and im->direct false, where the carry decays too slowly for it
 static void band_build_direct(hipStream_t s, const BandPrec &bp, BandImpl *im, const std::vector<int64_t> &first,
                               const std::vector<int32_t> &cmap)
 {
@@ -1784,18 +1798,15 @@ static void band_build_direct(hipStream_t s, const BandPrec &bp, BandImpl *im, c
     const int64_t ns = (int64_t)list.size(), nu = (int64_t)urep.size(), np = BD_LEV * BD_KK;
     im->nblk = (int64_t)blk.size();
     im->nslot = ns;
-    int32_t *dlist = nullptr, *durep = nullptr;
+    int32_t *dlist = nullptr;
     uint8_t *dpure = nullptr;
     unsigned long long *dworst = nullptr, worst = 0;
     MADAM_CHECK(hipMalloc(&im->blk, sizeof(BandBlk) * blk.size()));
     MADAM_CHECK(hipMalloc(&im->pslot, sizeof(int32_t) * nch));
     MADAM_CHECK(hipMalloc(&im->Pf, sizeof(double) * np * ns));
     MADAM_CHECK(hipMalloc(&im->Pb, sizeof(double) * np * ns));
-    MADAM_CHECK(hipMalloc(&im->PU, sizeof(double) * 2 * np * std::max<int64_t>(nu, 1)));
-    MADAM_CHECK(hipMalloc(&im->LuD, sizeof(double) * BAND_CH * BD_K * std::max<int64_t>(nu, 1)));
     MADAM_CHECK(hipMalloc(&dlist, sizeof(int32_t) * ns));
     MADAM_CHECK(hipMalloc(&dpure, ns));
-    MADAM_CHECK(hipMalloc(&durep, sizeof(int32_t) * std::max<int64_t>(nu, 1)));
     MADAM_CHECK(hipMalloc(&dworst, sizeof(unsigned long long)));
     MADAM_CHECK(hipMemsetAsync(dworst, 0, sizeof(unsigned long long), s));
     MADAM_CHECK(hipMemcpyAsync(im->blk, blk.data(), sizeof(BandBlk) * blk.size(), hipMemcpyHostToDevice, s));
@@ -1807,8 +1818,26 @@ static void band_build_direct(hipStream_t s, const BandPrec &bp, BandImpl *im, c
     k_band_products<<<g, 64, 0, s>>>(dlist, dpure, ns, im->ch, bp.Tb, 1, im->Pb, ns, 1);
     k_band_decay<<<gc, 64, 0, s>>>(im->pslot, nch, im->ch, im->Pf, ns, 0, dworst);
     k_band_decay<<<gc, 64, 0, s>>>(im->pslot, nch, im->ch, im->Pb, ns, 1, dworst);
+    MADAM_CHECK(hipGetLastError());
+    MADAM_CHECK(hipMemcpyAsync(&worst, dworst, sizeof(worst), hipMemcpyDeviceToHost, s));
+    MADAM_CHECK(hipStreamSynchronize(s));
+    (void)hipFree(dlist);
+    (void)hipFree(dpure);
+    (void)hipFree(dworst);
+    double w;
+    static_assert(sizeof w == sizeof worst, "");
+    memcpy(&w, &worst, sizeof w);
+    if (!(w < BD_NEGLIGIBLE)) {
+        band_drop_direct(im);
+        return;
+    }
+    MADAM_CHECK(hipMalloc(&im->PU, sizeof(double) * 2 * np * std::max<int64_t>(nu, 1)));
+    MADAM_CHECK(hipMalloc(&im->LuD, sizeof(double) * BAND_CH * BD_K * std::max<int64_t>(nu, 1)));
     if (nu > 0) {
         std::vector<uint8_t> one(nu, 1);
+        int32_t *durep = nullptr;
+        MADAM_CHECK(hipMalloc(&durep, sizeof(int32_t) * nu));
+        MADAM_CHECK(hipMalloc(&dpure, nu));
         MADAM_CHECK(hipMemcpyAsync(durep, urep.data(), sizeof(int32_t) * nu, hipMemcpyHostToDevice, s));
         MADAM_CHECK(hipMemcpyAsync(dpure, one.data(), nu, hipMemcpyHostToDevice, s));
         unsigned gu = (unsigned)((nu * BD_KD + 63) / 64);
@@ -1818,18 +1847,10 @@ static void band_build_direct(hipStream_t s, const BandPrec &bp, BandImpl *im, c
             im->Li, durep, nu, im->LuD);
         MADAM_CHECK(hipGetLastError());
         MADAM_CHECK(hipStreamSynchronize(s));   // one
+        (void)hipFree(durep);
+        (void)hipFree(dpure);
     }
-    MADAM_CHECK(hipGetLastError());
-    MADAM_CHECK(hipMemcpyAsync(&worst, dworst, sizeof(worst), hipMemcpyDeviceToHost, s));
-    MADAM_CHECK(hipStreamSynchronize(s));
-    (void)hipFree(dlist);
-    (void)hipFree(dpure);
-    (void)hipFree(durep);
-    (void)hipFree(dworst);
-    double w;
-    static_assert(sizeof w == sizeof worst, "");
-    memcpy(&w, &worst, sizeof w);
-    im->direct = w < BD_NEGLIGIBLE;
+    im->direct = true;
 }
 
 int band_capacity(const BandPrec &bp) { return bp.impl ? ((const BandImpl *)bp.impl)->rcap : 0; }
@@ -1931,10 +1952,7 @@ void band_free(BandPrec &bp)
         (void)hipFree(im->Gb);
         (void)hipFree(im->cg);
         (void)hipFree(im->Sg);
-        for (double *p : {im->Pf, im->Pb, im->PU, im->LuD})
-            if (p) (void)hipFree(p);
-        if (im->blk) (void)hipFree(im->blk);
-        if (im->pslot) (void)hipFree(im->pslot);
+        band_drop_direct(im);
         delete im;
     }
     if (bp.L) (void)hipFree(bp.L);

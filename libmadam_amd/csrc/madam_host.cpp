@@ -1270,7 +1270,7 @@ static void build_preconditioner(Context &c)
     for (;;) {
         std::vector<int> info(c.segp.size(), 0);
         if (band_build(s, c.band, c.segp.data(), c.d_segp.p, (int64_t)c.segp.size(), nband.data(), c.d_invcov.p, c.nof,
-                       c.d_nna.p, info.data(), !(c.kernel_variant & 16)) != 0)
+                       c.d_nna.p, info.data(), !(c.kernel_variant & 16), band_chain_pack(c.kernel_variant) < 0) != 0)
             fail("band preconditioner wider than %d baselines reached the factor kernels", BAND_WIDTH_GPU);
         c.band_ready = true;
         bool retry = false;

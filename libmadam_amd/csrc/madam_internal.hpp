@@ -436,7 +436,7 @@ inline int band_chain_pack(int kernel_variant)
 
 int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *dseg, int64_t nseg,
                const int *nband_seg_host, const double *invcov_dev, int64_t nof, const double *nna, int *info_out,
-               bool periodic = true);
+               bool periodic, bool direct);   // direct: the one-pass solve's tables too, where it can be used
 // z = M^-1 r for nrhs right-hand sides at a stride of vstride elements (T =
 // float or double; the factor and the solves are FP64)
 template <typename T>

@@ -90,3 +90,41 @@ def test_direct_batch_and_mixed():
             a = m.batch_result(r)["aa"]
             assert np.linalg.norm((a - a.mean()) - (one[r] - one[r].mean())) <= tol * np.linalg.norm(one[r])
     m.close()
+
+
+def test_tables_only_where_they_are_read():
+    """The products of the one-pass solve (3.9 KB per 64 flagged rows) are held where it is used: not with the
+    chains forced, nor where a low knee makes the carries decay too slowly, whose results are then the chains'."""
+    import torch
+    import libmadam_amd
+    nside, fs, ndet, nper = 8, 50.0, 2, 300000
+    scan = dict(fsample=fs, spin_period=2.0, prec_period=400.0, opening_turns=85.0 / 360.0, lon0_turns=0.0)
+
+    def pointing(d, n):
+        return oracle.expand_pointing(scan, dict(psi_turns=0.25 * d), nside, 0, n)
+
+    c = mc.ring_case(ndet=ndet, nsamp=nper * 4, nside=nside, base_first=0.08, prior=True, seed=3, pointing=pointing,
+                     nnz=1, extra_pars=dict(iter_max=5))
+    c["pixels"][np.random.default_rng(1).random(c["pixels"].size) < 0.1] = -1
+    white = c["psdvals"][-1]
+    used, z = {}, {}
+    for again in range(2):                      # the first time round the runtime allocates for itself
+        for knee in (0.1, 0.002):
+            c["psdvals"] = np.tile(white * (1.0 + (c["psdfreqs"] / knee) ** -1.5), ndet)
+            for variant in (0, 64):
+                m = libmadam_amd.Madam(0)
+                args = mc.call_args(c)
+                m.configure(*args[:4], *args[7:], c["nnz"])
+                m.set_kernel_variant(variant)
+                m.set_pointing(c["pixels"].copy(), c["pixweights"])
+                free = torch.cuda.mem_get_info()[0]
+                m.solve(c["signal"].copy())
+                used[knee, variant] = free - torch.cuda.mem_get_info()[0]
+                assert m.stats()["precond_kind"] == 3 and m.stats()["nband"] == 10 and m.stats()["ncg"] == 0
+                z[knee, variant] = m.apply(1, np.random.default_rng(5).standard_normal(ndet * nper))
+                m.close()
+    tables = 2 * 8 * 3 * 81 * (ndet * nper // 64)
+    assert used[0.1, 0] - used[0.1, 64] >= 0.9 * tables
+    assert used[0.002, 0] - used[0.1, 64] <= 0.1 * tables
+    assert not np.array_equal(z[0.1, 0], z[0.1, 64])
+    np.testing.assert_array_equal(z[0.002, 0], z[0.002, 64])
