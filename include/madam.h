@@ -142,6 +142,10 @@ int madam_get_filter(void *ctx, int ipsd, double *fcov);
  * (before the first solve on a pointing) = run records of the projections
  * whatever the number of samples */
 int madam_set_kernel_variant(void *ctx, int variant);
+/* for tests of memory shortage: the calling thread's device allocations first
+ * .. first + n - 1, counted from this call on, fail as out of memory (first < 0:
+ * none); returns the number it made since the last call */
+long madam_fail_allocations(long first, long n);
 /* pointing expansion of the synthetic ring scan: scan5 = {fsample, spin_period,
  * prec_period, opening_turns, lon0_turns}, dets3[ndet][3] = {psi_turns,
  * open_offset_turns, spin_offset_turns}; outputs pix[ndet][n], weights[ndet][n][3] */

@@ -110,6 +110,8 @@ def lib():
         L.madam_last_status.restype = i32
         L.madam_cache_handle.restype = i32
         L.madam_cache_handle.argtypes = [ct.POINTER(vp)]
+        L.madam_fail_allocations.restype = lg
+        L.madam_fail_allocations.argtypes = [lg, lg]
         L.destripe.restype = None
         L.destripe_with_cache.restype = None
         L.clear_caches.restype = None

@@ -26,6 +26,7 @@
 #include <cstring>
 #include <vector>
 
+#include "madam_context.hpp"
 #include "madam_internal.hpp"
 
 namespace madam {
@@ -1475,13 +1476,26 @@ static int kd_class(int kd)
     default: { constexpr int KD = 49; STMT; } break;      \
     }
 
+// frees the one-pass solve's tables
+static void band_drop_direct(BandImpl *im)
+{
+    im->direct = false;
+    for (double **p : {&im->Pf, &im->Pb, &im->PU, &im->LuD}) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+    }
+    if (im->blk) (void)hipFree(im->blk);
+    if (im->pslot) (void)hipFree(im->pslot);
+    im->blk = nullptr;
+    im->pslot = nullptr;
+}
+
 static void band_build_direct(hipStream_t s, const BandPrec &bp, BandImpl *im, const std::vector<int64_t> &first,
                               const std::vector<int32_t> &cmap);
 
-// Returns 0 on success; fills info_out[s] (0 ok, >0 failing column) for each segment.
-int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *dseg, int64_t nseg,
+static int band_tables(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *dseg, int64_t nseg,
                     const int *nband_seg_host, const double *invcov_dev, int64_t nof, const double *nna,
-                    int *info_out, bool periodic, bool direct)
+                    int *info_out, bool periodic, bool pieces, bool direct)
 {
     int kdmax = 0;
     for (int64_t i = 0; i < nseg; ++i)
@@ -1495,12 +1509,12 @@ int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *
     // storage for the factor over every baseline row of every segment
     int64_t rows_max = 0;
     for (int64_t i = 0; i < nseg; ++i) rows_max = std::max<int64_t>(rows_max, hseg[i].b0 + hseg[i].noba);
-    MADAM_CHECK(hipMalloc(&bp.L, sizeof(double) * (rows_max > 0 ? rows_max : 1) * K));
-    int *dnb = nullptr, *dinfo = nullptr;
-    MADAM_CHECK(hipMalloc(&dnb, sizeof(int) * (nseg > 0 ? nseg : 1)));
-    MADAM_CHECK(hipMalloc(&dinfo, sizeof(int) * (nseg > 0 ? nseg : 1)));
-    MADAM_CHECK(hipMemcpyAsync(dnb, nband_seg_host, sizeof(int) * nseg, hipMemcpyHostToDevice, s));
-    MADAM_CHECK(hipMemsetAsync(dinfo, 0, sizeof(int) * (nseg > 0 ? nseg : 1), s));
+    MADAM_CHECK(device_malloc(&bp.L, sizeof(double) * (rows_max > 0 ? rows_max : 1) * K));
+    DBuf<int> dnb, dinfo;
+    dnb.alloc(nseg);
+    dinfo.alloc(nseg);
+    MADAM_CHECK(hipMemcpyAsync(dnb.p, nband_seg_host, sizeof(int) * nseg, hipMemcpyHostToDevice, s));
+    MADAM_CHECK(hipMemsetAsync(dinfo.p, 0, sizeof(int) * (nseg > 0 ? nseg : 1), s));
     // A repeating factor is a few hundred columns after every change of nna and
     // copies (k_band_factor_w); where that comes to more than BP_SERIAL columns
     // in a segment the factor is made in pieces (8 detectors x 2^23 flagged
@@ -1514,73 +1528,76 @@ int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *
         longest = std::max<int64_t>(longest, hseg[i].noba);
         pfirst[i + 1] = pfirst[i] + (hseg[i].noba + BP_ROWS - 1) / BP_ROWS;
     }
-    bool pieces = false;
-    unsigned long long *dcnt = nullptr;   // nna changes per segment
-    MADAM_CHECK(hipMalloc(&dcnt, sizeof(unsigned long long) * ns1));
-    MADAM_CHECK(hipMemsetAsync(dcnt, 0, sizeof(unsigned long long) * ns1, s));
-    if (periodic && longest > BP_SERIAL && nseg <= 65535) {
+    DBuf<unsigned long long> dcnt;   // nna changes per segment
+    dcnt.alloc(ns1);
+    MADAM_CHECK(hipMemsetAsync(dcnt.p, 0, sizeof(unsigned long long) * ns1, s));
+    bool may = pieces && periodic && longest > BP_SERIAL && nseg <= 65535;
+    pieces = false;
+    if (may) {
         k_band_nna_changes<<<dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(64, 8192 / nseg)), (unsigned)nseg), 256,
-                             0, s>>>(dseg, nseg, nna, dcnt);
+                             0, s>>>(dseg, nseg, nna, dcnt.p);
         std::vector<unsigned long long> ch(nseg);
-        MADAM_CHECK(hipMemcpyAsync(ch.data(), dcnt, sizeof(ch[0]) * nseg, hipMemcpyDeviceToHost, s));
+        MADAM_CHECK(hipMemcpyAsync(ch.data(), dcnt.p, sizeof(ch[0]) * nseg, hipMemcpyDeviceToHost, s));
         MADAM_CHECK(hipStreamSynchronize(s));
         for (int64_t i = 0; i < nseg; ++i)
             pieces = pieces || std::min<int64_t>(hseg[i].noba, (int64_t)ch[i] * PER_CHANGE) > BP_SERIAL;
     }
     bp.nrows_factored = 0;
+    DBuf<int64_t> dpf;
+    DBuf<double> win;
+    DBuf<int> bad;
+    const int64_t npc = pfirst[nseg];
+    pieces = pieces && if_room([&] {
+        dpf.alloc(nseg + 1);
+        win.alloc((size_t)2 * K * K * npc);
+        bad.alloc(npc);
+    });
     if (pieces) {
-        int64_t *dpf = nullptr;
-        double *win = nullptr;
-        int *bad = nullptr;
-        const int64_t npc = pfirst[nseg];
-        MADAM_CHECK(hipMalloc(&dpf, sizeof(int64_t) * (nseg + 1)));
-        MADAM_CHECK(hipMalloc(&win, sizeof(double) * 2 * K * K * npc));
-        MADAM_CHECK(hipMalloc(&bad, sizeof(int) * npc));
-        MADAM_CHECK(hipMemcpyAsync(dpf, pfirst.data(), sizeof(int64_t) * (nseg + 1), hipMemcpyHostToDevice, s));
+        MADAM_CHECK(hipMemcpyAsync(dpf.p, pfirst.data(), sizeof(int64_t) * (nseg + 1), hipMemcpyHostToDevice, s));
         BAND_DISPATCH(KD, ({
-            k_band_factor_pieces<KD><<<(unsigned)npc, 64, 0, s>>>(dseg, nseg, dnb, dpf, invcov_dev, nof, nna, bp.L, win,
-                                                                  bad);
-            k_band_factor_check<KD><<<(unsigned)nseg, 64, 0, s>>>(dseg, nseg, dnb, dpf, invcov_dev, nof, nna, bp.L, win,
-                                                                  bad, dinfo);
+            k_band_factor_pieces<KD><<<(unsigned)npc, 64, 0, s>>>(dseg, nseg, dnb.p, dpf.p, invcov_dev, nof, nna, bp.L,
+                                                                  win.p, bad.p);
+            k_band_factor_check<KD><<<(unsigned)nseg, 64, 0, s>>>(dseg, nseg, dnb.p, dpf.p, invcov_dev, nof, nna, bp.L,
+                                                                  win.p, bad.p, dinfo.p);
         }));
         MADAM_CHECK(hipGetLastError());
-        MADAM_CHECK(hipMemcpyAsync(info_out, dinfo, sizeof(int) * nseg, hipMemcpyDeviceToHost, s));
+        MADAM_CHECK(hipMemcpyAsync(info_out, dinfo.p, sizeof(int) * nseg, hipMemcpyDeviceToHost, s));
         MADAM_CHECK(hipStreamSynchronize(s));
-        (void)hipFree(dpf);
-        (void)hipFree(win);
-        (void)hipFree(bad);
         for (int64_t i = 0; i < nseg; ++i)
             if (!hseg[i].skip && nband_seg_host[i] > 0) bp.nrows_factored += hseg[i].noba;
     } else {
-        int64_t *dper = nullptr;   // per_src[nseg][BAND_MAXJ], per_q[nseg][BAND_MAXJ]
+        DBuf<int64_t> dper;   // per_src[nseg][BAND_MAXJ], per_q[nseg][BAND_MAXJ]
         int64_t nj = ns1 * BAND_MAXJ;
-        MADAM_CHECK(hipMalloc(&dper, sizeof(int64_t) * 2 * nj));
-        MADAM_CHECK(hipMemsetAsync(dper, 0, sizeof(int64_t) * 2 * nj, s));
+        dper.alloc(2 * nj);
+        MADAM_CHECK(hipMemsetAsync(dper.p, 0, sizeof(int64_t) * 2 * nj, s));
         if (nseg > 0) {
-            BAND_DISPATCH(KD, (k_band_factor_w<KD><<<(unsigned)nseg, 64, 0, s>>>(dseg, nseg, dnb, invcov_dev, nof, nna,
-                                                                                bp.L, dinfo, periodic ? dper : nullptr,
-                                                                                dper + nj)));
+            BAND_DISPATCH(KD, (k_band_factor_w<KD><<<(unsigned)nseg, 64, 0, s>>>(dseg, nseg, dnb.p, invcov_dev, nof,
+                                                                                nna, bp.L, dinfo.p,
+                                                                                periodic ? dper.p : nullptr,
+                                                                                dper.p + nj)));
             if (periodic) {
                 unsigned gy = (unsigned)std::min<int64_t>(nseg, 65535);
                 unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>(256, 8192 / nseg));
-                k_band_fill_periodic<<<dim3(gx, gy), 256, 0, s>>>(dseg, nseg, K, dper, dper + nj, bp.L);
+                k_band_fill_periodic<<<dim3(gx, gy), 256, 0, s>>>(dseg, nseg, K, dper.p, dper.p + nj, bp.L);
             }
         }
         MADAM_CHECK(hipGetLastError());
-        MADAM_CHECK(hipMemcpyAsync(info_out, dinfo, sizeof(int) * nseg, hipMemcpyDeviceToHost, s));
+        MADAM_CHECK(hipMemcpyAsync(info_out, dinfo.p, sizeof(int) * nseg, hipMemcpyDeviceToHost, s));
         std::vector<int64_t> perq(nj, 0);
-        MADAM_CHECK(hipMemcpyAsync(perq.data(), dper + nj, sizeof(int64_t) * nj, hipMemcpyDeviceToHost, s));
+        MADAM_CHECK(hipMemcpyAsync(perq.data(), dper.p + nj, sizeof(int64_t) * nj, hipMemcpyDeviceToHost, s));
         MADAM_CHECK(hipStreamSynchronize(s));
-        (void)hipFree(dper);
         for (int64_t i = 0; i < nseg; ++i)
             if (!hseg[i].skip && nband_seg_host[i] > 0) {
                 bp.nrows_factored += hseg[i].noba;
                 for (int k = 0; k < BAND_MAXJ; ++k) bp.nrows_factored -= 64 * perq[i * BAND_MAXJ + k];
             }
     }
-    (void)hipFree(dnb);
-    (void)hipFree(dinfo);
-    (void)hipFree(dcnt);
+    dnb.release();
+    dinfo.release();
+    dcnt.release();
+    dpf.release();
+    win.release();
+    bad.release();
     // chunk table over the segments that factored
     std::vector<ChunkInfo> ch;
     std::vector<int64_t> first;
@@ -1603,6 +1620,7 @@ int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *
     bp.nrows = 0;
     for (const ChunkInfo &ci : ch) bp.nrows += ci.n;
     BandImpl *im = new BandImpl();
+    bp.impl = im;
     im->nseg_used = (int64_t)first.size() - 1;
     // groups of BAND_G chunks inside each segment
     std::vector<int64_t> gfirst, sgfirst;
@@ -1618,13 +1636,13 @@ int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *
     im->ngrp = (int64_t)gfirst.size();
     {
         int64_t ng = im->ngrp > 0 ? im->ngrp : 1;
-        MADAM_CHECK(hipMalloc(&im->gfirst, sizeof(int64_t) * ng));
-        MADAM_CHECK(hipMalloc(&im->gn, sizeof(int32_t) * ng));
-        MADAM_CHECK(hipMalloc(&im->sgfirst, sizeof(int64_t) * sgfirst.size()));
-        MADAM_CHECK(hipMalloc(&im->Gf, sizeof(double) * ng * KD * KD));
-        MADAM_CHECK(hipMalloc(&im->Gb, sizeof(double) * ng * KD * KD));
-        MADAM_CHECK(hipMalloc(&im->cg, sizeof(double) * ng * KD));
-        MADAM_CHECK(hipMalloc(&im->Sg, sizeof(double) * ng * KD));
+        MADAM_CHECK(device_malloc(&im->gfirst, sizeof(int64_t) * ng));
+        MADAM_CHECK(device_malloc(&im->gn, sizeof(int32_t) * ng));
+        MADAM_CHECK(device_malloc(&im->sgfirst, sizeof(int64_t) * sgfirst.size()));
+        MADAM_CHECK(device_malloc(&im->Gf, sizeof(double) * ng * KD * KD));
+        MADAM_CHECK(device_malloc(&im->Gb, sizeof(double) * ng * KD * KD));
+        MADAM_CHECK(device_malloc(&im->cg, sizeof(double) * ng * KD));
+        MADAM_CHECK(device_malloc(&im->Sg, sizeof(double) * ng * KD));
         if (im->ngrp > 0) {
             MADAM_CHECK(hipMemcpyAsync(im->gfirst, gfirst.data(), sizeof(int64_t) * gfirst.size(),
                                        hipMemcpyHostToDevice, s));
@@ -1634,20 +1652,20 @@ int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *
                                    hipMemcpyHostToDevice, s));
     }
     int64_t nc = bp.nchunk > 0 ? bp.nchunk : 1;
-    MADAM_CHECK(hipMalloc(&im->ch, sizeof(ChunkInfo) * nc));
-    MADAM_CHECK(hipMalloc(&im->seg_first, sizeof(int64_t) * first.size()));
-    MADAM_CHECK(hipMalloc(&bp.Tf, sizeof(double) * nc * KD * KD));
-    MADAM_CHECK(hipMalloc(&bp.Tb, sizeof(double) * nc * KD * KD));
-    MADAM_CHECK(hipMalloc(&im->s0f, sizeof(double) * nc * KD));
-    MADAM_CHECK(hipMalloc(&im->s0b, sizeof(double) * nc * KD));
-    MADAM_CHECK(hipMalloc(&im->sinf, sizeof(double) * nc * KD));
-    MADAM_CHECK(hipMalloc(&im->sinb, sizeof(double) * nc * KD));
+    MADAM_CHECK(device_malloc(&im->ch, sizeof(ChunkInfo) * nc));
+    MADAM_CHECK(device_malloc(&im->seg_first, sizeof(int64_t) * first.size()));
+    MADAM_CHECK(device_malloc(&bp.Tf, sizeof(double) * nc * KD * KD));
+    MADAM_CHECK(device_malloc(&bp.Tb, sizeof(double) * nc * KD * KD));
+    MADAM_CHECK(device_malloc(&im->s0f, sizeof(double) * nc * KD));
+    MADAM_CHECK(device_malloc(&im->s0b, sizeof(double) * nc * KD));
+    MADAM_CHECK(device_malloc(&im->sinf, sizeof(double) * nc * KD));
+    MADAM_CHECK(device_malloc(&im->sinb, sizeof(double) * nc * KD));
     if (bp.nchunk > 0)
         MADAM_CHECK(hipMemcpyAsync(im->ch, ch.data(), sizeof(ChunkInfo) * ch.size(), hipMemcpyHostToDevice, s));
     MADAM_CHECK(hipMemcpyAsync(im->seg_first, first.data(), sizeof(int64_t) * first.size(), hipMemcpyHostToDevice, s));
     if (bp.nchunk > 0) {
         im->NCP = (bp.nchunk + 63) / 64 * 64;
-        MADAM_CHECK(hipMalloc(&im->Li, sizeof(double) * im->NCP * BAND_CH * K));
+        MADAM_CHECK(device_malloc(&im->Li, sizeof(double) * im->NCP * BAND_CH * K));
         int64_t tot = im->NCP * BAND_CH * K;
         unsigned g = (unsigned)std::min<int64_t>((tot + 255) / 256, 65535 * 16);
         k_band_relayout<<<g, 256, 0, s>>>(im->ch, bp.nchunk, im->NCP, K, BAND_CH, bp.L, im->Li);
@@ -1667,15 +1685,15 @@ int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *
             MADAM_CHECK(hipGetLastError());
         }
         // runs of equal chunks and blocks
-        uint8_t *dceq = nullptr;
-        MADAM_CHECK(hipMalloc(&dceq, bp.nchunk));
+        DBuf<uint8_t> dceq;
+        dceq.alloc(bp.nchunk);
         k_band_chunk_eq<<<(unsigned)std::min<int64_t>((bp.nchunk + 255) / 256, 65535), 256, 0, s>>>(
-            im->ch, bp.nchunk, K, im->Li, dceq);
+            im->ch, bp.nchunk, K, im->Li, dceq.p);
         MADAM_CHECK(hipGetLastError());
         std::vector<uint8_t> ceq(bp.nchunk);
-        MADAM_CHECK(hipMemcpyAsync(ceq.data(), dceq, bp.nchunk, hipMemcpyDeviceToHost, s));
+        MADAM_CHECK(hipMemcpyAsync(ceq.data(), dceq.p, bp.nchunk, hipMemcpyDeviceToHost, s));
         MADAM_CHECK(hipStreamSynchronize(s));
-        (void)hipFree(dceq);
+        dceq.release();
         std::vector<int32_t> cmap(bp.nchunk), bmap(im->NCP / 64);
         for (int64_t c = 0; c < bp.nchunk; ++c) {
             cmap[c] = ceq[c] ? cmap[c - 1] : (int32_t)c;
@@ -1703,19 +1721,18 @@ int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *
             if (reps.empty() || reps.back() != wr) reps.push_back(wr);   // runs are contiguous
             uidx[w] = (int32_t)reps.size() - 1;
         }
-        MADAM_CHECK(hipMalloc(&im->uidx, sizeof(int32_t) * uidx.size()));
+        MADAM_CHECK(device_malloc(&im->uidx, sizeof(int32_t) * uidx.size()));
         MADAM_CHECK(hipMemcpyAsync(im->uidx, uidx.data(), sizeof(int32_t) * uidx.size(), hipMemcpyHostToDevice, s));
-        MADAM_CHECK(hipMalloc(&im->Lu, sizeof(double) * std::max<size_t>(reps.size(), 1) * BAND_CH * K));
+        MADAM_CHECK(device_malloc(&im->Lu, sizeof(double) * std::max<size_t>(reps.size(), 1) * BAND_CH * K));
         if (!reps.empty()) {
-            int32_t *dreps = nullptr;
-            MADAM_CHECK(hipMalloc(&dreps, sizeof(int32_t) * reps.size()));
-            MADAM_CHECK(hipMemcpyAsync(dreps, reps.data(), sizeof(int32_t) * reps.size(), hipMemcpyHostToDevice, s));
+            DBuf<int32_t> dreps;
+            dreps.alloc(reps.size());
+            MADAM_CHECK(hipMemcpyAsync(dreps.p, reps.data(), sizeof(int32_t) * reps.size(), hipMemcpyHostToDevice, s));
             int64_t tot = (int64_t)reps.size() * BAND_CH * K;
             k_band_compact_uniform<<<(unsigned)std::min<int64_t>((tot + 255) / 256, 65535), 256, 0, s>>>(
-                im->Li, K, dreps, (int64_t)reps.size(), im->Lu);
+                im->Li, K, dreps.p, (int64_t)reps.size(), im->Lu);
             MADAM_CHECK(hipGetLastError());
             MADAM_CHECK(hipStreamSynchronize(s));
-            (void)hipFree(dreps);
         }
         bp.nblock = (int64_t)bmap.size();
         // groups whose chunks repeat the previous group's one for one have the
@@ -1726,32 +1743,32 @@ int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *
             for (int t = 0; t < gn[g] && same; ++t) same = cmap[gfirst[g] + t] == cmap[gfirst[g - 1] + t];
             gmap[g] = same ? gmap[g - 1] : (int32_t)g;
         }
-        MADAM_CHECK(hipMalloc(&im->gmap, sizeof(int32_t) * gmap.size()));
+        MADAM_CHECK(device_malloc(&im->gmap, sizeof(int32_t) * gmap.size()));
         MADAM_CHECK(hipMemcpyAsync(im->gmap, gmap.data(), sizeof(int32_t) * gmap.size(), hipMemcpyHostToDevice, s));
-        MADAM_CHECK(hipMalloc(&im->cmap, sizeof(int32_t) * cmap.size()));
-        MADAM_CHECK(hipMalloc(&im->bmap, sizeof(int32_t) * bmap.size()));
+        MADAM_CHECK(device_malloc(&im->cmap, sizeof(int32_t) * cmap.size()));
+        MADAM_CHECK(device_malloc(&im->bmap, sizeof(int32_t) * bmap.size()));
         MADAM_CHECK(hipMemcpyAsync(im->cmap, cmap.data(), sizeof(int32_t) * cmap.size(), hipMemcpyHostToDevice, s));
         MADAM_CHECK(hipMemcpyAsync(im->bmap, bmap.data(), sizeof(int32_t) * bmap.size(), hipMemcpyHostToDevice, s));
         MADAM_CHECK(hipStreamSynchronize(s));   // the host tables above
-        if (direct) band_build_direct(s, bp, im, first, cmap);
+        if (direct && !if_room([&] { band_build_direct(s, bp, im, first, cmap); })) band_drop_direct(im);
     }
-    bp.impl = im;
     MADAM_CHECK(hipStreamSynchronize(s));
     return 0;
 }
 
-// the tables of the one-pass solve go
-static void band_drop_direct(BandImpl *im)
+// Returns 0 on success; fills info_out[s] (0 ok, >0 failing column) for each
+// segment.  Nothing stays allocated where it throws.
+int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *dseg, int64_t nseg,
+               const int *nband_seg_host, const double *invcov_dev, int64_t nof, const double *nna, int *info_out,
+               bool periodic, bool pieces, bool direct)
 {
-    im->direct = false;
-    for (double **p : {&im->Pf, &im->Pb, &im->PU, &im->LuD}) {
-        if (*p) (void)hipFree(*p);
-        *p = nullptr;
+    try {
+        return band_tables(s, bp, hseg, dseg, nseg, nband_seg_host, invcov_dev, nof, nna, info_out, periodic, pieces,
+                           direct);
+    } catch (...) {
+        band_free(bp);
+        throw;
     }
-    if (im->blk) (void)hipFree(im->blk);
-    if (im->pslot) (void)hipFree(im->pslot);
-    im->blk = nullptr;
-    im->pslot = nullptr;
 }
 
 // tables of the one-pass solve (3.9 KB per 64 rows where the factor does not
@@ -1798,32 +1815,30 @@ static void band_build_direct(hipStream_t s, const BandPrec &bp, BandImpl *im, c
     const int64_t ns = (int64_t)list.size(), nu = (int64_t)urep.size(), np = BD_LEV * BD_KK;
     im->nblk = (int64_t)blk.size();
     im->nslot = ns;
-    int32_t *dlist = nullptr;
-    uint8_t *dpure = nullptr;
-    unsigned long long *dworst = nullptr, worst = 0;
-    MADAM_CHECK(hipMalloc(&im->blk, sizeof(BandBlk) * blk.size()));
-    MADAM_CHECK(hipMalloc(&im->pslot, sizeof(int32_t) * nch));
-    MADAM_CHECK(hipMalloc(&im->Pf, sizeof(double) * np * ns));
-    MADAM_CHECK(hipMalloc(&im->Pb, sizeof(double) * np * ns));
-    MADAM_CHECK(hipMalloc(&dlist, sizeof(int32_t) * ns));
-    MADAM_CHECK(hipMalloc(&dpure, ns));
-    MADAM_CHECK(hipMalloc(&dworst, sizeof(unsigned long long)));
-    MADAM_CHECK(hipMemsetAsync(dworst, 0, sizeof(unsigned long long), s));
+    DBuf<int32_t> dlist;
+    DBuf<uint8_t> dpure;
+    DBuf<unsigned long long> dworst;
+    unsigned long long worst = 0;
+    MADAM_CHECK(device_malloc(&im->blk, sizeof(BandBlk) * blk.size()));
+    MADAM_CHECK(device_malloc(&im->pslot, sizeof(int32_t) * nch));
+    MADAM_CHECK(device_malloc(&im->Pf, sizeof(double) * np * ns));
+    MADAM_CHECK(device_malloc(&im->Pb, sizeof(double) * np * ns));
+    dlist.alloc(ns);
+    dpure.alloc(ns);
+    dworst.alloc(1);
+    MADAM_CHECK(hipMemsetAsync(dworst.p, 0, sizeof(unsigned long long), s));
     MADAM_CHECK(hipMemcpyAsync(im->blk, blk.data(), sizeof(BandBlk) * blk.size(), hipMemcpyHostToDevice, s));
     MADAM_CHECK(hipMemcpyAsync(im->pslot, pslot.data(), sizeof(int32_t) * nch, hipMemcpyHostToDevice, s));
-    MADAM_CHECK(hipMemcpyAsync(dlist, list.data(), sizeof(int32_t) * ns, hipMemcpyHostToDevice, s));
-    MADAM_CHECK(hipMemcpyAsync(dpure, pure.data(), ns, hipMemcpyHostToDevice, s));
+    MADAM_CHECK(hipMemcpyAsync(dlist.p, list.data(), sizeof(int32_t) * ns, hipMemcpyHostToDevice, s));
+    MADAM_CHECK(hipMemcpyAsync(dpure.p, pure.data(), ns, hipMemcpyHostToDevice, s));
     unsigned g = (unsigned)((ns * BD_KD + 63) / 64), gc = (unsigned)((nch + 63) / 64);
-    k_band_products<<<g, 64, 0, s>>>(dlist, dpure, ns, im->ch, bp.Tf, 0, im->Pf, ns, 1);
-    k_band_products<<<g, 64, 0, s>>>(dlist, dpure, ns, im->ch, bp.Tb, 1, im->Pb, ns, 1);
-    k_band_decay<<<gc, 64, 0, s>>>(im->pslot, nch, im->ch, im->Pf, ns, 0, dworst);
-    k_band_decay<<<gc, 64, 0, s>>>(im->pslot, nch, im->ch, im->Pb, ns, 1, dworst);
+    k_band_products<<<g, 64, 0, s>>>(dlist.p, dpure.p, ns, im->ch, bp.Tf, 0, im->Pf, ns, 1);
+    k_band_products<<<g, 64, 0, s>>>(dlist.p, dpure.p, ns, im->ch, bp.Tb, 1, im->Pb, ns, 1);
+    k_band_decay<<<gc, 64, 0, s>>>(im->pslot, nch, im->ch, im->Pf, ns, 0, dworst.p);
+    k_band_decay<<<gc, 64, 0, s>>>(im->pslot, nch, im->ch, im->Pb, ns, 1, dworst.p);
     MADAM_CHECK(hipGetLastError());
-    MADAM_CHECK(hipMemcpyAsync(&worst, dworst, sizeof(worst), hipMemcpyDeviceToHost, s));
+    MADAM_CHECK(hipMemcpyAsync(&worst, dworst.p, sizeof(worst), hipMemcpyDeviceToHost, s));
     MADAM_CHECK(hipStreamSynchronize(s));
-    (void)hipFree(dlist);
-    (void)hipFree(dpure);
-    (void)hipFree(dworst);
     double w;
     static_assert(sizeof w == sizeof worst, "");
     memcpy(&w, &worst, sizeof w);
@@ -1831,26 +1846,29 @@ static void band_build_direct(hipStream_t s, const BandPrec &bp, BandImpl *im, c
         band_drop_direct(im);
         return;
     }
-    MADAM_CHECK(hipMalloc(&im->PU, sizeof(double) * 2 * np * std::max<int64_t>(nu, 1)));
-    MADAM_CHECK(hipMalloc(&im->LuD, sizeof(double) * BAND_CH * BD_K * std::max<int64_t>(nu, 1)));
+    MADAM_CHECK(device_malloc(&im->PU, sizeof(double) * 2 * np * std::max<int64_t>(nu, 1)));
+    MADAM_CHECK(device_malloc(&im->LuD, sizeof(double) * BAND_CH * BD_K * std::max<int64_t>(nu, 1)));
     if (nu > 0) {
         std::vector<uint8_t> one(nu, 1);
-        int32_t *durep = nullptr;
-        MADAM_CHECK(hipMalloc(&durep, sizeof(int32_t) * nu));
-        MADAM_CHECK(hipMalloc(&dpure, nu));
-        MADAM_CHECK(hipMemcpyAsync(durep, urep.data(), sizeof(int32_t) * nu, hipMemcpyHostToDevice, s));
-        MADAM_CHECK(hipMemcpyAsync(dpure, one.data(), nu, hipMemcpyHostToDevice, s));
+        DBuf<int32_t> durep;
+        durep.alloc(nu);
+        dpure.alloc(nu);
+        MADAM_CHECK(hipMemcpyAsync(durep.p, urep.data(), sizeof(int32_t) * nu, hipMemcpyHostToDevice, s));
+        MADAM_CHECK(hipMemcpyAsync(dpure.p, one.data(), nu, hipMemcpyHostToDevice, s));
         unsigned gu = (unsigned)((nu * BD_KD + 63) / 64);
-        k_band_products<<<gu, 64, 0, s>>>(durep, dpure, nu, im->ch, bp.Tf, 0, im->PU, 1, 2 * np);
-        k_band_products<<<gu, 64, 0, s>>>(durep, dpure, nu, im->ch, bp.Tb, 1, im->PU + np, 1, 2 * np);
+        k_band_products<<<gu, 64, 0, s>>>(durep.p, dpure.p, nu, im->ch, bp.Tf, 0, im->PU, 1, 2 * np);
+        k_band_products<<<gu, 64, 0, s>>>(durep.p, dpure.p, nu, im->ch, bp.Tb, 1, im->PU + np, 1, 2 * np);
         k_band_compact_chunks<<<(unsigned)std::min<int64_t>((nu * BAND_CH * BD_K + 255) / 256, 65535), 256, 0, s>>>(
-            im->Li, durep, nu, im->LuD);
+            im->Li, durep.p, nu, im->LuD);
         MADAM_CHECK(hipGetLastError());
         MADAM_CHECK(hipStreamSynchronize(s));   // one
-        (void)hipFree(durep);
-        (void)hipFree(dpure);
     }
     im->direct = true;
+}
+
+void band_give_up_direct(const BandPrec &bp)
+{
+    if (bp.impl) band_drop_direct((BandImpl *)bp.impl);
 }
 
 int band_capacity(const BandPrec &bp) { return bp.impl ? ((const BandImpl *)bp.impl)->rcap : 0; }
@@ -1862,13 +1880,16 @@ void band_reserve(const BandPrec &bp, int nrhs)
     if (!im || bp.nchunk == 0 || nrhs <= im->rcap) return;
     int KD = bp.kd;
     int64_t nc = bp.nchunk, ng = im->ngrp > 0 ? im->ngrp : 1;
+    im->rcap = 0;   // no room at all while an allocation below may fail
     for (double **b : {&im->s0f, &im->s0b, &im->sinf, &im->sinb}) {
         (void)hipFree(*b);
-        MADAM_CHECK(hipMalloc(b, sizeof(double) * nc * KD * nrhs));
+        *b = nullptr;
+        MADAM_CHECK(device_malloc(b, sizeof(double) * nc * KD * nrhs));
     }
     for (double **b : {&im->cg, &im->Sg}) {
         (void)hipFree(*b);
-        MADAM_CHECK(hipMalloc(b, sizeof(double) * ng * KD * nrhs));
+        *b = nullptr;
+        MADAM_CHECK(device_malloc(b, sizeof(double) * ng * KD * nrhs));
     }
     im->rcap = nrhs;
 }

@@ -701,27 +701,11 @@ static void signal_rhs(Context &c, const TT *tod, const double *rhs4, double *yb
 // signals per pass of the shared binning (and subtraction): 4 or 8
 static int bin_group(int n) { return n <= 4 ? 4 : 8; }
 
-// device memory that may not be there: false leaves the buffer empty
-template <typename T>
-static bool try_alloc(DBuf<T> &b, size_t n)
-{
-    try {
-        b.alloc(n);
-    } catch (const HipError &e) {
-        if (e.err != hipErrorOutOfMemory) throw;
-        (void)hipGetLastError();
-        b.p = nullptr;
-        b.n = 0;
-        return false;
-    }
-    return true;
-}
-
 // binned maps rhs4[k] and right-hand sides yba[k] of the signals k = 1 ..
 // nrhs - 1 (the set-up has made those of the first): signals on the device are
-// binned bin_group at a time, from a copy with their samples side by side (32
-// or 64 bytes a sample; without the memory for it, one at a time, as signals
-// from the host are)
+// binned bin_group at a time, from a copy with their samples side by side (16
+// to 64 bytes a sample; where memory is short, one at a time, as signals from
+// the host are)
 template <typename TT, typename F>
 static void bin_signals(Context &c, BatchState &B, int nrhs, int on_device, F &&signal)
 {
@@ -735,8 +719,10 @@ static void bin_signals(Context &c, BatchState &B, int nrhs, int on_device, F &&
     const int gr = bin_group(nrhs - 1);
     DBuf<TT> turned;
     DBuf<int32_t> list;
-    if (on_device && nrhs > 2 && try_alloc(turned, (size_t)std::max<int64_t>(n, 1) * gr)) {
-        list.alloc(np + 1);
+    if (on_device && nrhs > 2 && !c.lean && if_room([&] {
+            list.alloc(np + 1);
+            turned.alloc((size_t)std::max<int64_t>(n, 1) * gr);
+        })) {
         for (int k0 = 1; k0 < nrhs; k0 += gr) {
             int nr = std::min(gr, nrhs - k0);
             batch_turn<TT>(s, gr, signal(k0), n, nr, turned.p);
@@ -971,8 +957,10 @@ static void solve_batch_t(Context &c, int nrhs, const TT *signals, int on_device
 
 void solve_batch(Context &c, int nrhs, const void *signals, int tod_f32, int on_device, int precision)
 {
-    if (tod_f32) solve_batch_t<float>(c, nrhs, (const float *)signals, on_device, precision);
-    else solve_batch_t<double>(c, nrhs, (const double *)signals, on_device, precision);
+    with_room(c, [&] {
+        if (tod_f32) solve_batch_t<float>(c, nrhs, (const float *)signals, on_device, precision);
+        else solve_batch_t<double>(c, nrhs, (const double *)signals, on_device, precision);
+    });
 }
 
 // Benchmark / continuation: exactly niter PCG steps of the last batch's PCG

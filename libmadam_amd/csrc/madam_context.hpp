@@ -72,7 +72,7 @@ struct DBuf {
     {
         if (count <= n && p) return;
         release();
-        MADAM_CHECK(hipMalloc(&p, sizeof(T) * (count > 0 ? count : 1)));
+        MADAM_CHECK(device_malloc(&p, sizeof(T) * (count > 0 ? count : 1)));
         n = count;
     }
     void release()
@@ -81,6 +81,9 @@ struct DBuf {
         p = nullptr;
         n = 0;
     }
+    DBuf() = default;
+    DBuf(const DBuf &) = delete;
+    DBuf &operator=(const DBuf &) = delete;
     ~DBuf() { release(); }
 };
 
@@ -253,6 +256,8 @@ struct Context {
     // configuration, pointing and kernel choice stay and reused when nna is
     // bitwise the same (they are functions of those alone)
     bool prec_cached = false;
+    // device memory has run short on this pointing: no tables that only save time
+    bool lean = false;
     uint64_t set_up = 0;   // builds of the pointing's and the preconditioner's tables so far
     int prec_cached_variant = 0;
     DBuf<double> d_nna_key;
@@ -328,6 +333,33 @@ struct Timer {
 
 void ensure_stream(Context &c);
 int group_for(const Context &c);
+// f, false where device memory is short for it
+template <typename F>
+bool if_room(F &&f)
+{
+    try {
+        f();
+        return true;
+    } catch (const HipError &e) {
+        if (e.err != hipErrorOutOfMemory) throw;
+    }
+    (void)hipGetLastError();
+    return false;
+}
+// frees the tables that only save time (run records, the one-pass band solve's
+// products), and keeps to what every solve needs until the next pointing
+void give_up_tables(Context &c);
+// f, and where device memory is short for it, f again without those tables.  f
+// starts over from its inputs.
+template <typename F>
+void with_room(Context &c, F &&f)
+{
+    if (!c.lean) {
+        if (if_room(f)) return;
+        give_up_tables(c);
+    }
+    f();
+}
 // binning, inversion, projection tables, initialize_a and (unless nna is
 // bitwise that of the cached set-up) segments, filters and preconditioner of
 // one solve (src/smadam.F90:316-400), for a TOD of type TT on the device

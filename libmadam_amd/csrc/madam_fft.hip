@@ -363,9 +363,9 @@ void fft_plan_init(FftPlan &p, int64_t nof, hipStream_t s)
     std::vector<double> hd(h.begin(), h.end());
     std::vector<float> hf(h.size());
     for (size_t i = 0; i < h.size(); ++i) hf[i] = (float)h[i];
-    MADAM_CHECK(hipMalloc(&p.tw_mem, sizeof(double) * hd.size()));
+    MADAM_CHECK(device_malloc(&p.tw_mem, sizeof(double) * hd.size()));
     MADAM_CHECK(hipMemcpyAsync(p.tw_mem, hd.data(), sizeof(double) * hd.size(), hipMemcpyHostToDevice, s));
-    MADAM_CHECK(hipMalloc(&p.tw32_mem, sizeof(float) * hf.size()));
+    MADAM_CHECK(device_malloc(&p.tw32_mem, sizeof(float) * hf.size()));
     MADAM_CHECK(hipMemcpyAsync(p.tw32_mem, hf.data(), sizeof(float) * hf.size(), hipMemcpyHostToDevice, s));
     MADAM_CHECK(hipStreamSynchronize(s));   // hd and hf are freed on return
     const double2 *b = (const double2 *)p.tw_mem;

@@ -635,7 +635,8 @@ static void build_filters(Context &c)
     MADAM_CHECK(hipStreamSynchronize(s));
     if (hbad) fail("non-positive PSD values are not supported by the noise filter");
     if (!c.fft_ready || c.fft.N != c.nof / 2) {
-        if (c.fft_ready) fft_plan_free(c.fft);
+        fft_plan_free(c.fft);
+        c.fft_ready = false;
         fft_plan_init(c.fft, c.nof, s);
         c.fft_ready = true;
     }
@@ -648,7 +649,7 @@ static void build_filters(Context &c)
 // dummy_is_flag: pixel 12 * nside_max**2, which a previous call leaves in the
 // caller's array for its flagged samples, flags the sample again (the cached
 // path, src/smadam.F90:713-715)
-static void set_pointing(Context &c, int32_t *pix, float *w, int on_device, bool dummy_is_flag = false)
+static void point(Context &c, int32_t *pix, float *w, int on_device, bool dummy_is_flag)
 {
     if (!c.configured) fail("madam_set_pointing called before configure");
     c.set_up++;
@@ -727,6 +728,7 @@ static void set_pointing(Context &c, int32_t *pix, float *w, int on_device, bool
         MADAM_CHECK(hipMemsetAsync(cnt.p, 0, sizeof(unsigned long long) * 3, s));
         int dsh = 0;
         while ((1ll << dsh) < c.ndeg) ++dsh;
+        c.pointed = false;   // the tables below are replaced one by one
         launch_pack(s, c.d_pix, c.d_w, c.nnz, c.nmap, c.ndet, c.nsamp, c.d_ivs.p, c.nival, c.d_dw_ival.p,
                     c.p.nsubchunk, c.pass, c.d_pixw.p, cs.k[0].p, (uint32_t)c.npix_map, c.d_pixc.p, dsh, cnt.p);
         MADAM_CHECK(hipGetLastError());
@@ -786,6 +788,12 @@ static void set_pointing(Context &c, int32_t *pix, float *w, int on_device, bool
     batch_invalidate(c);
 }
 
+static void set_pointing(Context &c, int32_t *pix, float *w, int on_device, bool dummy_is_flag = false)
+{
+    c.lean = false;
+    with_room(c, [&] { point(c, pix, w, on_device, dummy_is_flag); });
+}
+
 // ------------------------------------------------------------------ solve
 
 static void segtiles_alloc(Context::SegTiles &t, int64_t nent)
@@ -809,7 +817,7 @@ static constexpr int64_t RUN_SAMPLES = 1 << 18;
 template <typename T>
 static bool runs_wanted(const Context &c)
 {
-    if (c.rec_layout == REC16 || c.nactive <= 0) return false;
+    if (c.rec_layout == REC16 || c.nactive <= 0 || c.lean) return false;
     if (c.nactive < RUN_SAMPLES && !(c.kernel_variant & 128)) return false;
     return c.mean_run >= (sizeof(T) == 8 ? 2.0 : 1.3);
 }
@@ -869,24 +877,6 @@ static bool build_runs(Context &c, DBuf<W> &gw, DBuf<W> &sw)
     return true;
 }
 
-// Below two samples per run the FP64 operator reads samples, and the records
-// hold FP32 sums alone.
-void runs_prepare_fp32(Context &c)
-{
-    if (!runs_wanted<float>(c) || c.runs32_ok) return;
-    if (!c.runs_ok) {
-        c.runs32_ok = build_runs(c, c.d_rungw32, c.d_runsw32);
-        return;
-    }
-    if (c.nmap == 3) {
-        c.d_rungw32.alloc(c.n_rung);
-        c.d_runsw32.alloc(c.n_runs);
-        runs_cast(c.stream, c.d_rungw.p, c.d_rungw32.p, c.n_rung);
-        runs_cast(c.stream, c.d_runsw.p, c.d_runsw32.p, c.n_runs);
-    }
-    c.runs32_ok = true;
-}
-
 static void release_runs(Context &c)
 {
     c.runs_ok = c.runs32_ok = false;
@@ -897,7 +887,32 @@ static void release_runs(Context &c)
     c.d_rungw32.release();
     c.d_runsw32.release();
     c.d_rungst.release();
-    c.sr_r = Context::SegTiles();
+    c.sr_r.heads.release();
+    c.sr_r.k0.release();
+    c.sr_r.fix_end.release();
+    c.sr_r.fix_ord.release();
+}
+
+// Below two samples per run the FP64 operator reads samples, and the records
+// hold FP32 sums alone.
+void runs_prepare_fp32(Context &c)
+{
+    if (!runs_wanted<float>(c) || c.runs32_ok) return;
+    if (!c.runs_ok) {
+        if (!if_room([&] { c.runs32_ok = build_runs(c, c.d_rungw32, c.d_runsw32); })) release_runs(c);
+        return;
+    }
+    c.runs32_ok = if_room([&] {
+        if (c.nmap != 3) return;
+        c.d_rungw32.alloc(c.n_rung);
+        c.d_runsw32.alloc(c.n_runs);
+        runs_cast(c.stream, c.d_rungw.p, c.d_rungw32.p, c.n_rung);
+        runs_cast(c.stream, c.d_runsw.p, c.d_runsw32.p, c.n_runs);
+    });
+    if (!c.runs32_ok) {
+        c.d_rungw32.release();
+        c.d_runsw32.release();
+    }
 }
 
 template <typename T>
@@ -923,6 +938,15 @@ template <typename T>
 static bool use_runs(const Context &c)
 {
     return (sizeof(T) == 8 ? c.runs_ok : c.runs32_ok) && runs_wanted<T>(c);
+}
+
+void give_up_tables(Context &c)
+{
+    MADAM_CHECK(hipStreamSynchronize(c.stream));
+    c.lean = true;
+    c.set_up++;
+    release_runs(c);
+    if (c.band_ready) band_give_up_direct(c.band);
 }
 
 int64_t runs_read(const Context &c, bool fp32)
@@ -1011,7 +1035,7 @@ static void build_segtiles(Context &c)
     c.d_sr_part.alloc(2 * (nt > 0 ? nt : 1));
     // (buffers of the pointing before are kept only where this one's solves can use them)
     if (runs_wanted<double>(c)) {
-        c.runs_ok = build_runs(c, c.d_rungw, c.d_runsw);
+        if (!if_room([&] { c.runs_ok = build_runs(c, c.d_rungw, c.d_runsw); })) release_runs(c);
     } else {
         c.d_rungw.release();
         c.d_runsw.release();
@@ -1270,7 +1294,8 @@ static void build_preconditioner(Context &c)
     for (;;) {
         std::vector<int> info(c.segp.size(), 0);
         if (band_build(s, c.band, c.segp.data(), c.d_segp.p, (int64_t)c.segp.size(), nband.data(), c.d_invcov.p, c.nof,
-                       c.d_nna.p, info.data(), !(c.kernel_variant & 16), band_chain_pack(c.kernel_variant) < 0) != 0)
+                       c.d_nna.p, info.data(), !(c.kernel_variant & 16), !c.lean,
+                       !c.lean && band_chain_pack(c.kernel_variant) < 0) != 0)
             fail("band preconditioner wider than %d baselines reached the factor kernels", BAND_WIDTH_GPU);
         c.band_ready = true;
         bool retry = false;
@@ -1618,10 +1643,12 @@ void solve_setup(Context &c, const TT *tod)
             int differ = 1;
             d2h(&differ, c.d_flag.p, 1, s);
             MADAM_CHECK(hipStreamSynchronize(s));
-            reuse = differ == 0;
+            // (no room: band_reserve ran out of memory)
+            reuse = differ == 0 && (c.precond_kind != 3 || band_capacity(c.band) > 0);
         }
         if (!reuse) {
             c.set_up++;
+            c.prec_cached = false;
             build_segments(c);
         }
         c.stats[ST_PREC_REUSED] = reuse ? 1 : 0;
@@ -1655,7 +1682,7 @@ void solve_setup(Context &c, const TT *tod)
 template void solve_setup<double>(Context &, const double *);
 template void solve_setup<float>(Context &, const float *);
 
-static void solve(Context &c, double *signal, int on_device)
+static void solve_once(Context &c, double *signal, int on_device)
 {
     if (!c.pointed) fail("madam_solve called before the pointing was set");
     hipStream_t s = c.stream;
@@ -1714,6 +1741,12 @@ static void solve(Context &c, double *signal, int on_device)
     MADAM_CHECK(hipStreamSynchronize(s));
     c.stats[ST_T_TOTAL] = now() - tstart;
     c.solved = true;
+}
+
+// (the signal is cleaned last, after every allocation)
+static void solve(Context &c, double *signal, int on_device)
+{
+    with_room(c, [&] { solve_once(c, signal, on_device); });
 }
 
 // restore_pixels for host arrays: flagged samples -> 12 * nside_max**2
@@ -2440,6 +2473,24 @@ static int guarded(F &&f)
     return 1;
 }
 
+static thread_local long g_allocations = 0, g_fail_first = -1, g_fail_end = -1;
+
+hipError_t madam::device_malloc(void **p, size_t bytes)
+{
+    const long k = g_allocations++;
+    if (k >= g_fail_first && k < g_fail_end) return hipErrorOutOfMemory;
+    return hipMalloc(p, bytes);
+}
+
+MADAM_API long madam_fail_allocations(long first, long n)
+{
+    const long made = g_allocations;
+    g_allocations = 0;
+    g_fail_first = first;
+    g_fail_end = first < 0 ? -1 : first + n;
+    return made;
+}
+
 static int g_last_status = 0;
 
 // The reference aborts the MPI job on any error (src/mpi_wrappers.f90:120-134).
@@ -2506,7 +2557,7 @@ MADAM_API int madam_iterate(void *ctx, int niter, int restart)
 {
     return guarded([&] {
         Context &c = *(Context *)ctx;
-        if (!c.solved || !c.p.kfirst) fail("madam_iterate needs a completed madam_solve with destriping");
+        if (!c.solved || !c.p.kfirst || !c.tiles_built) fail("madam_iterate needs a completed madam_solve with destriping");
         if (restart) pcg_init(c);
         pcg_steps(c, niter, false);
     });

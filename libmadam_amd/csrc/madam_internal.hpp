@@ -174,6 +174,16 @@ struct HipError {
     HipError(hipError_t e, const char *w, const char *f, int l) : err(e), what(w), file(f), line(l) {}
 };
 
+// hipMalloc for every buffer of the library.  It counts the calling thread's
+// allocations, of which madam_fail_allocations can have some fail.
+hipError_t device_malloc(void **p, size_t bytes);
+template <typename T>
+hipError_t device_malloc(T **p, size_t bytes)
+{
+    *p = nullptr;
+    return device_malloc((void **)p, bytes);
+}
+
 // ------------------------------------------------------------------ kernels.hip
 
 void launch_flag_and_count(hipStream_t s, int32_t *pix, const float *w, int nnz, int ndet, int64_t nsamp,
@@ -436,7 +446,7 @@ inline int band_chain_pack(int kernel_variant)
 
 int band_build(hipStream_t s, BandPrec &bp, const Segment *hseg, const Segment *dseg, int64_t nseg,
                const int *nband_seg_host, const double *invcov_dev, int64_t nof, const double *nna, int *info_out,
-               bool periodic, bool direct);   // direct: the one-pass solve's tables too, where it can be used
+               bool periodic, bool pieces, bool direct);   // direct: the one-pass solve's tables too, where it can be used
 // z = M^-1 r for nrhs right-hand sides at a stride of vstride elements (T =
 // float or double; the factor and the solves are FP64)
 template <typename T>
@@ -445,6 +455,8 @@ void band_apply(hipStream_t s, const BandPrec &bp, const T *r, T *z, int nrhs = 
 void band_reserve(const BandPrec &bp, int nrhs);
 // the right-hand sides there is room for (the buffers move when that grows)
 int band_capacity(const BandPrec &bp);
+// frees the one-pass solve's tables: the chains take its place
+void band_give_up_direct(const BandPrec &bp);
 void band_free(BandPrec &bp);
 
 // ------------------------------------------------------------------ pointing.hip

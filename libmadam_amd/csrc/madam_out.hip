@@ -157,10 +157,9 @@ void copy_out(Context &c, const std::vector<OutItem> &items)
     (void)hipGetLastError();
     size_t total = 0;
     for (const OutItem &it : items) total += (size_t)it.n * elem_bytes(it.kind) + 8;
-    if (total <= OUT_SMALL) {
+    DBuf<char> d;
+    if (total <= OUT_SMALL && if_room([&] { d.alloc(total); })) {
         // everything in one launch into device scratch, and one copy
-        DBuf<char> d;
-        d.alloc(total);
         std::vector<char> h(total);
         OutPieces ps;
         size_t off = 0, i0 = 0;
@@ -226,8 +225,7 @@ void copy_out(Context &c, const std::vector<OutItem> &items)
     SlotLease slots(want, s);
     if (slots.p.empty()) {
         // every slot is lent: lay out in device scratch and let the runtime copy
-        DBuf<char> d;
-        d.alloc(OUT_SLOT);
+        with_room(c, [&] { d.alloc(OUT_SLOT); });
         for (const Chunk &ck : chunks) {
             const OutItem &it = items[ck.item];
             size_t eb = elem_bytes(it.kind);
