@@ -90,7 +90,9 @@ struct Resident {
 // records, CSR and compact records and the TOD (~90 B); per map pixel the
 // pixel matrices, maps and tables (~300 B); per baseline the PCG vectors,
 // band factor and slot tables (~260 B, x R right-hand sides for the vectors);
-// plus the FFT batch buffer and a fixed allowance
+// plus the FFT batch buffer and a fixed allowance.  The signals of a group side
+// by side (16 to 64 B a sample) stay below what its jobs are estimated at
+// together.
 size_t estimate_bytes(const Job &j, long nside_max, long nbase_est, int nrhs)
 {
     size_t n = (size_t)j.ndet * j.nsamp;
@@ -98,6 +100,17 @@ size_t estimate_bytes(const Job &j, long nside_max, long nbase_est, int nrhs)
     size_t nb = (size_t)j.ndet * nbase_est;
     size_t per_rhs = (size_t)(j.tod_f32 ? 4 : 8) * n + nb * 80 + npix * 3 * 8;
     return n * 90 + npix * 300 + nb * 260 + (size_t)nrhs * per_rhs + (256ull << 20);
+}
+
+// the tables that a solve of its own does without where memory is short: run
+// records of both sides (per run a word, FP64 and, in a mixed solve, FP32
+// weight sums, and 2 B of segment tables: 30 B a side and 2 samples, or 14 B and
+// 1.3 samples; 22 B in FP64 alone) and the one-pass band solve's products (3.9
+// KB per 64 baselines)
+size_t estimate_tables(const Job &j, long nbase_est)
+{
+    size_t n = (size_t)j.ndet * j.nsamp;
+    return n * (j.precision == 1 ? 30 : 22) + (size_t)j.ndet * nbase_est * 62;
 }
 
 long parse_long(const std::string &pars, const char *key, long dflt)
@@ -499,6 +512,8 @@ MADAM_API long madam_server_submit(void *srv, const char *parstring, long ndet, 
     j->est_bytes = estimate_bytes(*j, nside, nbase, 1);
     std::lock_guard<std::mutex> lk(s->mu);
     if (j->est_bytes > s->budget) return -1;
+    // (a job that fits the budget only without the tables has it to itself)
+    j->est_bytes = std::min(j->est_bytes + estimate_tables(*j, nbase), s->budget);
     j->id = s->next_id++;
     j->t_submit = wall();
     s->jobs[j->id] = j;
