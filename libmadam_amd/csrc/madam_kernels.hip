@@ -1489,12 +1489,6 @@ int dots_nblocks(int64_t n)
     return (int)b;
 }
 
-// which = 0: sum a*b (1 value)
-// which = 1: sum a*b, sum c*b, sum a*a (3 values: rz, rz2, rr with a=r, b=z, c=ro)
-// Only elements with mask != 0 count.  Each thread takes chunks of 8 elements
-// and issues all of a chunk's loads (mask as one 8-byte word, the vectors as
-// 16-byte pairs) before the arithmetic; the block partials and their final
-// sum are in a fixed order, so the result depends on n alone.
 // The end of the step's scalars (t: rz, rz2, rr): scal[2..4], beta = (scal[2]
 // - scal[3]) / scal[0] into scal[5], the old rz into scal[6], the new one into
 // scal[0]; then the exit tests of src/smadam_routines.f90:905-918, whose
@@ -1567,6 +1561,12 @@ __device__ inline void dots_tail(double s0, double s1, double s2, double *partia
     }
 }
 
+// which = 0: sum a*b (1 value)
+// which = 1: sum a*b, sum c*b, sum a*a (3 values: rz, rz2, rr with a=r, b=z, c=ro)
+// Only elements with mask != 0 count.  Each thread takes chunks of 8 elements
+// and issues all of a chunk's loads (mask as one 8-byte word, the vectors as
+// 16-byte pairs) before the arithmetic; the block partials and their final
+// sum are in a fixed order, so the result depends on n alone.
 __global__ void __launch_bounds__(TPB) k_dots(int which, const double *a, const double *b, const double *c,
                                               const int8_t *mask, int64_t n, double *partials, DotsEnd fin)
 {
