@@ -122,7 +122,8 @@ def bytes_fp64(st, ndet, nsamp, npix, nbtot, s=8):
     and pw (1 value)"""
     rec = st.get("rec_bytes") or 16
     nact = st["nactive"]
-    if st.get("run_records") and rec < 16:   # run records: a word and two weight sums per run
+    # run records: a word and two weight sums per run (the pixel side is taken to have as many)
+    if st.get("run_records") and rec < 16:
         rec = (4 + (2 * s if rec == 12 else 0)) * st["run_records"] / (ndet * nsamp)
     return dict(gather=ndet * nsamp * rec + npix * 3 * s + nbtot * 5 * s,
                 scatter=nact * rec + nbtot * s + npix * (8 + 6 * s + 4 * s))

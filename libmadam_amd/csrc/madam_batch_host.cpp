@@ -476,14 +476,13 @@ static std::vector<uint64_t> step_key(Context &c, BatchState &B, const Vec<T> &v
                             (uint64_t)B.bt_c.nitems,
                             (uint64_t)B.bt_c.nfix,
                             (uint64_t)B.bt_c.nparts,
-                            (uint64_t)c.runs_ok,
-                            (uint64_t)c.runs32_ok,
+                            (uint64_t)(c.rg.ok64 | c.rg.ok32 << 1 | c.rs.ok64 << 2 | c.rs.ok32 << 3),
                             (uint64_t)band_capacity(c.band)};
     for (const void *p : std::initializer_list<const void *>{
              v.x, v.r, v.ro, v.z, v.p, v.ap, v.pw, v.m, v.part, B.dots.p, B.sc.p, B.active.p, B.d_segR.p, B.fftwork.p,
              Ops<T>::dwb(c, B), Ops<T>::nna(c, B), Ops<T>::cc(c, B), Ops<T>::m4(c, B), Ops<T>::fcov32(B),
              Ops<T>::fprec32(B), B.bt.items, B.bt.fix, B.bt_c.items, B.bt_c.fix, B.rg_rec.p, B.rg_st.p, B.rg_base.p,
-             B.rs_rec.p, c.d_rung.p, c.d_rungw.p, c.d_rungw32.p, c.d_runs.p, c.d_runsw.p, c.d_runsw32.p})
+             B.rs_rec.p, c.rg.word.p, c.rg.w64.p, c.rg.w32.p, c.rs.word.p, c.rs.w64.p, c.rs.w32.p})
         k.push_back((uint64_t)(uintptr_t)p);
     return k;
 }

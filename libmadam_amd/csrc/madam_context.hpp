@@ -206,19 +206,22 @@ struct Context {
         int64_t nent = 0;
         bool ok = false;
     } sr_s, sr_g;
-    // run records of the one-right-hand-side projections (madam_runs.hip):
-    // mean_run is the estimated samples per run, runs_ok / runs32_ok whether
-    // the records of this pointing exist with FP64 / FP32 weight sums
+    // run records of the one-right-hand-side projections (madam_runs.hip), per
+    // side: the words, and the weight sums in the types that are read (ok*:
+    // there for this pointing).  mean_run is the estimated number of samples per
+    // run of the baseline side, len the counted one of a side (0: not counted).
+    struct Runs {
+        DBuf<uint32_t> word;
+        DBuf<double2> w64;
+        DBuf<float2> w32;
+        int64_t n = 0;
+        double len = 0;
+        bool ok64 = false, ok32 = false;
+    } rg, rs;
     double mean_run = 0;
-    bool runs_ok = false;
     int run_sh = 0;
-    int64_t n_rung = 0, n_runs = 0;
-    DBuf<uint32_t> d_rung, d_runs;
-    DBuf<double2> d_rungw, d_runsw;
-    DBuf<float2> d_rungw32, d_runsw32;
-    bool runs32_ok = false;
-    DBuf<int64_t> d_rungst;
-    SegTiles sr_r;   // pixel-side segment tables over the runs
+    DBuf<int64_t> d_rungst;   // baseline side: first run of each baseline
+    SegTiles sr_r;            // pixel side: segment tables over the runs
     DBuf<int32_t> d_nzq;
     DBuf<int64_t> d_segstart_s;   // CSR start of each non-empty cross pixel (pixel-side ordinal order)
     DBuf<double> d_ccinv_c;   // inverse cross-pixel matrices in the pixel side's ordinal order
@@ -369,8 +372,7 @@ void cg_apply(Context &c, const double *r, double *z);
 // the two projections of one right-hand side, from the run records where the
 // pointing has them: m4 = ccinv P^T W F p (pw = p dwb in slot order), and
 // ap += nna p - F^T W P m4 (add 0: ap =)
-// the FP32 weight sums of the run records, before FP32 projections (allocates:
-// call outside graph capture)
+// the run records that the FP32 projections read (allocates: call outside graph capture)
 void runs_prepare_fp32(Context &c);
 // runs that the baseline side reads in FP64 / FP32 (0: it reads samples)
 int64_t runs_read(const Context &c, bool fp32);

@@ -781,7 +781,10 @@ static void point(Context &c, int32_t *pix, float *w, int on_device, bool dummy_
     c.stats[ST_NACTIVE] = (double)total;
     c.pointed = true;
     c.tiles_built = false;
-    c.runs_ok = c.runs32_ok = false;
+    for (Context::Runs *r : {&c.rg, &c.rs}) {
+        r->ok64 = r->ok32 = false;
+        r->len = 0;
+    }
     c.stats[ST_RUN_RECORDS] = 0;
     c.prec_cached = false;
     c.stats[ST_POINTING_REUSED] = 0;
@@ -806,138 +809,168 @@ static void segtiles_alloc(Context::SegTiles &t, int64_t nent)
     t.fix_ord.alloc(nt > 0 ? nt : 1);
 }
 
-// Whether the one-right-hand-side projections in type T read run records:
-// where a run's record (20 bytes in FP64, 12 in FP32, 4 for temperature) is
-// smaller than its samples' (12 or 4 bytes each) by enough to pay for the
-// separate weight stream (both sides measured in madam_runs.hip).  Building
-// them takes some 0.5 ms of launches and allocations, which a solve of fewer
-// than RUN_SAMPLES samples does not earn back (a 4,000-sample destripe: 5.8 ms
-// without, 6.4 ms with); kernel variant + 128 builds them for any number.
+// Whether the one-right-hand-side projections in type T read run records.
+// Building them takes some 0.5 ms of launches and allocations, which a solve of
+// fewer than RUN_SAMPLES samples does not earn back (a 4,000-sample destripe:
+// 5.8 ms without, 6.4 ms with); kernel variant + 128 builds them for any number.
+// Each side then reads them where a run (20 bytes in FP64, 12 in FP32, 4 for
+// temperature) costs less than its samples (12 or 4 bytes each).  Measured on
+// 3.4e7 samples, us per launch, runs / samples:
+//   baseline side, FP64: 2.05 samples per run 103 / 89, 2.2 97 / 90, 2.5 86 / 89
+//   (detectors on one boresight share the sample records' map loads; on their
+//   own boresights 126 / 125, 119 / 123, 107 / 118); FP32 1.33 91 / 88, 1.5 83 / 86
+//   (own boresights 120 / 129, 107 / 124)
+//   pixel side, FP64: 1.43 102 / 92, 1.65 80 / 79, 2.1 63 / 80; FP32 1.17 79 / 77,
+//   1.2 76 / 77, 1.43 56 / 80; temperature 1.04 47 / 49
+// The pixel side's runs end at every map pixel, which cross pixels may hold
+// many of, so their number is counted; the baseline side's is estimated when
+// the pointing is packed, and a count far below the estimate is believed.
 static constexpr int64_t RUN_SAMPLES = 1 << 18;
 template <typename T>
-static bool runs_wanted(const Context &c)
+static bool runs_considered(const Context &c)
 {
     if (c.rec_layout == REC16 || c.nactive <= 0 || c.lean) return false;
     if (c.nactive < RUN_SAMPLES && !(c.kernel_variant & 128)) return false;
     return c.mean_run >= (sizeof(T) == 8 ? 2.0 : 1.3);
 }
 
-// run records of both projections with weight sums of type W, and the pixel
-// side's segment tables over them; false where the word cannot hold the indices
-template <typename W>
-static bool build_runs(Context &c, DBuf<W> &gw, DBuf<W> &sw)
+template <typename T>
+static bool runs_wanted(const Context &c, const Context::Runs &r)
 {
-    hipStream_t s = c.stream;
-    int dsh = 0;
-    while ((1ll << dsh) < c.ndeg) ++dsh;
-    int sh = 1;
-    while ((1ll << sh) < std::max(c.npix_cross, c.nbtot)) ++sh;
-    if (sh > 28) return false;
-    uint32_t maxrun = (1u << (32 - sh)) - 1u;
-    int64_t n = (int64_t)c.ndet * c.nsamp, nent = c.nactive, nmax = std::max(n, nent);
-    DBuf<uint32_t> mask;
-    DBuf<unsigned long long> words;
-    DBuf<int32_t> counts;
-    DBuf<int64_t> offs, tmp, seg;
-    int64_t nsp = runs_spans(nmax);
-    mask.alloc(std::max<int64_t>(c.nsamp, nent) / 32 + 1);
-    words.alloc(nmax / 64 + 9);
-    counts.alloc(nsp);
-    offs.alloc(nsp + 1);
-    tmp.alloc((nsp + 1 + 4095) / 4096 + 1);
-    auto total = [&](int64_t m) {
-        int64_t t = 0;
-        d2h(&t, offs.p + runs_spans(m), 1, s);
-        MADAM_CHECK(hipStreamSynchronize(s));
-        return t;
-    };
-    const bool pol = c.nmap == 3;
-    // baseline side: the samples in time order
-    runs_mark(s, c.d_pixc.p, c.rec_layout, n, c.nsamp, dsh, maxrun, c.d_bstart.p, c.nbase, mask.p, words.p, counts.p,
-              offs.p, tmp.p);
-    c.n_rung = total(n);
-    c.d_rung.alloc(c.n_rung);
-    if (pol) gw.alloc(c.n_rung);
-    runs_write<W>(s, c.d_pixc.p, c.rec_layout, n, dsh, sh, words.p, offs.p, c.d_rung.p, gw.p);
-    c.d_rungst.alloc((size_t)c.ndet * (c.nbase + 1));
-    runs_base_starts(s, c.d_bstart.p, c.nbase, c.ndet, c.nsamp, words.p, offs.p, c.d_rungst.p);
-    // pixel side: the CSR entries
-    runs_mark(s, c.d_entc.p, c.rec_layout, nent, nent, 0, maxrun, c.d_segstart_s.p, c.nzpix, mask.p, words.p, counts.p,
-              offs.p, tmp.p);
-    c.n_runs = total(nent);
-    c.d_runs.alloc(c.n_runs);
-    if (pol) sw.alloc(c.n_runs);
-    runs_write<W>(s, c.d_entc.p, c.rec_layout, nent, 0, sh, words.p, offs.p, c.d_runs.p, sw.p);
-    seg.alloc(c.nzpix + 1);
-    runs_pixel_starts(s, c.d_segstart_s.p, c.nzpix, words.p, offs.p, seg.p);
-    segtiles_alloc(c.sr_r, c.n_runs);
-    segred_build(s, seg.p, c.nzpix, c.n_runs, c.sr_r.heads.p, c.sr_r.k0.p, c.sr_r.fix_end.p, c.sr_r.fix_ord.p);
-    MADAM_CHECK(hipStreamSynchronize(s));
-    c.run_sh = sh;
-    return true;
+    if (!runs_considered<T>(c)) return false;
+    const bool fp64 = sizeof(T) == 8, pol = c.nmap == 3;
+    if (&r == &c.rs) return r.len == 0 || !pol || r.len >= (fp64 ? 1.7 : 1.2);
+    const double line = fp64 ? (pol ? 2.25 : 2.0) : 1.3;
+    return c.mean_run >= line && (r.len == 0 || r.len >= 0.9 * line);
 }
 
-static void release_runs(Context &c)
+template <typename T>
+static auto &run_sums(Context::Runs &r)
 {
-    c.runs_ok = c.runs32_ok = false;
-    c.d_rung.release();
-    c.d_runs.release();
-    c.d_rungw.release();
-    c.d_runsw.release();
-    c.d_rungw32.release();
-    c.d_runsw32.release();
-    c.d_rungst.release();
+    if constexpr (sizeof(T) == 8) return r.w64;
+    else return r.w32;
+}
+
+template <typename T>
+static bool &run_ok(Context::Runs &r)
+{
+    if constexpr (sizeof(T) == 8) return r.ok64;
+    else return r.ok32;
+}
+
+// frees the sums of type T, and the side's other tables where no type reads
+// them (nor may on this pointing: FP32 operators come after the FP64 one)
+template <typename T>
+static void release_runs(Context &c, Context::Runs &r)
+{
+    run_ok<T>(r) = false;
+    run_sums<T>(r).release();
+    if (r.ok64 || r.ok32 || (sizeof(T) == 8 && runs_wanted<float>(c, r))) return;
+    r.word.release();
+    if (&r == &c.rg) {
+        c.d_rungst.release();
+        return;
+    }
     c.sr_r.heads.release();
     c.sr_r.k0.release();
     c.sr_r.fix_end.release();
     c.sr_r.fix_ord.release();
 }
 
-// Below two samples per run the FP64 operator reads samples, and the records
-// hold FP32 sums alone.
-void runs_prepare_fp32(Context &c)
+// one side's run records with weight sums for the operator in type T (the pixel
+// side: and the segment tables over them); false where they do not pay
+template <typename T>
+static bool build_runs(Context &c, Context::Runs &r)
 {
-    if (!runs_wanted<float>(c) || c.runs32_ok) return;
-    if (!c.runs_ok) {
-        if (!if_room([&] { c.runs32_ok = build_runs(c, c.d_rungw32, c.d_runsw32); })) release_runs(c);
-        return;
+    hipStream_t s = c.stream;
+    const bool base = &r == &c.rg, pol = c.nmap == 3;
+    int dsh = 0;
+    if (base)
+        while ((1ll << dsh) < c.ndeg) ++dsh;
+    int sh = 1;
+    while ((1ll << sh) < std::max(c.npix_cross, c.nbtot)) ++sh;
+    if (sh > 28) return false;
+    c.run_sh = sh;
+    uint32_t maxrun = (1u << (32 - sh)) - 1u;
+    // baseline side: the samples in time order; pixel side: the CSR entries
+    const int64_t n = base ? (int64_t)c.ndet * c.nsamp : c.nactive, period = base ? c.nsamp : n;
+    const char *rec = base ? c.d_pixc.p : c.d_entc.p;
+    DBuf<uint32_t> mask;
+    DBuf<unsigned long long> words;
+    DBuf<int32_t> counts;
+    DBuf<int64_t> offs, tmp, seg;
+    int64_t nsp = runs_spans(n);
+    mask.alloc(period / 32 + 1);
+    words.alloc(n / 64 + 9);
+    counts.alloc(nsp);
+    offs.alloc(nsp + 1);
+    tmp.alloc((nsp + 1 + 4095) / 4096 + 1);
+    runs_mark(s, rec, c.rec_layout, n, period, dsh, maxrun, base ? c.d_bstart.p : c.d_segstart_s.p,
+              base ? c.nbase : c.nzpix, mask.p, words.p, counts.p, offs.p, tmp.p);
+    d2h(&r.n, offs.p + nsp, 1, s);
+    MADAM_CHECK(hipStreamSynchronize(s));
+    r.len = (double)c.nactive / std::max<int64_t>(r.n, 1);
+    if (!runs_wanted<T>(c, r)) return false;
+    auto &sums = run_sums<T>(r);
+    r.word.alloc(r.n);
+    if (pol) sums.alloc(r.n);
+    runs_write(s, rec, c.rec_layout, n, dsh, sh, words.p, offs.p, r.word.p, sums.p);
+    if (base) {
+        c.d_rungst.alloc((size_t)c.ndet * (c.nbase + 1));
+        runs_base_starts(s, c.d_bstart.p, c.nbase, c.ndet, c.nsamp, words.p, offs.p, c.d_rungst.p);
+    } else {
+        seg.alloc(c.nzpix + 1);
+        runs_pixel_starts(s, c.d_segstart_s.p, c.nzpix, words.p, offs.p, seg.p);
+        segtiles_alloc(c.sr_r, r.n);
+        segred_build(s, seg.p, c.nzpix, r.n, c.sr_r.heads.p, c.sr_r.k0.p, c.sr_r.fix_end.p, c.sr_r.fix_ord.p);
     }
-    c.runs32_ok = if_room([&] {
-        if (c.nmap != 3) return;
-        c.d_rungw32.alloc(c.n_rung);
-        c.d_runsw32.alloc(c.n_runs);
-        runs_cast(c.stream, c.d_rungw.p, c.d_rungw32.p, c.n_rung);
-        runs_cast(c.stream, c.d_runsw.p, c.d_runsw32.p, c.n_runs);
-    });
-    if (!c.runs32_ok) {
-        c.d_rungw32.release();
-        c.d_runsw32.release();
+    MADAM_CHECK(hipStreamSynchronize(s));
+    return true;
+}
+
+// the run records that the operator in type T reads
+template <typename T>
+static void prepare_runs(Context &c)
+{
+    for (Context::Runs *r : {&c.rg, &c.rs}) {
+        bool &ok = run_ok<T>(*r);
+        if (!ok && runs_wanted<T>(c, *r) && !if_room([&] {
+                if (sizeof(T) == 4 && r->ok64) {   // the FP64 sums, rounded
+                    if (c.nmap == 3) {
+                        r->w32.alloc(r->n);
+                        runs_cast(c.stream, r->w64.p, r->w32.p, r->n);
+                    }
+                    ok = true;
+                } else {
+                    ok = build_runs<T>(c, *r);
+                }
+            }))
+            ok = false;
+        // sums of the pointing before are kept only where this one reads them
+        if (!ok) release_runs<T>(c, *r);
     }
 }
+
+void runs_prepare_fp32(Context &c) { prepare_runs<float>(c); }
 
 template <typename T>
 static RunView<T> run_view(Context &c)
 {
     RunView<T> v;
     v.sh = c.run_sh;
-    v.per_base = (double)c.n_rung / std::max<int64_t>(c.nbtot, 1);
+    v.per_base = (double)c.rg.n / std::max<int64_t>(c.nbtot, 1);
     v.gst = c.d_rungst.p;
-    v.gword = c.d_rung.p;
-    v.sword = c.d_runs.p;
-    if (sizeof(T) == 8) {
-        v.gw = c.d_rungw.p;
-        v.sw = c.d_runsw.p;
-    } else {
-        v.gw = c.d_rungw32.p;
-        v.sw = c.d_runsw32.p;
-    }
+    v.gword = c.rg.word.p;
+    v.sword = c.rs.word.p;
+    v.gw = run_sums<T>(c.rg).p;
+    v.sw = run_sums<T>(c.rs).p;
     return v;
 }
 
 template <typename T>
-static bool use_runs(const Context &c)
+static bool use_runs(const Context &c, const Context::Runs &r)
 {
-    return (sizeof(T) == 8 ? c.runs_ok : c.runs32_ok) && runs_wanted<T>(c);
+    return (sizeof(T) == 8 ? r.ok64 : r.ok32) && runs_considered<T>(c);
 }
 
 void give_up_tables(Context &c)
@@ -945,20 +978,23 @@ void give_up_tables(Context &c)
     MADAM_CHECK(hipStreamSynchronize(c.stream));
     c.lean = true;
     c.set_up++;
-    release_runs(c);
+    for (Context::Runs *r : {&c.rg, &c.rs}) {
+        release_runs<double>(c, *r);
+        release_runs<float>(c, *r);
+    }
     if (c.band_ready) band_give_up_direct(c.band);
 }
 
 int64_t runs_read(const Context &c, bool fp32)
 {
-    return (fp32 ? use_runs<float>(c) : use_runs<double>(c)) ? c.n_rung : 0;
+    return (fp32 ? use_runs<float>(c, c.rg) : use_runs<double>(c, c.rg)) ? c.rg.n : 0;
 }
 
 template <typename T>
 void project_to_map(Context &c, const T *pw, const T *cc_c, T *m4)
 {
-    if (use_runs<T>(c))
-        launch_scatter_run<T>(c.stream, c.nmap, c.n_runs, run_view<T>(c), pw, c.sr_r.heads.p, c.sr_r.k0.p,
+    if (use_runs<T>(c, c.rs))
+        launch_scatter_run<T>(c.stream, c.nmap, c.rs.n, run_view<T>(c), pw, c.sr_r.heads.p, c.sr_r.k0.p,
                               c.sr_r.fix_end.p, c.sr_r.fix_ord.p, c.d_nzq.p, c.nzpix, cc_c, m4, c.d_sr_part.p);
     else
         launch_scatter_seg<T>(c.stream, c.nmap, c.nactive, c.rec_layout == REC16 ? (const void *)c.d_ent.p : c.d_entc.p,
@@ -971,7 +1007,7 @@ template void project_to_map<float>(Context &, const float *, const float *, flo
 template <typename T>
 void project_to_baselines(Context &c, const T *m4, const T *dwb, const T *nna, const T *p, T *ap, int add)
 {
-    if (use_runs<T>(c))
+    if (use_runs<T>(c, c.rg))
         launch_gather_run<T>(c.stream, c.nmap, c.ndet, c.nbase, run_view<T>(c), m4, dwb, nna, p, ap, add);
     else
         launch_gather_flat<T>(c.stream, c.nmap, c.ndet, c.nsamp, c.nbase, c.d_bstart.p,
@@ -1033,14 +1069,7 @@ static void build_segtiles(Context &c)
     }
     int64_t nt = std::max(segred_ntiles(c.nactive), segred_ntiles((int64_t)c.ndet * c.nsamp));
     c.d_sr_part.alloc(2 * (nt > 0 ? nt : 1));
-    // (buffers of the pointing before are kept only where this one's solves can use them)
-    if (runs_wanted<double>(c)) {
-        if (!if_room([&] { c.runs_ok = build_runs(c, c.d_rungw, c.d_runsw); })) release_runs(c);
-    } else {
-        c.d_rungw.release();
-        c.d_runsw.release();
-        if (!runs_wanted<float>(c)) release_runs(c);
-    }
+    prepare_runs<double>(c);
 }
 
 

@@ -146,3 +146,67 @@ def test_runs_that_only_fp32_reads(nnz):
             steps[nsamp, variant] = r["info"]["pcg_steps"]
             m.close()
     assert abs(steps[2 ** 16 - 1, 0] - steps[2 ** 16 - 1, 128]) <= 0.1 * steps[2 ** 16 - 1, 0] + 2
+
+
+def operator(c, ndet, nsamp, nside, ncross, per, nnz, x):
+    """F^T W (F x - P m), m = (P^T W P)^-1 P^T W F x on the well-conditioned pixels, and the size of its terms."""
+    ok = c["pixels"].reshape(-1) >= 0
+    q = c["pixels"].reshape(-1)[ok] // (nside // ncross) ** 2
+    nb = x.size // ndet
+    b = (np.arange(nsamp) // per + np.arange(ndet)[:, None] * nb).reshape(-1)[ok]
+    w = c["pixweights"].reshape(-1, nnz)[ok].astype(np.float64)
+    dw = c["weights"][0]
+    npix = 12 * ncross ** 2
+    cc = np.zeros((npix, nnz, nnz))
+    for i in range(nnz):
+        for j in range(nnz):
+            cc[:, i, j] = dw * np.bincount(q, w[:, i] * w[:, j], npix)
+    ev = np.linalg.eigvalsh(cc)
+    good = (ev[:, -1] > 0) & (ev[:, 0] > 1e-3 * ev[:, -1])
+    inv = np.zeros_like(cc)
+    inv[good] = np.linalg.inv(cc[good])
+    v = dw * x[b]
+    mp = np.einsum("qij,qj->qi", inv, np.stack([np.bincount(q, w[:, j] * v, npix) for j in range(nnz)], -1))
+    use = good[q]
+    ref = np.bincount(b[use], v[use] - dw * np.einsum("sj,sj->s", w[use], mp[q[use]]), x.size)
+    return ref, np.bincount(b[use], np.abs(v[use]), x.size)
+
+
+# the sides decide for themselves: long runs on cross pixels that hold 64 map pixels of one sample each (baseline
+# side only), runs between the two lines (pixel side only), temperature (both), and a solve that wants neither
+@pytest.mark.parametrize("nside,ncross,spin,per,nnz,base_runs,pixel_runs", [
+    (32, 4, 4.0, 50, 3, True, False), (8, 8, 2.47, 50, 3, False, True), (32, 4, 4.0, 50, 1, True, True),
+    (32, 16, 4.3, 5, 3, False, False)])
+def test_sides_use_runs_where_they_pay(nside, ncross, spin, per, nnz, base_runs, pixel_runs):
+    import libmadam_amd
+    ndet, nsamp = 3, 20003
+    scan = dict(fsample=50.0, spin_period=spin, prec_period=4000.0, opening_turns=85.0 / 360.0, lon0_turns=0.0)
+    c = mc.ring_case(ndet=ndet, nsamp=nsamp, nside=nside, base_first=per / 50.0, nnz=nnz, seed=nside,
+                     pointing=lambda d, n: oracle.expand_pointing(scan, dict(psi_turns=0.125 * d), nside, 0, n),
+                     extra_pars=dict(nside_cross=ncross))
+    # samples per run, of time-ordered cross pixels and of map pixels (whose entries may meet again later)
+    pix = c["pixels"].reshape(ndet, nsamp)[0]
+
+    def length(p):
+        return nsamp / (1 + np.sum((p[1:] != p[:-1]) | (np.arange(1, nsamp) % per == 0)))
+    cross, fine = length(pix // (nside // ncross) ** 2), length(pix)
+    print("samples per run: cross %.2f, map %.2f" % (cross, fine))
+    if nnz == 3:
+        assert (cross >= 2.3) == base_runs and (cross >= 2.05 or not pixel_runs) and (fine >= 1.8) == pixel_runs
+    m = libmadam_amd.Madam(0)
+    args = mc.call_args(c)
+    m.configure(*args[:4], *args[7:], c["nnz"])
+    m.set_kernel_variant(128)
+    m.set_pointing(c["pixels"], c["pixweights"])
+    m.solve(c["signal"].copy())
+    x = np.random.default_rng(7).standard_normal(ndet * m.sizes()["nbase"])
+    got = m.apply(2, x)
+    assert (m.stats()["run_records"] > 0) == base_runs
+    ref, size = operator(c, ndet, nsamp, nside, ncross, per, nnz, x)
+    assert np.linalg.norm(got - ref) <= 1e-12 * np.linalg.norm(size)
+    # the mixed solve, whose sides have lines of their own
+    m.solve_batch(c["signal"].reshape(1, ndet, -1).copy(), precision=1)
+    r = m.batch_result(0)
+    res = r["yba"].reshape(-1) - m.apply(2, r["aa"])
+    assert np.linalg.norm(res) <= 1.01e-6 * np.linalg.norm(r["yba"])
+    m.close()
