@@ -877,10 +877,27 @@ static void release_runs(Context &c, Context::Runs &r)
     c.sr_r.fix_ord.release();
 }
 
+// scratch of the builder, for both sides
+struct RunScratch {
+    DBuf<uint32_t> mask;
+    DBuf<unsigned long long> words;
+    DBuf<int32_t> counts;
+    DBuf<int64_t> offs, tmp;
+    void alloc(const Context &c)
+    {
+        const int64_t n = (int64_t)c.ndet * c.nsamp, nsp = runs_spans(n);   // (the CSR entries are no more)
+        mask.alloc(std::max<int64_t>(c.nsamp, c.nactive) / 32 + 1);
+        words.alloc(n / 64 + 9);
+        counts.alloc(nsp);
+        offs.alloc(nsp + 1);
+        tmp.alloc((nsp + 1 + 4095) / 4096 + 1);
+    }
+};
+
 // one side's run records with weight sums for the operator in type T (the pixel
 // side: and the segment tables over them); false where they do not pay
 template <typename T>
-static bool build_runs(Context &c, Context::Runs &r)
+static bool build_runs(Context &c, Context::Runs &r, RunScratch &t)
 {
     hipStream_t s = c.stream;
     const bool base = &r == &c.rg, pol = c.nmap == 3;
@@ -895,36 +912,28 @@ static bool build_runs(Context &c, Context::Runs &r)
     // baseline side: the samples in time order; pixel side: the CSR entries
     const int64_t n = base ? (int64_t)c.ndet * c.nsamp : c.nactive, period = base ? c.nsamp : n;
     const char *rec = base ? c.d_pixc.p : c.d_entc.p;
-    DBuf<uint32_t> mask;
-    DBuf<unsigned long long> words;
-    DBuf<int32_t> counts;
-    DBuf<int64_t> offs, tmp, seg;
-    int64_t nsp = runs_spans(n);
-    mask.alloc(period / 32 + 1);
-    words.alloc(n / 64 + 9);
-    counts.alloc(nsp);
-    offs.alloc(nsp + 1);
-    tmp.alloc((nsp + 1 + 4095) / 4096 + 1);
+    t.alloc(c);
     runs_mark(s, rec, c.rec_layout, n, period, dsh, maxrun, base ? c.d_bstart.p : c.d_segstart_s.p,
-              base ? c.nbase : c.nzpix, mask.p, words.p, counts.p, offs.p, tmp.p);
-    d2h(&r.n, offs.p + nsp, 1, s);
+              base ? c.nbase : c.nzpix, t.mask.p, t.words.p, t.counts.p, t.offs.p, t.tmp.p);
+    d2h(&r.n, t.offs.p + runs_spans(n), 1, s);
     MADAM_CHECK(hipStreamSynchronize(s));
     r.len = (double)c.nactive / std::max<int64_t>(r.n, 1);
     if (!runs_wanted<T>(c, r)) return false;
     auto &sums = run_sums<T>(r);
     r.word.alloc(r.n);
     if (pol) sums.alloc(r.n);
-    runs_write(s, rec, c.rec_layout, n, dsh, sh, words.p, offs.p, r.word.p, sums.p);
+    runs_write(s, rec, c.rec_layout, n, dsh, sh, t.words.p, t.offs.p, r.word.p, sums.p);
     if (base) {
         c.d_rungst.alloc((size_t)c.ndet * (c.nbase + 1));
-        runs_base_starts(s, c.d_bstart.p, c.nbase, c.ndet, c.nsamp, words.p, offs.p, c.d_rungst.p);
+        runs_base_starts(s, c.d_bstart.p, c.nbase, c.ndet, c.nsamp, t.words.p, t.offs.p, c.d_rungst.p);
     } else {
+        DBuf<int64_t> seg;
         seg.alloc(c.nzpix + 1);
-        runs_pixel_starts(s, c.d_segstart_s.p, c.nzpix, words.p, offs.p, seg.p);
+        runs_pixel_starts(s, c.d_segstart_s.p, c.nzpix, t.words.p, t.offs.p, seg.p);
         segtiles_alloc(c.sr_r, r.n);
         segred_build(s, seg.p, c.nzpix, r.n, c.sr_r.heads.p, c.sr_r.k0.p, c.sr_r.fix_end.p, c.sr_r.fix_ord.p);
+        MADAM_CHECK(hipStreamSynchronize(s));   // seg
     }
-    MADAM_CHECK(hipStreamSynchronize(s));
     return true;
 }
 
@@ -932,6 +941,7 @@ static bool build_runs(Context &c, Context::Runs &r)
 template <typename T>
 static void prepare_runs(Context &c)
 {
+    RunScratch t;
     for (Context::Runs *r : {&c.rg, &c.rs}) {
         bool &ok = run_ok<T>(*r);
         if (!ok && runs_wanted<T>(c, *r) && !if_room([&] {
@@ -942,7 +952,7 @@ static void prepare_runs(Context &c)
                     }
                     ok = true;
                 } else {
-                    ok = build_runs<T>(c, *r);
+                    ok = build_runs<T>(c, *r, t);
                 }
             }))
             ok = false;
