@@ -259,7 +259,12 @@ __global__ void __launch_bounds__(64) k_band_factor_w(const Segment *seg, int64_
 // ended in.  Equal bits: the piece is what the serial chain gives.  Otherwise
 // (or where a pivot failed on the way) it factors the piece again from the
 // true window, so the factor always has the serial chain's bits.
-static constexpr int BP_ROWS = 1024, BP_WARM = 512;
+// Wider bands remember longer: with 30 baselines most pieces' windows differ in
+// their last bits after the warm-up, with 50 all of them do, and the second pass
+// is the serial chain again.  Preconditioner of 2 x 168 k flagged rows, serial /
+// pieces: 10 baselines 39 / 3.2 ms, 20 52 / 4.3, 30 76 / 78 to 103, 50 143 / 181;
+// so pieces serve the two narrow classes.
+static constexpr int BP_ROWS = 1024, BP_WARM = 512, BP_KD = 19;
 
 template <int KD>
 struct BandWin {
@@ -392,11 +397,11 @@ __global__ void __launch_bounds__(64) k_band_factor_pieces(const Segment *seg, i
     if (lane == 0) bad[pc] = f >= 0 ? 1 : 0;
 }
 
-// wave per segment: see above; info as k_band_factor_w
+// wave per segment: see above; info as k_band_factor_w; bad[piece] = 2 where it was factored again
 template <int KD>
 __global__ void __launch_bounds__(64) k_band_factor_check(const Segment *seg, int64_t nseg, const int *nband_seg,
                                                           const int64_t *pfirst, const double *invcov, int64_t nof,
-                                                          const double *nna, double *Lb, double *win, const int *bad,
+                                                          const double *nna, double *Lb, double *win, int *bad,
                                                           int *info)
 {
     constexpr int K = KD + 1;
@@ -423,6 +428,7 @@ __global__ void __launch_bounds__(64) k_band_factor_check(const Segment *seg, in
             ok = __ballot(!eq) == 0;
         }
         if (ok) continue;
+        if (lane == 0) bad[pc] = 2;
         // from the true window; a segment's first piece starts from its own
         BandWin<KD> w;
         if (t == 0) {
@@ -1531,7 +1537,7 @@ static int band_tables(hipStream_t s, BandPrec &bp, const Segment *hseg, const S
     DBuf<unsigned long long> dcnt;   // nna changes per segment
     dcnt.alloc(ns1);
     MADAM_CHECK(hipMemsetAsync(dcnt.p, 0, sizeof(unsigned long long) * ns1, s));
-    bool may = pieces && periodic && longest > BP_SERIAL && nseg <= 65535;
+    bool may = pieces && KD <= BP_KD && periodic && longest > BP_SERIAL && nseg <= 65535;
     pieces = false;
     if (may) {
         k_band_nna_changes<<<dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(64, 8192 / nseg)), (unsigned)nseg), 256,
@@ -1563,8 +1569,16 @@ static int band_tables(hipStream_t s, BandPrec &bp, const Segment *hseg, const S
         MADAM_CHECK(hipGetLastError());
         MADAM_CHECK(hipMemcpyAsync(info_out, dinfo.p, sizeof(int) * nseg, hipMemcpyDeviceToHost, s));
         MADAM_CHECK(hipStreamSynchronize(s));
+        std::vector<int> again(npc);
+        MADAM_CHECK(hipMemcpyAsync(again.data(), bad.p, sizeof(int) * npc, hipMemcpyDeviceToHost, s));
+        MADAM_CHECK(hipStreamSynchronize(s));
         for (int64_t i = 0; i < nseg; ++i)
-            if (!hseg[i].skip && nband_seg_host[i] > 0) bp.nrows_factored += hseg[i].noba;
+            if (!hseg[i].skip && nband_seg_host[i] > 0) {
+                bp.nrows_factored += hseg[i].noba;
+                for (int64_t t = pfirst[i]; t < pfirst[i + 1]; ++t)
+                    if (again[t] == 2)
+                        bp.nrows_factored += std::min<int64_t>(BP_ROWS, hseg[i].noba - (t - pfirst[i]) * BP_ROWS);
+            }
     } else {
         DBuf<int64_t> dper;   // per_src[nseg][BAND_MAXJ], per_q[nseg][BAND_MAXJ]
         int64_t nj = ns1 * BAND_MAXJ;

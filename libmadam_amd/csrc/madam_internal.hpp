@@ -432,7 +432,8 @@ struct BandPrec {
     // partitions (and 64-partition blocks) that are not bitwise repeats of the previous one
     int64_t nchunk_unique = 0, nblock = 0, nblock_unique = 0;
     int64_t nrows = 0;      // baseline rows the factored segments cover
-    int64_t nrows_factored = 0;   // of those, rows the column loop computed (the rest repeat a block)
+    int64_t nrows_factored = 0;   // rows the column loops computed (fewer where blocks repeat, more where pieces are
+                                  // factored again)
     // carry chains: -1 several chains per wave when there are enough of them,
     // 1 always, 0 never (one chain per wave); the same results either way
     int chain_pack = -1;
